@@ -221,10 +221,10 @@ ForceArgs force_args(const chan_ctx *c) {
   a.F0 = c->F0;
   a.gain = c->gain;
   a.der = c->der;
+  a.derF = c->derF;
   for (int k = 0; k < 3; k++) a.src[k] = c->gain ? c->src[k] : -1;
   a.out = nullptr;
   a.g = c->g;
-  a.chunk = 48;
   return a;
 }
 
@@ -316,6 +316,7 @@ int chan_create(const chan_params *p, chan_ctx **out) {
   if ((rc = dalloc_bytes(&c->twz, (size_t)fft::tw_table_size(g.nzd) * esz))) return bail(rc);
   if ((rc = dalloc_bytes(&c->twx, (size_t)fft::tw_table_size(2 * g.nxd) * esz))) return bail(rc);
   if ((rc = dalloc(&c->der, (size_t)(g.ny - 1) * 20))) return bail(rc);
+  if ((rc = dalloc(&c->derT, (size_t)g.Ny * 20)) || (rc = dalloc(&c->derF, (size_t)g.Ny * 10))) return bail(rc);
   if ((rc = dalloc(&c->d0fac, (size_t)(g.ny + 1) * 5))) return bail(rc);
   if ((rc = dalloc(&c->y, (size_t)g.Ny))) return bail(rc);
   if ((rc = dalloc(&c->dy, (size_t)g.ny + 1))) return bail(rc);
@@ -336,6 +337,30 @@ int chan_create(const chan_params *p, chan_ctx **out) {
       hipMemcpy(c->y, h.y, sizeof(double) * g.Ny, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(c->dy, h.dy, sizeof(double) * (g.ny + 1), hipMemcpyHostToDevice) != hipSuccess)
     return bail(fail(CHAN_E_STATE, "upload of the set-up failed"));
+  {
+    // row r's weights in the stencils of the interior rows r-2..r+2; those of
+    // a body force have its wall rows folded in: F(0) = F(ny) = 0, and the
+    // ghost values F(-1) = -(d4[2] F(1) + d4[3] F(2) + d4[4] F(3)) / d4[0] of
+    // row 1 and F(ny+1) of row ny-1 likewise
+    std::vector<double> t((size_t)g.Ny * 20, 0.0), tf((size_t)g.Ny * 10, 0.0);
+    for (int r = -1; r <= g.ny + 1; r++)
+      for (int m = 0; m < 5; m++) {
+        const int iy = r - 2 + m, j = 4 - m;
+        if (iy < 1 || iy > g.ny - 1) continue;
+        const double *d = h.der + (size_t)(iy - 1) * 20, *d4 = d + 15;
+        for (int f = 0; f < 4; f++) t[(size_t)(r + 1) * 20 + 4 * m + f] = d[5 * f + j];
+        if (r < 1 || r > g.ny - 1) continue;
+        for (int f = 0; f < 2; f++) {
+          double w = d[5 * f + j];
+          if (iy == 1) w -= d[5 * f] * d4[j] / d4[0];
+          if (iy == g.ny - 1) w -= d[5 * f + 4] * d4[j] / d4[4];
+          tf[(size_t)(r + 1) * 10 + 2 * m + f] = w;
+        }
+      }
+    if (hipMemcpy(c->derT, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(c->derF, tf.data(), tf.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
+      return bail(fail(CHAN_E_STATE, "upload of the set-up failed"));
+  }
   DevScalars s0;
   std::memset(&s0, 0, sizeof s0);
   s0.meanpx = p->meanpx;
@@ -359,7 +384,7 @@ int chan_destroy(chan_ctx *c) {
   }
   for (auto e : c->pool) hipEventDestroy(e);
   void *bufs[] = {c->V, c->old, c->rhs, c->L, c->col00, c->A, c->B, c->P, c->twz, c->twx,
-                  c->der, c->d0fac, c->y, c->dy, c->sc, c->stat, c->F0, c->gain, c->Fkeep};
+                  c->der, c->derT, c->derF, c->d0fac, c->y, c->dy, c->sc, c->stat, c->F0, c->gain, c->Fkeep};
   for (void *b : bufs)
     if (b) hipFree(b);
   if (c->st) hipStreamDestroy(c->st);
@@ -610,51 +635,49 @@ static int products(chan_ctx *c, int plane0, int nplanes, bool prods, int cfl) {
 }
 
 template <typename R>
-static int rhs_t(chan_ctx *c, const double ode[3], bool keep) {
+static int rhs_t(chan_ctx *c, const double ode[3], bool keep, bool store_old) {
   RhsArgs<R> a;
   a.P = static_cast<const cx<R> *>(c->P);
   a.V = c->V;
   a.old = static_cast<cx<R> *>(c->old);
   a.rhs = c->rhs;
-  a.der = c->der;
+  a.derT = c->derT;
   a.sc = c->sc;
+  a.store_old = store_old;
   a.g = c->g;
   a.ode0 = ode[0];
   a.ode1 = ode[1];
   a.ode2 = ode[2];
   a.dt = c->deltat;
   a.ni = c->prm.ni;
-  a.chunk = 48;
-  a.force = c->F0 || c->gain;
-  if (keep) c->kept_state = a.force ? 1 : 2;
-  if (a.force) {
-    ForceArgs f = force_args(c);
+  a.chunk = 0;
+  const bool force = c->F0 || c->gain;
+  if (keep) c->kept_state = force ? 1 : 2;
+  ForceArgs f = force_args(c);
+  if (force && keep) {
+    f.out = c->Fkeep;
     int rc;
-    if (keep) {
-      f.out = c->Fkeep;
-      if ((rc = timed(c, "force_keep", [&] { return launch_force(c->st, f); }))) return rc;
-    }
-    f.out = c->rhs;
-    if ((rc = timed(c, "force", [&] { return launch_force_terms(c->st, f); }))) return rc;
+    if ((rc = timed(c, "force_keep", [&] { return launch_force(c->st, f); }))) return rc;
   }
-  return timed(c, "rhs", [&] { return launch_rhs<R>(c->st, a); });
+  return timed(c, "rhs", [&] { return launch_rhs<R>(c->st, a, force ? &f : nullptr); });
 }
 
 // keep: store the applied force when keeping is on (chan_step asks only in
-// its last substep, whose force is the one that stays)
-static int buildrhs(chan_ctx *c, const double ode[3], bool compute_cfl, bool keep) {
+// its last substep, whose force is the one that stays).  store_old: leave the
+// explicit terms behind for a following substep with ode[2] != 0.
+static int buildrhs(chan_ctx *c, const double ode[3], bool compute_cfl, bool keep, bool store_old) {
   const Geom &g = c->g;
   int rc;
   if ((rc = products(c, 0, g.Ny, true, compute_cfl ? 1 : 0))) return rc;
   keep = keep && c->Fkeep;
-  return c->split ? rhs_t<float>(c, ode, keep) : rhs_t<double>(c, ode, keep);
+  return c->split ? rhs_t<float>(c, ode, keep, store_old) : rhs_t<double>(c, ode, keep, store_old);
 }
 }  // extern "C++"
 
 int chan_buildrhs(chan_ctx *c, const double ode[3], int32_t compute_cfl) {
   if (!c || !ode) return fail(CHAN_E_ARG, "null argument");
   if (!c->field_set) return fail(CHAN_E_STATE, "buildrhs before set_field");
-  return buildrhs(c, ode, compute_cfl != 0, true);
+  return buildrhs(c, ode, compute_cfl != 0, true, true);
 }
 
 int chan_linsolve(chan_ctx *c, double lambda) {
@@ -777,23 +800,29 @@ int chan_outstats(chan_ctx *c, double row[11]) {
   return 0;
 }
 
-int chan_step(chan_ctx *c, double row[11]) {
-  if (!c || !row) return fail(CHAN_E_ARG, "null argument");
+// One time step.  store_old: also leave the third substep's explicit terms
+// behind; a following step's first substep (ode[2] = 0) does not read them.
+static int time_step(chan_ctx *c, double row[11], bool store_old) {
   int rc;
   const double *ode[3] = {RK1, RK2, RK3};
   for (int k = 0; k < 3; k++) {
     c->time = c->time + 2.0 / ode[k][0] * c->deltat;
     if (!c->field_set) return fail(CHAN_E_STATE, "step before set_field");
-    if ((rc = buildrhs(c, ode[k], k == 2, k == 2))) return rc;
+    if ((rc = buildrhs(c, ode[k], k == 2, k == 2, k < 2 || store_old))) return rc;
     if ((rc = chan_linsolve(c, ode[k][0] / c->deltat))) return rc;
   }
   return chan_outstats(c, row);
 }
 
+int chan_step(chan_ctx *c, double row[11]) {
+  if (!c || !row) return fail(CHAN_E_ARG, "null argument");
+  return time_step(c, row, true);
+}
+
 int chan_steps(chan_ctx *c, int32_t n, double *rows) {
   if (!c || (n > 0 && !rows)) return fail(CHAN_E_ARG, "null argument");
   for (int32_t i = 0; i < n; i++) {
-    int rc = chan_step(c, rows + 11 * (size_t)i);
+    int rc = time_step(c, rows + 11 * (size_t)i, i + 1 == n);
     if (rc) return rc;
   }
   return 0;

@@ -44,12 +44,12 @@ struct RhsArgs {
   cx<R> *old;            // [2][ny-1][ps] previous explicit terms (eta, d2v); in the split
                          // mode FP32, as the products they are formed from
   cx<double> *rhs;       // [2][ny-1][ps]
-  const double *der;     // [(ny-1)][4][5]
+  const double *derT;    // [Ny][5][4]: row r's weights d0, d1, d2, d4 in the rows r-2..r+2
   const DevScalars *sc;  // meanpx, meanpz
-  bool force;            // rhs holds the body-force terms (k_force_terms) on entry
+  bool store_old;        // leave this substep's explicit terms in old
   Geom g;
   double ode0, ode1, ode2, dt, ni;
-  int chunk;
+  int chunk;  // rows per thread, set by launch_rhs
 };
 
 // Body force F_d = F0_d + gain[d][plane][col] * V_src[d]; either part may be
@@ -57,10 +57,10 @@ struct RhsArgs {
 struct ForceArgs {
   const cx<double> *V, *F0;  // [3][Ny][ps]; F0 may be null
   const double *gain, *der;  // gain [3][Ny][Nz+1]
+  const double *derF;        // [Ny][5][2]: a force row's weights d0, d1 in the rows r-2..r+2
   int src[3];
-  cx<double> *out;  // k_force: [3][Ny][ps]; k_force_terms: [2][ny-1][ps]
+  cx<double> *out;  // k_force: [3][Ny][ps]
   Geom g;
-  int chunk;
 };
 
 struct SolveArgs {
@@ -113,9 +113,8 @@ hipError_t launch_fs768_test(const cx<double> *in, cx<double> *out, const cx<dou
 hipError_t launch_fft_bench(int N, int sign, int variant, const cx<double> *in, cx<double> *out, const cx<double> *tw,
                             int batch, int inner);
 template <typename R>
-hipError_t launch_rhs(hipStream_t st, const RhsArgs<R> &a);
+hipError_t launch_rhs(hipStream_t st, const RhsArgs<R> &a, const ForceArgs *force);  // force null: none
 hipError_t launch_force(hipStream_t st, const ForceArgs &a);
-hipError_t launch_force_terms(hipStream_t st, const ForceArgs &a);
 hipError_t launch_stats(hipStream_t st, const cx<double> *V, const double *avg, double *out, const Geom &g);
 hipError_t launch_solve(hipStream_t st, const SolveArgs &a);
 hipError_t launch_mean(hipStream_t st, const MeanArgs &a);

@@ -1,27 +1,43 @@
 // k_rhs.hip -- K4: right-hand sides of the v-eta formulation for every
 // interior row and wavenumber pair (buildrhs, dnsdata.f90:611-673).
 //
-// One thread per (pair, chunk of rows) walks y with a five-row window of the
-// six products and three velocity components held in registers, so each
-// plane is read once.  For each row it forms rhsu/rhsv/rhsw from the compact
-// d0/d1/d2 stencils of the products (the DD macro, :609-610), the explicit
-// terms of the D2v and eta equations (:637-661), the implicit operators
-// OS/SQ (:476-477) and the CN-RK3 time scheme (:486), writes the new rhs and
-// replaces the stored explicit term.
+// With kx = al, kz = be, k2 = kx^2 + kz^2, the explicit terms of the D2v and
+// eta equations (:637-661) are stencils of four combinations of the six
+// products, formed once per row and pair:
+//   G1 = k2 vv - kx^2 uu - 2 kx kz uw - kz^2 ww,  G2 = i kx uv + i kz vw
+//   G3 = kx kz (uu - ww) + (kz^2 - kx^2) uw,      G4 = i kx vw - i kz uv
+//   D2v: D1(G1) + D2(G2) + k2 D0(G2),             eta: D0(G3) + D1(G4)
+// (the (0,0) mode's eta slot carries the mean flow: G4 = -(Re uv + i Re vw)).
+// The implicit operators OS/SQ (:476-477) and the time derivative are one
+// stencil of v and one of eta = i kz u - i kx w.
 //
-// With a body force, k_force_terms first forms the force terms of buildrhs
-// (dnsdata.f90:643-659) from F = F0 + gain * V_src with the wall treatment
-// of :616-628 (F zero on the wall rows, ghost rows that make the compact D4
-// of the first and last interior rows vanish) and leaves them in the rhs
-// buffer; the FORCE variant of k_rhs adds them to the explicit terms as it
-// overwrites that buffer.  A five-row force window inside k_rhs itself would
-// push it past the register file.
+// One thread per (pair, chunk of rows) walks y and adds each row, as it is
+// read, to the sums of the five output rows whose stencils reach it: four
+// complex sums per pending row (explicit and implicit part of each equation),
+// 80 FP64 registers' worth, where a five-row window of the nine fields that
+// are read would be 90 complex values.  It then finishes the oldest row with
+// the CN-RK3 time scheme (:486), writes the new rhs and replaces the stored
+// explicit term.  The stencil coefficients come transposed (row r's weights
+// in the five rows r-2..r+2), wave-uniform through the scalar cache.
+//
+// A body force enters the same sums as it is formed from F = F0 + gain * V_src
+// (:643-659): D1(-i kx F_u - i kz F_w) and -k2 D0(F_v) in the D2v equation,
+// D0(i kz F_u - i kx F_w) in the eta equation.  Its wall treatment (:616-628:
+// F zero on the wall rows, ghost rows that make the compact D4 of the first
+// and last interior rows vanish) is in the weights: the force has a table of
+// its own, in which the ghost row is eliminated from rows 1 and ny-1 and the
+// rows outside 1..ny-1 weigh nothing.  A feedback force reads only its gains
+// besides what the right-hand side reads anyway: against force terms formed
+// by a kernel of their own and read back, 34 for 155 us per substep at
+// 63x96x47, 1.19 for 2.23 ms at 191x384x189.
+//
+// Bound by HBM on large grids: 5.8 GB per launch at 191x384x189 (FP64) in 1.21
+// ms, 4.8 TB/s, where a five-row window of the nine fields in two waves per
+// SIMD and 48-row chunks took 1.39; by the length of the walk on small ones
+// (31x64x31: 11.8 us, 61 before).
 #include "chan_internal.hpp"
 
 namespace chan {
-
-__device__ __forceinline__ cx<double> imul(double a, cx<double> X) { return cx<double>{-(a * X.y), a * X.x}; }
-__device__ __forceinline__ cx<double> neg(cx<double> X) { return cx<double>{-X.x, -X.y}; }
 
 // ghost rows of the body force (dnsdata.f90:617-628): with F(0) = F(-1) = 0 the
 // compact D4 of row 1 is d4(0)F(1) + d4(1)F(2) + d4(2)F(3), and
@@ -33,164 +49,6 @@ __device__ __forceinline__ cx<double> ghost_lo(const double *d4, cx<double> f1, 
 __device__ __forceinline__ cx<double> ghost_hi(const double *d4, cx<double> f3, cx<double> f2, cx<double> f1) {
   const cx<double> s = add(add(scl(d4[0], f3), scl(d4[1], f2)), scl(d4[2], f1));
   return cx<double>{-s.x / d4[4], -s.y / d4[4]};
-}
-
-// one-wave blocks: each lane walks a long row chunk, and smaller blocks spread
-// the waves more evenly over the CUs (1.7% faster than 256-thread blocks in
-// FP64 at 191x384x189)
-constexpr int RHS_BLOCK = 64;
-
-template <typename R, bool FORCE>
-__global__ __launch_bounds__(256) void k_rhs(RhsArgs<R> a, const double *__restrict__ der,
-                                             const DevScalars *__restrict__ sc) {
-  // der and sc are separate restrict arguments so that their wave-uniform
-  // values come through the scalar cache instead of vector registers.
-  const Geom g = a.g;
-  const int p = blockIdx.x * RHS_BLOCK + threadIdx.x;
-  if (p >= g.npair) return;
-  const int ix = p / g.Nz, iz = p % g.Nz - g.nz;
-  const double al = g.alfa0 * ix, be = g.beta0 * iz;
-  const double k2 = (g.alfa0 * ix) * (g.alfa0 * ix) + (g.beta0 * iz) * (g.beta0 * iz);
-  const int y0 = 1 + (int)blockIdx.y * a.chunk;
-  if (y0 > g.ny - 1) return;
-  const int y1 = min(g.ny - 1, y0 + a.chunk - 1);
-  const size_t ps = g.ps, pstride = (size_t)g.Ny * ps;
-  const bool mean = (ix == 0 && iz == 0);
-  const double meanpx = sc->meanpx, meanpz = sc->meanpz;
-
-  // window slot j holds row iy-2+j; plane index of row r is r+1.  The stored
-  // explicit terms of row iy are loaded one iteration early into nxo,
-  // unconditionally (clamped row), so the loads overlap the previous row.
-  const size_t rs = (size_t)(g.ny - 1) * ps;  // component stride of old/rhs
-  cx<double> wp[6][5], wv[3][5], nxo[2], nxf[2];
-  auto load_row = [&](int r, int j) {
-    const size_t off = (size_t)(r + 1) * ps + p;
-#pragma unroll
-    for (int q = 0; q < 6; q++) {
-      const cx<R> v = a.P[q * pstride + off];
-      wp[q][j] = cx<double>{(double)v.x, (double)v.y};
-    }
-#pragma unroll
-    for (int c = 0; c < 3; c++) wv[c][j] = a.V[c * pstride + off];
-  };
-#pragma unroll
-  for (int j = 0; j < 4; j++) load_row(y0 - 2 + j, j);
-  auto ldold = [&](size_t i) {
-    const cx<R> o = a.old[i];
-    return cx<double>{(double)o.x, (double)o.y};
-  };
-  nxo[0] = ldold((size_t)(y0 - 1) * ps + p);
-  nxo[1] = ldold(rs + (size_t)(y0 - 1) * ps + p);
-  // force terms of the eta and D2v equations, left in rhs by k_force_terms
-  if constexpr (FORCE) {
-    nxf[0] = a.rhs[(size_t)(y0 - 1) * ps + p];
-    nxf[1] = a.rhs[rs + (size_t)(y0 - 1) * ps + p];
-  }
-
-  for (int iy = y0; iy <= y1; iy++) {
-    load_row(iy + 2, 4);
-    const cx<double> old_eta = nxo[0], old_v = nxo[1];
-    cx<double> f_eta = {0.0, 0.0}, f_v = {0.0, 0.0};
-    if constexpr (FORCE) {
-      f_eta = nxf[0];
-      f_v = nxf[1];
-    }
-    {
-      const int on = min(iy, g.ny - 2);
-      nxo[0] = ldold((size_t)on * ps + p);
-      nxo[1] = ldold(rs + (size_t)on * ps + p);
-      if constexpr (FORCE) {
-        nxf[0] = a.rhs[(size_t)on * ps + p];
-        nxf[1] = a.rhs[rs + (size_t)on * ps + p];
-      }
-    }
-    const double *d = der + (size_t)(iy - 1) * 20;  // d0[5] d1[5] d2[5] d4[5]
-    auto DD = [&](int f, int q) {
-      cx<double> s = scl(d[f * 5 + 0], wp[q][0]);
-#pragma unroll
-      for (int j = 1; j < 5; j++) s = add(s, scl(d[f * 5 + j], wp[q][j]));
-      return s;
-    };
-
-    // products: 0 uu, 1 vv, 2 ww, 3 uv, 4 vw, 5 uw
-    const cx<double> DD0_6 = DD(0, 5), DD1_6 = DD(1, 5);
-    const cx<double> rhsu = sub(sub(neg(imul(al, DD(0, 0))), DD(1, 3)), imul(be, DD0_6));
-    const cx<double> rhsv = sub(sub(neg(imul(al, DD(0, 3))), DD(1, 1)), imul(be, DD(0, 4)));
-    const cx<double> rhsw = sub(sub(neg(imul(al, DD0_6)), DD(1, 4)), imul(be, DD(0, 2)));
-    cx<double> expl =
-        sub(add(imul(al, add(add(imul(al, DD(1, 0)), DD(2, 3)), imul(be, DD1_6))),
-                imul(be, add(add(imul(al, DD1_6), DD(2, 4)), imul(be, DD(1, 2))))),
-            scl(k2, rhsv));
-    if constexpr (FORCE) expl = add(expl, f_v);
-    const size_t o = (size_t)(iy - 1) * ps + p;
-    // D2v equation: unknown D2(v) - k2 D0(v), implicit OS v
-    {
-      cx<double> s2 = scl(d[10], wv[1][0]), s0 = scl(d[0], wv[1][0]);
-#pragma unroll
-      for (int j = 1; j < 5; j++) {
-        s2 = add(s2, scl(d[10 + j], wv[1][j]));
-        s0 = add(s0, scl(d[j], wv[1][j]));
-      }
-      const cx<double> unkn = sub(s2, scl(k2, s0));
-      cx<double> impl = {0.0, 0.0};
-#pragma unroll
-      for (int j = 0; j < 5; j++) {
-        const double os = a.ni * (d[15 + j] - 2.0 * k2 * d[10 + j] + k2 * k2 * d[j]);
-        impl = add(impl, scl(os, wv[1][j]));
-      }
-      const cx<double> old = old_v;
-      const cx<double> un = scl(a.ode0, unkn);
-      const cx<double> r = sub(add(add(cx<double>{un.x / a.dt, un.y / a.dt}, impl), scl(a.ode1, expl)), scl(a.ode2, old));
-      a.old[rs + o] = cx<R>{(R)expl.x, (R)expl.y};
-      a.rhs[rs + o] = r;
-    }
-    // eta equation (or the mean flow Re u + i Re w in mode (0,0))
-    {
-      cx<double> ex, unkn, impl;
-      if (mean) {
-        ex = cx<double>{rhsu.x + meanpx, rhsw.x + meanpz};
-        if constexpr (FORCE) ex = add(ex, f_eta);
-        double a1 = d[0] * wv[0][0].x, a3 = d[0] * wv[2][0].x, b1 = d[10] * wv[0][0].x, b3 = d[10] * wv[2][0].x;
-#pragma unroll
-        for (int j = 1; j < 5; j++) {
-          a1 += d[j] * wv[0][j].x;
-          a3 += d[j] * wv[2][j].x;
-          b1 += d[10 + j] * wv[0][j].x;
-          b3 += d[10 + j] * wv[2][j].x;
-        }
-        unkn = cx<double>{a1, a3};
-        impl = cx<double>{a.ni * b1, a.ni * b3};
-      } else {
-        ex = sub(imul(be, rhsu), imul(al, rhsw));
-        if constexpr (FORCE) ex = add(ex, f_eta);
-        cx<double> s1 = scl(d[0], wv[0][0]), s3 = scl(d[0], wv[2][0]);
-#pragma unroll
-        for (int j = 1; j < 5; j++) {
-          s1 = add(s1, scl(d[j], wv[0][j]));
-          s3 = add(s3, scl(d[j], wv[2][j]));
-        }
-        unkn = sub(imul(be, s1), imul(al, s3));
-        impl = cx<double>{0.0, 0.0};
-#pragma unroll
-        for (int j = 0; j < 5; j++) {
-          const double sq = a.ni * (d[10 + j] - k2 * d[j]);
-          impl = add(impl, scl(sq, sub(imul(be, wv[0][j]), imul(al, wv[2][j]))));
-        }
-      }
-      const cx<double> old = old_eta;
-      const cx<double> un = scl(a.ode0, unkn);
-      const cx<double> r = sub(add(add(cx<double>{un.x / a.dt, un.y / a.dt}, impl), scl(a.ode1, ex)), scl(a.ode2, old));
-      a.old[o] = cx<R>{(R)ex.x, (R)ex.y};
-      a.rhs[o] = r;
-    }
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-#pragma unroll
-      for (int q = 0; q < 6; q++) wp[q][j] = wp[q][j + 1];
-#pragma unroll
-      for (int c = 0; c < 3; c++) wv[c][j] = wv[c][j + 1];
-    }
-  }
 }
 
 // F_c at interior row r (1 <= r <= ny-1) of pair p: the static part plus the
@@ -217,48 +75,154 @@ __device__ __forceinline__ cx<double> force_row(const ForceArgs &a, const double
   return cx<double>{0.0, 0.0};
 }
 
-// The force terms of buildrhs for rows y0..y1 of pair p (one thread per pair
-// and chunk of rows, five-row window of F):
-//   out[0] (eta)  i kz D0(F_u) - i kx D0(F_w), or (D0 Re F_u, D0 Re F_w) in
-//                 the mode (0,0) (rD0, dnsdata.f90:650-652, 657-659);
-//   out[1] (D2v)  -k2 D0(F_v) - i kx D1(F_u) - i kz D1(F_w) (:643-645).
-__global__ __launch_bounds__(256) void k_force_terms(ForceArgs a, const double *__restrict__ der) {
+// one-wave blocks: each lane walks a row chunk, and smaller blocks spread the
+// waves more evenly over the CUs
+constexpr int RHS_BLOCK = 64;
+
+// RD: the previous explicit terms enter (ode2 != 0); the first RK3 substep
+// has ode2 = 0 and does not read them.
+template <typename R, bool FORCE, bool RD>
+__global__ __launch_bounds__(RHS_BLOCK) void k_rhs(RhsArgs<R> a, ForceArgs fa, const double *__restrict__ derT,
+                                                   const double *__restrict__ derF, const DevScalars *__restrict__ sc) {
+  // derT, derF and sc are separate restrict arguments so that their
+  // wave-uniform values come through the scalar cache instead of vector
+  // registers.
   const Geom g = a.g;
-  const int p = blockIdx.x * 256 + threadIdx.x;
+  const int p = blockIdx.x * RHS_BLOCK + threadIdx.x;
   if (p >= g.npair) return;
   const int ix = p / g.Nz, iz = p % g.Nz - g.nz;
-  const bool mean = (ix == 0 && iz == 0);
-  const int col = mean ? g.Nz : iz + g.nz;
   const double al = g.alfa0 * ix, be = g.beta0 * iz;
-  const double k2 = (g.alfa0 * ix) * (g.alfa0 * ix) + (g.beta0 * iz) * (g.beta0 * iz);
+  const double al2 = al * al, be2 = be * be, albe = al * be, k2 = al2 + be2;
   const int y0 = 1 + (int)blockIdx.y * a.chunk;
   if (y0 > g.ny - 1) return;
   const int y1 = min(g.ny - 1, y0 + a.chunk - 1);
-  const size_t ps = g.ps, rs = (size_t)(g.ny - 1) * ps;
-  cx<double> w[3][5];
+  const size_t ps = g.ps, pstride = (size_t)g.Ny * ps;
+  const bool mean = (ix == 0 && iz == 0);
+  const int col = mean ? g.Nz : iz + g.nz;
+  // weights of the implicit v stencil: cA D2 + cB D0 + ni D4, and of eta: cC D0 + ni D2
+  const double rdt = a.ode0 / a.dt;
+  const double cA = rdt - 2.0 * a.ni * k2, cB = k2 * (a.ni * k2 - rdt), cC = rdt - a.ni * k2;
+  const size_t rs = (size_t)(g.ny - 1) * ps;  // component stride of old/rhs
+
+  // the row being read; all loads are unconditional, with the row clamped
+  cx<R> np[6];
+  cx<double> nv[3], nold[2] = {{0.0, 0.0}, {0.0, 0.0}};
+  cx<double> nf[3];  // static force
+  double ng[3];      // feedback gains
+  auto load = [&](int r) {  // row r (its plane is r + 1)
+    const size_t off = (size_t)(r + 1) * ps + p;
 #pragma unroll
-  for (int c = 0; c < 3; c++)
+    for (int q = 0; q < 6; q++) np[q] = a.P[q * pstride + off];
 #pragma unroll
-    for (int j = 0; j < 4; j++) w[c][j] = force_row(a, der, c, a.src[c], y0 - 2 + j, p, col);
-  for (int iy = y0; iy <= y1; iy++) {
+    for (int c = 0; c < 3; c++) nv[c] = a.V[c * pstride + off];
+    if constexpr (FORCE) {
 #pragma unroll
-    for (int c = 0; c < 3; c++) w[c][4] = force_row(a, der, c, a.src[c], iy + 2, p, col);
-    const double *d = der + (size_t)(iy - 1) * 20;
-    auto S = [&](int f, int c) {
-      cx<double> s = scl(d[f * 5 + 0], w[c][0]);
+      for (int c = 0; c < 3; c++) {
+        nf[c] = fa.F0 ? fa.F0[c * pstride + off] : cx<double>{0.0, 0.0};
+        ng[c] = fa.src[c] >= 0 ? fa.gain[((size_t)c * g.Ny + (r + 1)) * (g.Nz + 1) + col] : 0.0;
+      }
+    }
+    if constexpr (RD) {  // explicit terms of the row that r completes
+      const size_t o = (size_t)(max(r - 2, 1) - 1) * ps + p;
+      const cx<R> oe = a.old[o], ov = a.old[rs + o];
+      nold[0] = cx<double>{(double)oe.x, (double)oe.y};
+      nold[1] = cx<double>{(double)ov.x, (double)ov.y};
+    }
+  };
+  // sums of the pending rows r-2..r+2 (slot m = row r-2+m): explicit and
+  // implicit parts of the D2v (v) and eta (e) equations
+  cx<double> sev[5], siv[5], see[5], sie[5];
 #pragma unroll
-      for (int j = 1; j < 5; j++) s = add(s, scl(d[f * 5 + j], w[c][j]));
-      return s;
-    };
-    const cx<double> d0u = S(0, 0), d0w = S(0, 2);
-    const cx<double> te = mean ? cx<double>{d0u.x, d0w.x} : sub(imul(be, d0u), imul(al, d0w));
-    const cx<double> tv = sub(sub(neg(scl(k2, S(0, 1))), imul(al, S(1, 0))), imul(be, S(1, 2)));
-    a.out[(size_t)(iy - 1) * ps + p] = te;
-    a.out[rs + (size_t)(iy - 1) * ps + p] = tv;
+  for (int m = 0; m < 5; m++) sev[m] = siv[m] = see[m] = sie[m] = cx<double>{0.0, 0.0};
+  load(y0 - 2);
+  for (int r = y0 - 2; r <= y1 + 2; r++) {
+    const auto D = [](cx<R> v) { return cx<double>{(double)v.x, (double)v.y}; };
+    const cx<double> uu = D(np[0]), vv = D(np[1]), ww = D(np[2]), uv = D(np[3]), vw = D(np[4]), uw = D(np[5]);
+    const cx<double> u = nv[0], v = nv[1], w = nv[2], old_e = nold[0], old_v = nold[1];
+    cx<double> F[3];
+    if constexpr (FORCE) {
+      // zero where nothing is to be read into the force, whatever F0 holds there
+      const bool in = r >= 1 && r <= g.ny - 1;
 #pragma unroll
-    for (int c = 0; c < 3; c++)
+      for (int c = 0; c < 3; c++) {
+        F[c] = cx<double>{0.0, 0.0};
+        if (in) {
+          F[c] = nf[c];
+          const int s = fa.src[c];
+          if (s >= 0) F[c] = add(F[c], scl(ng[c], s == 0 ? u : (s == 1 ? v : w)));
+        }
+      }
+    }
+    load(min(r + 1, g.ny + 1));
+    cx<double> G1, G2, G3, G4, eta;
+    G1.x = k2 * vv.x - al2 * uu.x - be2 * ww.x - 2.0 * albe * uw.x;
+    G1.y = k2 * vv.y - al2 * uu.y - be2 * ww.y - 2.0 * albe * uw.y;
+    G2 = cx<double>{-(al * uv.y + be * vw.y), al * uv.x + be * vw.x};
+    G3.x = albe * (uu.x - ww.x) + (be2 - al2) * uw.x;
+    G3.y = albe * (uu.y - ww.y) + (be2 - al2) * uw.y;
+    G4 = cx<double>{be * uv.y - al * vw.y, al * vw.x - be * uv.x};
+    eta = cx<double>{al * w.y - be * u.y, be * u.x - al * w.x};
+    if (mean) {
+      G4 = cx<double>{-uv.x, -vw.x};
+      eta = cx<double>{u.x, w.x};
+    }
+    cx<double> H0, H1, H3;  // force terms: D0(H0) + D1(H1) in D2v, D0(H3) in eta
+    if constexpr (FORCE) {
+      H0 = cx<double>{-k2 * F[1].x, -k2 * F[1].y};
+      H1 = cx<double>{al * F[0].y + be * F[2].y, -(al * F[0].x + be * F[2].x)};
+      H3 = mean ? cx<double>{F[0].x, F[2].x} : cx<double>{al * F[2].y - be * F[0].y, be * F[0].x - al * F[2].x};
+    }
+    const double *df = derF + (size_t)(r + 1) * 10;  // [m][d0, d1]
+    const double *d = derT + (size_t)(r + 1) * 20;  // [m][d0, d1, d2, d4]
 #pragma unroll
-      for (int j = 0; j < 4; j++) w[c][j] = w[c][j + 1];
+    for (int m = 0; m < 5; m++) {
+      const double d0 = d[4 * m], d1 = d[4 * m + 1], d2 = d[4 * m + 2], d4 = d[4 * m + 3];
+      const double w2 = d2 + k2 * d0, wi = cA * d2 + cB * d0 + a.ni * d4, wj = cC * d0 + a.ni * d2;
+      sev[m].x += d1 * G1.x + w2 * G2.x;
+      sev[m].y += d1 * G1.y + w2 * G2.y;
+      if constexpr (FORCE) {
+        const double f0 = df[2 * m], f1 = df[2 * m + 1];
+        sev[m].x += f0 * H0.x + f1 * H1.x;
+        sev[m].y += f0 * H0.y + f1 * H1.y;
+        see[m].x += f0 * H3.x;
+        see[m].y += f0 * H3.y;
+      }
+      siv[m].x += wi * v.x;
+      siv[m].y += wi * v.y;
+      see[m].x += d0 * G3.x + d1 * G4.x;
+      see[m].y += d0 * G3.y + d1 * G4.y;
+      sie[m].x += wj * eta.x;
+      sie[m].y += wj * eta.y;
+    }
+    const int iy = r - 2;  // complete now
+    if (iy >= y0) {
+      const size_t o = (size_t)(iy - 1) * ps + p;
+      cx<double> ee = see[0];
+      if (mean) {
+        ee.x += sc->meanpx;
+        ee.y += sc->meanpz;
+      }
+      cx<double> rv = {siv[0].x + a.ode1 * sev[0].x, siv[0].y + a.ode1 * sev[0].y};
+      cx<double> re = {sie[0].x + a.ode1 * ee.x, sie[0].y + a.ode1 * ee.y};
+      if constexpr (RD) {
+        rv = sub(rv, scl(a.ode2, old_v));
+        re = sub(re, scl(a.ode2, old_e));
+      }
+      a.rhs[rs + o] = rv;
+      a.rhs[o] = re;
+      if (a.store_old) {
+        a.old[rs + o] = cx<R>{(R)sev[0].x, (R)sev[0].y};
+        a.old[o] = cx<R>{(R)ee.x, (R)ee.y};
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+      sev[m] = sev[m + 1];
+      siv[m] = siv[m + 1];
+      see[m] = see[m + 1];
+      sie[m] = sie[m + 1];
+    }
+    sev[4] = siv[4] = see[4] = sie[4] = cx<double>{0.0, 0.0};
   }
 }
 
@@ -291,23 +255,44 @@ hipError_t launch_force(hipStream_t st, const ForceArgs &a) {
   return hipGetLastError();
 }
 
-hipError_t launch_force_terms(hipStream_t st, const ForceArgs &a) {
-  dim3 grid(pair_blocks(a.g, 256), (unsigned)((a.g.ny - 1 + a.chunk - 1) / a.chunk));
-  hipLaunchKernelGGL(k_force_terms, grid, dim3(256), 0, st, a, a.der);
-  return hipGetLastError();
+// Rows per chunk.  Every chunk reads four rows of its neighbours again, so
+// long chunks move least, but each is one serial walk: on small grids chunks
+// are halved until two waves per CU walk (31x64x31: 11.8 us with 3 rows, 42.8
+// with 48; 100x97x77: 67 us with 24, 99 with 96, 97 with 4).  From 1024
+// blocks of pairs on, short chunks make the whole grid advance through y as
+// one front, whose shared rows the memory-side cache still holds
+// (191x384x189: 1.21 ms with 8 rows, 1.30 with 48 or 96; 191x128x189 418 and
+// 445 us; 127x384x127, 510 blocks, 602 and 594 us, 578 with 96; with a body
+// force 1.19 and 1.29 ms at 191x384x189).
+static int rhs_chunk(const Geom &g) {
+  const int blocks = (g.npair + RHS_BLOCK - 1) / RHS_BLOCK;
+  if (blocks >= 1024) return 8;
+  int c = 96;
+  while (c > 2 && blocks * ((g.ny - 1 + c - 1) / c) < 2 * g.ncu) c = (c + 1) / 2;
+  return c;
+}
+
+template <typename R, bool FORCE>
+static void start_rhs(dim3 grid, hipStream_t st, const RhsArgs<R> &a, const ForceArgs &f) {
+  if (a.ode2 != 0.0)
+    hipLaunchKernelGGL((k_rhs<R, FORCE, true>), grid, dim3(RHS_BLOCK), 0, st, a, f, a.derT, f.derF, a.sc);
+  else
+    hipLaunchKernelGGL((k_rhs<R, FORCE, false>), grid, dim3(RHS_BLOCK), 0, st, a, f, a.derT, f.derF, a.sc);
 }
 
 template <typename R>
-hipError_t launch_rhs(hipStream_t st, const RhsArgs<R> &a) {
+hipError_t launch_rhs(hipStream_t st, const RhsArgs<R> &args, const ForceArgs *force) {
+  RhsArgs<R> a = args;
+  a.chunk = rhs_chunk(a.g);
   dim3 grid(pair_blocks(a.g, RHS_BLOCK), (unsigned)((a.g.ny - 1 + a.chunk - 1) / a.chunk));
-  if (a.force)
-    hipLaunchKernelGGL((k_rhs<R, true>), grid, dim3(RHS_BLOCK), 0, st, a, a.der, a.sc);
+  if (force)
+    start_rhs<R, true>(grid, st, a, *force);
   else
-    hipLaunchKernelGGL((k_rhs<R, false>), grid, dim3(RHS_BLOCK), 0, st, a, a.der, a.sc);
+    start_rhs<R, false>(grid, st, a, ForceArgs{});
   return hipGetLastError();
 }
 
-template hipError_t launch_rhs<double>(hipStream_t, const RhsArgs<double> &);
-template hipError_t launch_rhs<float>(hipStream_t, const RhsArgs<float> &);
+template hipError_t launch_rhs<double>(hipStream_t, const RhsArgs<double> &, const ForceArgs *);
+template hipError_t launch_rhs<float>(hipStream_t, const RhsArgs<float> &, const ForceArgs *);
 
 }  // namespace chan
