@@ -180,7 +180,7 @@ def main():
     roof = None
     if ktimes:
         groups = {"zinv": ["zinv"], "xpass": ["xpass"], "zfwd": ["zfwd"], "rhs": ["rhs"],
-                  "solve": ["solve_ve", "mean", "uw"]}
+                  "solve": ["solve_lds", "solve_ve", "mean", "uw"]}
         best = None
         for g, ks in groups.items():
             tot = sum(ktimes.get(k, (0, 0.0))[1] for k in ks)

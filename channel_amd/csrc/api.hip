@@ -109,6 +109,38 @@ __global__ __launch_bounds__(256) void k_copy(const double4 *__restrict__ a, dou
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) b[i] = a[i];
 }
 
+// the table of k_solve_lds (SROW)
+void solve_table(const HostSetup &h, int ny, std::vector<double> &t) {
+  const int n = ny - 1, m = n / 2;
+  t.assign((size_t)n * SROW, 0.0);
+  const int src[4] = {0, 10, 15, 5};  // d0, d2, d4, d1
+  for (int r = 0; r < n; r++)
+    for (int k = 0; k < 4; k++)
+      for (int j = 0; j < 5; j++) t[(size_t)r * SROW + 5 * k + j] = h.der[(size_t)r * 20 + src[k] + (r < m ? 4 - j : j)];
+  // D0 factors: from the upper wall the set-up's, from the lower one the same
+  // elimination in the mirrored rows
+  for (int r = n - 1; r >= m; r--)
+    for (int j = 0; j < 5; j++) t[(size_t)r * SROW + 20 + j] = h.d0fac[(size_t)r * 5 + j];
+  double l1[2] = {0, 0}, l2[2] = {0, 0};
+  for (int r = 0; r < m; r++) {
+    double *A = &t[(size_t)r * SROW + 20];
+    for (int j = 0; j < 5; j++) A[j] = t[(size_t)r * SROW + j];
+    if (r == 0) A[3] = A[4] = 0.0;  // the wall columns
+    if (r == 1) A[4] = 0.0;
+    A[3] -= A[4] * l2[1];
+    A[2] -= A[4] * l2[0];
+    A[2] -= A[3] * l1[1];
+    A[1] -= A[3] * l1[0];
+    A[2] = 1.0 / A[2];
+    A[0] *= A[2];
+    A[1] *= A[2];
+    for (int j = 0; j < 2; j++) {
+      l2[j] = l1[j];
+      l1[j] = A[j];
+    }
+  }
+}
+
 template <typename T>
 void twiddles(std::vector<cx<T>> &w, int n) {
   w.resize((size_t)fft::tw_table_size(n));
@@ -316,7 +348,8 @@ int chan_create(const chan_params *p, chan_ctx **out) {
   if ((rc = dalloc_bytes(&c->twz, (size_t)fft::tw_table_size(g.nzd) * esz))) return bail(rc);
   if ((rc = dalloc_bytes(&c->twx, (size_t)fft::tw_table_size(2 * g.nxd) * esz))) return bail(rc);
   if ((rc = dalloc(&c->der, (size_t)(g.ny - 1) * 20))) return bail(rc);
-  if ((rc = dalloc(&c->derT, (size_t)g.Ny * 20)) || (rc = dalloc(&c->derF, (size_t)g.Ny * 10))) return bail(rc);
+  if ((rc = dalloc(&c->derT, (size_t)g.Ny * 20)) || (rc = dalloc(&c->derF, (size_t)g.Ny * 10)) ||
+      (rc = dalloc(&c->tab, (size_t)(g.ny - 1) * SROW))) return bail(rc);
   if ((rc = dalloc(&c->d0fac, (size_t)(g.ny + 1) * 5))) return bail(rc);
   if ((rc = dalloc(&c->y, (size_t)g.Ny))) return bail(rc);
   if ((rc = dalloc(&c->dy, (size_t)g.ny + 1))) return bail(rc);
@@ -357,7 +390,10 @@ int chan_create(const chan_params *p, chan_ctx **out) {
           tf[(size_t)(r + 1) * 10 + 2 * m + f] = w;
         }
       }
-    if (hipMemcpy(c->derT, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
+    std::vector<double> tb;
+    solve_table(h, g.ny, tb);
+    if (hipMemcpy(c->tab, tb.data(), tb.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(c->derT, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(c->derF, tf.data(), tf.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
       return bail(fail(CHAN_E_STATE, "upload of the set-up failed"));
   }
@@ -384,7 +420,7 @@ int chan_destroy(chan_ctx *c) {
   }
   for (auto e : c->pool) hipEventDestroy(e);
   void *bufs[] = {c->V, c->old, c->rhs, c->L, c->col00, c->A, c->B, c->P, c->twz, c->twx,
-                  c->der, c->derT, c->derF, c->d0fac, c->y, c->dy, c->sc, c->stat, c->F0, c->gain, c->Fkeep};
+                  c->der, c->derT, c->derF, c->tab, c->d0fac, c->y, c->dy, c->sc, c->stat, c->F0, c->gain, c->Fkeep};
   for (void *b : bufs)
     if (b) hipFree(b);
   if (c->st) hipStreamDestroy(c->st);
@@ -691,12 +727,32 @@ int chan_linsolve(chan_ctx *c, double lambda) {
   s.L = c->L;
   s.der = c->der;
   std::memcpy(s.bc, c->hs.bc, sizeof s.bc);
+  for (int k = 0; k < 2; k++) {
+    const double *lw = c->hs.bc[k ? BC_V0 : BC_ETA0], *lg = c->hs.bc[k ? BC_V0M1 : BC_ETA0M1];
+    const double *hw = c->hs.bc[k ? BC_VN : BC_ETAN], *hg = c->hs.bc[k ? BC_VNP1 : BC_ETANP1];
+    for (int j = 0; j < 5; j++) {
+      s.wall[k].lo_ghost[j] = lg[j] / lg[0];
+      s.wall[k].lo_wall[j] = lw[j] / lw[1];
+      s.wall[k].hi_ghost[j] = hg[j] / hg[4];
+      s.wall[k].hi_wall[j] = hw[j] / hw[3];
+    }
+  }
   s.g = g;
   s.lambda = lambda;
   s.ni = c->prm.ni;
   s.u0 = c->prm.u0;
   s.uN = c->prm.uN;
-  if ((rc = timed(c, "solve_ve", [&] { return launch_solve(c->st, s); }))) return rc;
+  UwArgs u;
+  u.V = c->V;
+  u.tab = c->tab;
+  u.der = c->der;
+  u.d0fac = c->d0fac;
+  std::memcpy(u.bnd, c->hs.bnd, sizeof u.bnd);
+  u.g = g;
+  const bool lds = solve_in_lds(g);
+  if ((rc = lds ? timed(c, "solve_lds", [&] { return launch_solve_lds(c->st, s, u); })
+                : timed(c, "solve_ve", [&] { return launch_solve(c->st, s); })))
+    return rc;
   MeanArgs m;
   m.V = c->V;
   m.y = c->y;
@@ -710,13 +766,7 @@ int chan_linsolve(chan_ctx *c, double lambda) {
   m.cpi = c->prm.cpi;
   m.cpi_type = c->prm.cpi_type;
   if ((rc = timed(c, "mean", [&] { return launch_mean(c->st, m); }))) return rc;
-  UwArgs u;
-  u.V = c->V;
-  u.der = c->der;
-  u.d0fac = c->d0fac;
-  std::memcpy(u.bnd, c->hs.bnd, sizeof u.bnd);
-  u.g = g;
-  return timed(c, "uw", [&] { return launch_uw(c->st, u); });
+  return lds ? 0 : timed(c, "uw", [&] { return launch_uw(c->st, u); });
 }
 
 int chan_initial(chan_ctx *c) {

@@ -36,6 +36,16 @@ struct DevScalars {
   double pad[8];
 };
 
+// x / d as the division rounds it, from r = 1/d rounded to nearest: q = x r
+// and one correction by the exact remainder x - q d.  For finite x and
+// normal d the corrected quotient is the correctly rounded one (Markstein's
+// theorem: r within half an ulp of 1/d, q within an ulp of x/d); an
+// infinite x gives NaN.
+__device__ __forceinline__ double div_by(double x, double d, double r) {
+  const double q = x * r;
+  return fma(fma(-q, d, x), r, q);
+}
+
 // ---------------------------------------------------------- kernel args --
 template <typename R>
 struct RhsArgs {
@@ -63,6 +73,12 @@ struct ForceArgs {
   Geom g;
 };
 
+// Wall columns folded into the rows next to a wall: each ghost or wall row's
+// entries over its own diagonal one.
+struct WallRatios {
+  double lo_ghost[5], lo_wall[5], hi_ghost[5], hi_wall[5];
+};
+
 struct SolveArgs {
   cx<double> *V;           // [3][Ny][ps]; components 1,2 receive eta and v, pair
                            // slot npair of component 1 the ucor response
@@ -71,6 +87,7 @@ struct SolveArgs {
                            // row per (kx, |kz|) group, gs <= ps
   const double *der;
   double bc[8][5];
+  WallRatios wall[2];  // of eta, v
   Geom g;
   double lambda, ni, u0, uN;
 };
@@ -85,8 +102,14 @@ struct MeanArgs {
   int cpi, cpi_type;
 };
 
+// Doubles per row of the table of k_solve_lds: d0, d2, d4, d1 and the five
+// factors of the D0 band of a row, and one of padding.  The rows iy <= (ny-1)/2
+// are mirrored (weights in reverse order, D0 factorised from row 1 upwards).
+constexpr int SROW = 26;
+
 struct UwArgs {
   cx<double> *V;
+  const double *tab;  // [ny-1][SROW]
   const double *der;
   const double *d0fac;
   double bnd[10][5];
@@ -117,6 +140,8 @@ hipError_t launch_rhs(hipStream_t st, const RhsArgs<R> &a, const ForceArgs *forc
 hipError_t launch_force(hipStream_t st, const ForceArgs &a);
 hipError_t launch_stats(hipStream_t st, const cx<double> *V, const double *avg, double *out, const Geom &g);
 hipError_t launch_solve(hipStream_t st, const SolveArgs &a);
+bool solve_in_lds(const Geom &g);  // whether launch_solve_lds serves the grid, in place of launch_solve and launch_uw
+hipError_t launch_solve_lds(hipStream_t st, const SolveArgs &a, const UwArgs &u);
 hipError_t launch_mean(hipStream_t st, const MeanArgs &a);
 hipError_t launch_uw(hipStream_t st, const UwArgs &a);
 hipError_t launch_flowrate(hipStream_t st, const MeanArgs &a);

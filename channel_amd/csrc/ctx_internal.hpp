@@ -26,7 +26,7 @@ struct chan_ctx {
   // the split mode
   bool split = false;
   void *A = nullptr, *B = nullptr, *P = nullptr, *twz = nullptr, *twx = nullptr;
-  double *der = nullptr, *derT = nullptr, *derF = nullptr, *d0fac = nullptr, *y = nullptr, *dy = nullptr;
+  double *der = nullptr, *derT = nullptr, *derF = nullptr, *tab = nullptr, *d0fac = nullptr, *y = nullptr, *dy = nullptr;
   double *stat = nullptr;  // statistics: [3][ny+1] mean in, [7][ny+1] profiles out
   // body force: static field [3][Ny][ps] and feedback gains [3][Ny][Nz+1]
   chan::cx<double> *F0 = nullptr;

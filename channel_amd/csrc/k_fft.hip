@@ -142,16 +142,6 @@ __device__ __forceinline__ void block_max_atomic(double m, double *red, unsigned
   if (threadIdx.x == 0) atomicMax(out, (unsigned long long)__double_as_longlong(r));
 }
 
-// x / d as the division rounds it, from r = 1/d rounded to nearest: q = x r
-// and one correction by the exact remainder x - q d.  For finite x and
-// normal d the corrected quotient is the correctly rounded one (Markstein's
-// theorem: r within half an ulp of 1/d, q within an ulp of x/d); an
-// infinite x gives NaN, which the CFL check reports as it reports Inf.
-__device__ __forceinline__ double div_by(double x, double d, double r) {
-  const double q = x * r;
-  return fma(fma(-q, d, x), r, q);
-}
-
 // x modes per thread of the x pass: nxd >= 3(nx+1)/2 bounds Nx by M/3
 template <int E>
 constexpr int xmodes() {
@@ -380,7 +370,8 @@ __global__ __launch_bounds__((xteams<M, R>() * fft::Plan<M>::T), 2) void k_xpass
 
   // CFL maximum over the interior planes (dnsdata.f90:552-556).  FP64 gives
   // the reference's quotients (div_by: the correctly rounded divisions from
-  // three reciprocals per row); the split mode, whose samples are FP32,
+  // three reciprocals per row; its NaN for an infinite sample is reported as
+  // the CFL check reports Inf); the split mode, whose samples are FP32,
   // multiplies by the reciprocals (within an FP64 rounding of the quotients).
   if (cfl_on && iy >= 1 && iy <= g.ny - 1) {
     const double dyv = dy[iy];
