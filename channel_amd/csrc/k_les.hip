@@ -29,23 +29,23 @@ namespace chan {
 
 struct LesState {
   int n = 0;                  // samples (ny+1) Mx Mz
-  float *Gp = nullptr;        // [n][9] physical gradients
+  float *Gp = nullptr;        // [9][n] physical gradients
   float *Xf = nullptr;        // [n][46] features (host query)
-  __bf16 *Xb = nullptr;       // [n][64] normalised BF16 MLP inputs
   float *Y = nullptr;         // [n][6] MLP outputs
   float2 *T = nullptr;        // [6][ny+1][npair] spectral stresses
   float2 *twz = nullptr;      // [Mz] exp(+2 pi i k / Mz)
-  float2 *twx = nullptr;      // [Mx] exp(+2 pi i k / Mx)
+  float2 *phx = nullptr;      // [Nx][Mx up to XT] exp(+2 pi i ix xj / Mx)
+  float2 *phxT = nullptr;     // [Mx][Nx up to XT] the same
   double *ydc = nullptr;      // [ny+1][3] y-difference coefficients of rows iy-1, iy, iy+1
   int *ydr = nullptr;         // [ny+1] first row of each stencil
   double *yplus = nullptr;    // [ny+1] wall distance in wall units
-  float *norm = nullptr;      // [46 xmean][46 xscale][6 tmean][6 tscale]
+  float *norm = nullptr;      // [46 xmean][46 xscale][6 tmean][6 tscale][46 1/xscale]
   double *wall = nullptr;     // [2][5] wall-gradient stencils d140, d14n
 };
 
 void les_free(LesState *s) {
   if (!s) return;
-  void *b[] = {s->Gp, s->Xf, s->Xb, s->Y, s->T, s->twz, s->twx, s->ydc, s->ydr, s->yplus, s->norm, s->wall};
+  void *b[] = {s->Gp, s->Xf, s->Y, s->T, s->twz, s->phx, s->phxT, s->ydc, s->ydr, s->yplus, s->norm, s->wall};
   for (void *p : b)
     if (p) (void)hipFree(p);
   delete s;
@@ -76,67 +76,124 @@ LesGeom les_geom(const chan_ctx *c) {
   return q;
 }
 
-__device__ __forceinline__ float2 cmulf(float2 a, float2 b) { return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
+// a b with its fused operations written out, so that the sums formed from it do
+// not depend on how the compiler would fuse them
+__device__ __forceinline__ float2 cmulf(float2 a, float2 b) {
+  return make_float2(fmaf(a.x, b.x, -(a.y * b.y)), fmaf(a.y, b.x, a.x * b.y));
+}
 
-// The three derivatives (d = x, y, z) of component c on row iy, in physical
-// space: Gp[(iy Mx + x) Mz + z][3c + d].  One block per (row, component);
-// LDS holds the spectral coefficients of one derivative and its z transform.
-__global__ __launch_bounds__(256) void k_les_grad(const cx<double> *__restrict__ V, LesGeom q,
-                                                  const double *__restrict__ ydc, const int *__restrict__ ydr,
-                                                  const float2 *__restrict__ twz, const float2 *__restrict__ twx,
-                                                  float *__restrict__ Gp) {
-  extern __shared__ float2 sm[];
-  float2 *S = sm;             // [npair]
-  float2 *H = sm + q.npair;   // [Nx][Mz]
-  const int iy = blockIdx.x, c = blockIdx.y;
+// The transforms below are direct sums whose terms a thread adds in index order.
+// One output per thread, they spent their time on a modulo and two or three LDS
+// reads per term (943 us for the gradients at 31x64x31, 208 for the stresses);
+// a thread now takes a tile of outputs that share each term's operand, with the
+// phase index advanced by addition, and a block one derivative or stress of one
+// row (65 and 66 us; the LDS reads of the shared operands bound them now).
+constexpr int ZT = 8;     // x modes per thread in the z sums
+constexpr int XT = 8;     // x points (or modes) per thread in the x sums
+constexpr int GT = 384;   // threads: 8 x 96 points of the 96 x 96 grid in whole rounds
+
+__host__ __device__ __forceinline__ int round_up(int n, int k) { return (n + k - 1) / k * k; }
+// The phases of the x sums, e^{+2 pi i ix xj / Mx}, come as [Nx][Mx up to XT] and
+// transposed as [Mx][Nx up to XT].  k_les_grad stages them in LDS where they fit
+// beside the rest (PL: 65 us for 74 at 31x64x31); k_les_tau, whose plane already
+// fills LDS, reads them through the cache (66 us for 74: two blocks per CU
+// instead of one).
+inline size_t grad_phases(const LesGeom &q) { return sizeof(float2) * (size_t)q.Nx * round_up(q.Mx, XT); }
+inline size_t tau_phases(const LesGeom &q) { return sizeof(float2) * (size_t)q.Mx * round_up(q.Nx, XT); }
+// the rest of k_les_grad: S [Nz][Nx up to ZT], H [Nx][Mz], the z phases
+inline size_t grad_lds(const LesGeom &q) {
+  return sizeof(float2) * ((size_t)q.Nz * round_up(q.Nx, ZT) + (size_t)q.Nx * q.Mz + q.Mz);
+}
+constexpr size_t LDS_MAX = 160 * 1024;
+
+// Derivative d = x, y, z of component c on row iy in physical space:
+// Gp[3c + d][(iy Mx + x) Mz + z].  One block per (row, 3c + d).
+template <bool PL>
+__global__ __launch_bounds__(GT) void k_les_grad(const cx<double> *__restrict__ V, LesGeom q,
+                                                 const double *__restrict__ ydc, const int *__restrict__ ydr,
+                                                 const float2 *__restrict__ twz, const float2 *__restrict__ phx,
+                                                 float *__restrict__ Gp) {
+  extern __shared__ __align__(16) float2 sm[];
+  const int NxP = round_up(q.Nx, ZT), MxP = round_up(q.Mx, XT);
+  float2 *S = sm;                         // [Nz][NxP] spectral coefficients
+  float2 *XL = S + (size_t)q.Nz * NxP;    // [Nx][MxP] phases of the x sum (PL)
+  float2 *H = XL + (PL ? (size_t)q.Nx * MxP : 0);  // [Nx][Mz] after the z sum
+  float2 *Z = H + (size_t)q.Nx * q.Mz;    // [Mz] e^{+2 pi i k / Mz}
+  const int iy = blockIdx.x, c = blockIdx.y / 3, d = blockIdx.y % 3;
   const size_t cs = (size_t)c * q.Ny * q.ps;
-  for (int d = 0; d < 3; d++) {
-    for (int p = threadIdx.x; p < q.npair; p += 256) {
-      const int ix = p / q.Nz, iz = p % q.Nz - q.nz;
-      float2 s;
-      if (d == 1) {
-        const int r0 = ydr[iy];
-        double re = 0.0, im = 0.0;
-        for (int k = 0; k < 3; k++) {
-          const cx<double> v = V[cs + (size_t)(r0 + k + 1) * q.ps + p];
-          re += ydc[3 * iy + k] * v.x;
-          im += ydc[3 * iy + k] * v.y;
-        }
-        s = make_float2((float)re, (float)im);
-      } else {
-        const cx<double> v = V[cs + (size_t)(iy + 1) * q.ps + p];
-        const double k = d == 0 ? q.alfa0 * ix : q.beta0 * iz;  // i k v
-        s = make_float2((float)(-k * v.y), (float)(k * v.x));
+  for (int i = threadIdx.x; i < q.Mz; i += GT) Z[i] = twz[i];
+  if constexpr (PL)
+    for (int i = threadIdx.x; i < q.Nx * MxP; i += GT) XL[i] = phx[i];
+  for (int i = threadIdx.x; i < q.Nz * (NxP - q.Nx); i += GT)
+    S[(i / (NxP - q.Nx)) * NxP + q.Nx + i % (NxP - q.Nx)] = make_float2(0.f, 0.f);
+  for (int p = threadIdx.x; p < q.npair; p += GT) {
+    const int ix = p / q.Nz, j = p % q.Nz, iz = j - q.nz;
+    float2 s;
+    if (d == 1) {
+      const int r0 = ydr[iy];
+      double re = 0.0, im = 0.0;
+      for (int k = 0; k < 3; k++) {
+        const cx<double> v = V[cs + (size_t)(r0 + k + 1) * q.ps + p];
+        re += ydc[3 * iy + k] * v.x;
+        im += ydc[3 * iy + k] * v.y;
       }
-      S[p] = s;
+      s = make_float2((float)re, (float)im);
+    } else {
+      const cx<double> v = V[cs + (size_t)(iy + 1) * q.ps + p];
+      const double k = d == 0 ? q.alfa0 * ix : q.beta0 * iz;  // i k v
+      s = make_float2((float)(-k * v.y), (float)(k * v.x));
     }
-    __syncthreads();
-    // z: H[ix][zk] = sum_iz S e^{+2 pi i iz zk / Mz}
-    for (int o = threadIdx.x; o < q.Nx * q.Mz; o += 256) {
-      const int ix = o / q.Mz, zk = o % q.Mz;
-      float2 acc = make_float2(0.f, 0.f);
-      for (int j = 0; j < q.Nz; j++) {
-        const int iz = j - q.nz;
-        const int e = (int)(((long)((iz % q.Mz) + q.Mz) * zk) % q.Mz);
-        const float2 t = cmulf(S[ix * q.Nz + j], twz[e]);
-        acc.x += t.x;
-        acc.y += t.y;
+    S[j * NxP + ix] = s;
+  }
+  __syncthreads();
+  // z: H[ix][zk] = sum_iz S e^{+2 pi i iz zk / Mz}, ZT modes ix at a time
+  for (int o = threadIdx.x; o < (NxP / ZT) * q.Mz; o += GT) {
+    const int ix0 = (o / q.Mz) * ZT, zk = o % q.Mz;
+    float2 acc[ZT];
+#pragma unroll
+    for (int k = 0; k < ZT; k++) acc[k] = make_float2(0.f, 0.f);
+    int e = (int)(((long)(q.Mz - q.nz % q.Mz) * zk) % q.Mz);  // phase of iz = -nz
+    for (int j = 0; j < q.Nz; j++) {
+      const float2 w = Z[e];
+      e += zk;
+      e -= e >= q.Mz ? q.Mz : 0;
+      const float2 *Sj = S + j * NxP + ix0;
+#pragma unroll
+      for (int k = 0; k < ZT; k++) {
+        const float2 t = cmulf(Sj[k], w);
+        acc[k].x += t.x;
+        acc[k].y += t.y;
       }
-      H[o] = acc;
     }
-    __syncthreads();
-    // x: Hermitian sum over kx
-    for (int o = threadIdx.x; o < q.Mx * q.Mz; o += 256) {
-      const int xj = o / q.Mz, zk = o % q.Mz;
-      float f = H[zk].x, g = 0.f;
-      for (int ix = 1; ix < q.Nx; ix++) {
-        const float2 t = cmulf(H[ix * q.Mz + zk], twx[(ix * xj) % q.Mx]);
-        g += t.x;
+#pragma unroll
+    for (int k = 0; k < ZT; k++)
+      if (ix0 + k < q.Nx) H[(ix0 + k) * q.Mz + zk] = acc[k];
+  }
+  __syncthreads();
+  // x: Hermitian sum over kx, XT points at a time
+  float *G = Gp + (size_t)blockIdx.y * (q.ny + 1) * q.Mx * q.Mz + (size_t)iy * q.Mx * q.Mz;
+  for (int o = threadIdx.x; o < (MxP / XT) * q.Mz; o += GT) {
+    const int x0 = (o / q.Mz) * XT, zk = o % q.Mz;
+    float g[XT];
+#pragma unroll
+    for (int k = 0; k < XT; k++) g[k] = 0.f;
+    for (int ix = 1; ix < q.Nx; ix++) {
+      const float2 h = H[ix * q.Mz + zk];
+      const float2 *Xi = PL ? XL + ix * MxP + x0 : phx + (size_t)ix * MxP + x0;
+#pragma unroll
+      for (int k = 0; k < XT; k++) {
+        const float2 t = cmulf(h, Xi[k]);
+        g[k] += t.x;
       }
-      f += 2.f * g;
-      Gp[((size_t)iy * q.Mx * q.Mz + o) * 9 + 3 * c + d] = f;
     }
-    __syncthreads();
+    const float f0 = H[zk].x;
+#pragma unroll
+    for (int k = 0; k < XT; k++) {
+      if (x0 + k >= q.Mx) break;
+      float f = f0;
+      f += 2.f * g[k];
+      G[(size_t)(x0 + k) * q.Mz + zk] = f;
+    }
   }
 }
 
@@ -157,70 +214,86 @@ __global__ void k_les_yplus(const cx<double> *__restrict__ V, LesGeom q, const d
   }
 }
 
-// One thread per sample: the 46 features, raw into Xf (when given) and
-// normalised BF16 into Xb (when given)
+// One thread per sample: its 46 features for the host query
 __global__ __launch_bounds__(256) void k_les_features(const float *__restrict__ Gp, LesGeom q,
-                                                      const double *__restrict__ yplus, const float *__restrict__ norm,
-                                                      float *__restrict__ Xf, __bf16 *__restrict__ Xb) {
+                                                      const double *__restrict__ yplus, float *__restrict__ Xf) {
   const int plane = q.Mx * q.Mz;
   const int n = (q.ny + 1) * plane;
   const int s = blockIdx.x * 256 + threadIdx.x;
   if (s >= n) return;
   const int iy = s / plane, o = s % plane;
   const int rows[5] = {iy, iy - 2, iy - 1, iy + 1, iy + 2};
-  float f[mlp::KP];
 #pragma unroll
   for (int k = 0; k < 5; k++) {
     const int r = min(max(rows[k], 0), q.ny);
-    const float *g = Gp + ((size_t)r * plane + o) * 9;
 #pragma unroll
-    for (int j = 0; j < 9; j++) f[9 * k + j] = g[j];
+    for (int j = 0; j < 9; j++) Xf[(size_t)s * 46 + 9 * k + j] = Gp[(size_t)j * n + (size_t)r * plane + o];
   }
-  f[45] = (float)yplus[iy];
-  if (Xf)
-    for (int j = 0; j < 46; j++) Xf[(size_t)s * 46 + j] = f[j];
-  if (Xb) {
-#pragma unroll
-    for (int j = 0; j < mlp::KP; j++)
-      Xb[(size_t)s * mlp::KP + j] = (__bf16)(j < 46 ? (f[j] - norm[j]) / norm[46 + j] : 0.0f);
-  }
+  Xf[(size_t)s * 46 + 45] = (float)yplus[iy];
+}
+
+// LDS of k_les_tau: the plane [Mx][Mz], H [Mz][Nx up to ZT], the z phases
+inline size_t tau_lds(const LesGeom &q) {
+  return sizeof(float) * (size_t)round_up(q.Mx * q.Mz, 4) + sizeof(float2) * ((size_t)q.Mz * round_up(q.Nx, ZT) + q.Mz);
 }
 
 // Spectral stresses of row iy, component qq: T = (1/(Mx Mz)) sum tau e^{-i(kx x + kz z)}
-__global__ __launch_bounds__(256) void k_les_tau(const float *__restrict__ Y, LesGeom q, const float *__restrict__ norm,
-                                                 const float2 *__restrict__ twz, const float2 *__restrict__ twx,
-                                                 float2 *__restrict__ T) {
-  extern __shared__ float2 sm[];
-  float *P = reinterpret_cast<float *>(sm);        // [Mx][Mz]
-  float2 *H = sm + (q.Mx * q.Mz + 1) / 2;         // [Nx][Mz]
+__global__ __launch_bounds__(GT) void k_les_tau(const float *__restrict__ Y, LesGeom q, const float *__restrict__ norm,
+                                                const float2 *__restrict__ twz, const float2 *__restrict__ phxT,
+                                                float2 *__restrict__ T) {
+  extern __shared__ __align__(16) float2 sm[];
+  const int NxP = round_up(q.Nx, XT);
+  static_assert(XT == ZT, "one padding of the x modes");
+  float *P = reinterpret_cast<float *>(sm);                                // [Mx][Mz]
+  float2 *H = reinterpret_cast<float2 *>(P + round_up(q.Mx * q.Mz, 4));    // [Mz][NxP]
+  float2 *Z = H + (size_t)q.Mz * NxP;                                      // [Mz]
   const int iy = blockIdx.x, qq = blockIdx.y;
   const int plane = q.Mx * q.Mz;
   const float tm = norm[92 + qq], ts = norm[98 + qq];
-  for (int o = threadIdx.x; o < plane; o += 256) P[o] = Y[((size_t)iy * plane + o) * 6 + qq] * ts + tm;
+  for (int i = threadIdx.x; i < q.Mz; i += GT) Z[i] = twz[i];
+  for (int o = threadIdx.x; o < plane; o += GT) P[o] = Y[((size_t)iy * plane + o) * 6 + qq] * ts + tm;
   __syncthreads();
-  for (int o = threadIdx.x; o < q.Nx * q.Mz; o += 256) {
-    const int ix = o / q.Mz, zk = o % q.Mz;
-    float2 acc = make_float2(0.f, 0.f);
+  for (int o = threadIdx.x; o < (NxP / XT) * q.Mz; o += GT) {
+    const int ix0 = (o / q.Mz) * XT, zk = o % q.Mz;
+    float2 acc[XT];
+#pragma unroll
+    for (int k = 0; k < XT; k++) acc[k] = make_float2(0.f, 0.f);
     for (int xj = 0; xj < q.Mx; xj++) {
-      const float2 w = twx[(ix * xj) % q.Mx];
       const float v = P[xj * q.Mz + zk];
-      acc.x += v * w.x;
-      acc.y -= v * w.y;  // conj
+      const float2 *w = phxT + (size_t)xj * NxP + ix0;
+#pragma unroll
+      for (int k = 0; k < XT; k++) {
+        acc[k].x = fmaf(v, w[k].x, acc[k].x);
+        acc[k].y = fmaf(-v, w[k].y, acc[k].y);  // conj
+      }
     }
-    H[o] = make_float2(acc.x / q.Mx, acc.y / q.Mx);
+#pragma unroll
+    for (int k = 0; k < XT; k++) H[zk * NxP + ix0 + k] = make_float2(acc[k].x / q.Mx, acc[k].y / q.Mx);
   }
   __syncthreads();
-  for (int p = threadIdx.x; p < q.npair; p += 256) {
-    const int ix = p / q.Nz, iz = p % q.Nz - q.nz;
-    float2 acc = make_float2(0.f, 0.f);
+  for (int o = threadIdx.x; o < (NxP / ZT) * q.Nz; o += GT) {
+    const int ix0 = (o / q.Nz) * ZT, j = o % q.Nz, iz = j - q.nz;
+    float2 acc[ZT];
+#pragma unroll
+    for (int k = 0; k < ZT; k++) acc[k] = make_float2(0.f, 0.f);
+    const int de = ((iz % q.Mz) + q.Mz) % q.Mz;  // phase step of iz
+    int e = 0;
     for (int zk = 0; zk < q.Mz; zk++) {
-      const int e = (int)(((long)((iz % q.Mz) + q.Mz) * zk) % q.Mz);
-      const float2 w = make_float2(twz[e].x, -twz[e].y);
-      const float2 t = cmulf(H[ix * q.Mz + zk], w);
-      acc.x += t.x;
-      acc.y += t.y;
+      const float2 w = make_float2(Z[e].x, -Z[e].y);
+      e += de;
+      e -= e >= q.Mz ? q.Mz : 0;
+#pragma unroll
+      for (int k = 0; k < ZT; k++) {
+        const float2 t = cmulf(H[zk * NxP + ix0 + k], w);
+        acc[k].x += t.x;
+        acc[k].y += t.y;
+      }
     }
-    T[((size_t)qq * (q.ny + 1) + iy) * q.npair + p] = make_float2(acc.x / q.Mz, acc.y / q.Mz);
+#pragma unroll
+    for (int k = 0; k < ZT; k++)
+      if (ix0 + k < q.Nx)
+        T[((size_t)qq * (q.ny + 1) + iy) * q.npair + (ix0 + k) * q.Nz + j] =
+            make_float2(acc[k].x / q.Mz, acc[k].y / q.Mz);
   }
 }
 
@@ -290,17 +363,22 @@ int les_state(chan_ctx *c, LesState **out) {
     return code;
   };
   const size_t n = (size_t)s->n;
-  if ((rc = lmal(&s->Gp, n * 9)) || (rc = lmal(&s->Xf, n * 46)) || (rc = lmal(&s->Xb, n * mlp::KP)) ||
-      (rc = lmal(&s->Y, n * 6)) || (rc = lmal(&s->T, (size_t)6 * (q.ny + 1) * q.npair)) ||
-      (rc = lmal(&s->twz, (size_t)q.Mz)) || (rc = lmal(&s->twx, (size_t)q.Mx)) ||
+  if ((rc = lmal(&s->Gp, n * 9)) || (rc = lmal(&s->Y, n * 6)) || (rc = lmal(&s->T, (size_t)6 * (q.ny + 1) * q.npair)) ||
+      (rc = lmal(&s->twz, (size_t)q.Mz)) || (rc = lmal(&s->phx, grad_phases(q) / sizeof(float2))) || (rc = lmal(&s->phxT, tau_phases(q) / sizeof(float2))) ||
       (rc = lmal(&s->ydc, (size_t)3 * (q.ny + 1))) || (rc = lmal(&s->ydr, (size_t)q.ny + 1)) ||
-      (rc = lmal(&s->yplus, (size_t)q.ny + 1)) || (rc = lmal(&s->norm, (size_t)104)) || (rc = lmal(&s->wall, (size_t)10)))
+      (rc = lmal(&s->yplus, (size_t)q.ny + 1)) || (rc = lmal(&s->norm, (size_t)mlp::NORM_RECIP + 46)) || (rc = lmal(&s->wall, (size_t)10)))
     return bail(rc);
   // twiddles
   std::vector<float2> tz(q.Mz), tx(q.Mx);
   const double pi2 = 2.0 * 3.14159265358979323846;
   for (int k = 0; k < q.Mz; k++) tz[k] = make_float2((float)cos(pi2 * k / q.Mz), (float)sin(pi2 * k / q.Mz));
   for (int k = 0; k < q.Mx; k++) tx[k] = make_float2((float)cos(pi2 * k / q.Mx), (float)sin(pi2 * k / q.Mx));
+  const int MxP = round_up(q.Mx, XT), NxP = round_up(q.Nx, XT);
+  std::vector<float2> px((size_t)q.Nx * MxP), pxT((size_t)q.Mx * NxP);
+  for (int ix = 0; ix < q.Nx; ix++)
+    for (int xj = 0; xj < MxP; xj++) px[(size_t)ix * MxP + xj] = tx[(int)((long long)ix * xj % q.Mx)];
+  for (int xj = 0; xj < q.Mx; xj++)
+    for (int ix = 0; ix < NxP; ix++) pxT[(size_t)xj * NxP + ix] = tx[(int)((long long)ix * xj % q.Mx)];
   // second-order differences on the stretched rows 0..ny (numpy.gradient, edge_order 2)
   const double *y = c->hs.y + 1;  // y[iy], iy = 0..ny
   const int ny = q.ny;
@@ -332,7 +410,8 @@ int les_state(chan_ctx *c, LesState **out) {
   std::memcpy(wall, c->hs.bnd[B_D140], 5 * sizeof(double));
   std::memcpy(wall + 5, c->hs.bnd[B_D14N], 5 * sizeof(double));
   if (hipMemcpy(s->twz, tz.data(), tz.size() * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(s->twx, tx.data(), tx.size() * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess ||
+      hipMemcpy(s->phx, px.data(), px.size() * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess ||
+      hipMemcpy(s->phxT, pxT.data(), pxT.size() * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(s->ydc, dc.data(), dc.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(s->ydr, dr.data(), dr.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(s->wall, wall, sizeof wall, hipMemcpyHostToDevice) != hipSuccess)
@@ -342,19 +421,30 @@ int les_state(chan_ctx *c, LesState **out) {
   return 0;
 }
 
-// gradients, y+ and features of the resident field (Xf and/or Xb)
-int les_features(chan_ctx *c, LesState *s, bool raw, bool bf16) {
+// The closure runs where one row's transform fits in 64 KiB: spectral
+// coefficients and one z-transformed row, or one physical plane and the same.
+int les_fits(const LesGeom &q, bool stresses) {
+  const size_t h = sizeof(float2) * (size_t)q.Nx * q.Mz;
+  const size_t b = h + (stresses ? sizeof(float) * ((size_t)q.Mx * q.Mz + 1) + 16 : sizeof(float2) * (size_t)q.npair);
+  if (b > 64 * 1024) return set_error(CHAN_E_SIZE, "closure grid too large (%zu bytes of LDS per row)", b);
+  return 0;  // grad_lds and tau_lds, at most twice that for the padding of Nx >= 4, then fit in 160 KiB
+}
+
+// gradients and y+ of the resident field
+int les_gradients(chan_ctx *c, LesState *s) {
   const LesGeom q = les_geom(c);
-  const size_t lds_g = sizeof(float2) * ((size_t)q.npair + (size_t)q.Nx * q.Mz);
-  if (lds_g > 64 * 1024) return set_error(CHAN_E_SIZE, "closure grid too large (%zu bytes of LDS per row)", lds_g);
-  hipLaunchKernelGGL(k_les_grad, dim3(q.ny + 1, 3), dim3(256), lds_g, c->st, c->V, q, s->ydc, s->ydr, s->twz, s->twx,
-                     s->Gp);
+  int rc;
+  if ((rc = les_fits(q, false))) return rc;
+  const size_t lds = grad_lds(q), all = lds + grad_phases(q);
+  if (all <= LDS_MAX)
+    hipLaunchKernelGGL(k_les_grad<true>, dim3(q.ny + 1, 9), dim3(GT), all, c->st, c->V, q, s->ydc, s->ydr, s->twz, s->phx,
+                       s->Gp);
+  else
+    hipLaunchKernelGGL(k_les_grad<false>, dim3(q.ny + 1, 9), dim3(GT), lds, c->st, c->V, q, s->ydc, s->ydr, s->twz,
+                       s->phx, s->Gp);
   LCHK(hipGetLastError());
   hipLaunchKernelGGL(k_les_yplus, dim3(1), dim3(256), 0, c->st, c->V, q, s->wall, c->y, c->prm.ymin, c->prm.ymax,
                      c->prm.ni, s->yplus);
-  LCHK(hipGetLastError());
-  hipLaunchKernelGGL(k_les_features, dim3((s->n + 255) / 256), dim3(256), 0, c->st, s->Gp, q, s->yplus, s->norm,
-                     raw ? s->Xf : nullptr, bf16 ? s->Xb : nullptr);
   LCHK(hipGetLastError());
   return 0;
 }
@@ -372,7 +462,10 @@ int chan_les_features(chan_ctx *c, float *X) {
   LesState *s;
   int rc;
   if ((rc = les_state(c, &s))) return rc;
-  if ((rc = les_features(c, s, true, false))) return rc;
+  if (!s->Xf && (rc = lmal(&s->Xf, (size_t)s->n * 46))) return rc;
+  if ((rc = les_gradients(c, s))) return rc;
+  hipLaunchKernelGGL(k_les_features, dim3((s->n + 255) / 256), dim3(256), 0, c->st, s->Gp, les_geom(c), s->yplus, s->Xf);
+  LCHK(hipGetLastError());
   LCHK(hipMemcpyAsync(X, s->Xf, sizeof(float) * 46 * (size_t)s->n, hipMemcpyDeviceToHost, c->st));
   LCHK(hipStreamSynchronize(c->st));
   return 0;
@@ -392,13 +485,15 @@ int chan_les_closure_force(chan_ctx *c, chan_mlp *m, const float *norm) {
   if ((rc = les_state(c, &s))) return rc;
   for (int j = 0; j < 46; j++)
     if (!(norm[46 + j] > 0.0f)) return set_error(CHAN_E_ARG, "feature scale %d is not positive", j);
-  LCHK(hipMemcpyAsync(s->norm, norm, sizeof(float) * 104, hipMemcpyHostToDevice, c->st));
-  if ((rc = les_features(c, s, false, true))) return rc;
-  LCHK(mlp::forward_device(m, s->Xb, s->n, s->Y, c->st));
+  float nv[mlp::NORM_RECIP + 46];
+  std::memcpy(nv, norm, sizeof(float) * mlp::NORM_RECIP);
+  for (int j = 0; j < 46; j++) nv[mlp::NORM_RECIP + j] = 1.0f / norm[46 + j];
+  LCHK(hipMemcpyAsync(s->norm, nv, sizeof nv, hipMemcpyHostToDevice, c->st));
+  if ((rc = les_gradients(c, s))) return rc;
   const LesGeom q = les_geom(c);
-  const size_t lds_t = sizeof(float) * ((size_t)q.Mx * q.Mz + 1) + sizeof(float2) * (size_t)q.Nx * q.Mz + 16;
-  if (lds_t > 64 * 1024) return set_error(CHAN_E_SIZE, "closure grid too large (%zu bytes of LDS per row)", lds_t);
-  hipLaunchKernelGGL(k_les_tau, dim3(q.ny + 1, 6), dim3(256), lds_t, c->st, s->Y, q, s->norm, s->twz, s->twx, s->T);
+  LCHK(mlp::forward_gradients(m, mlp::LesSource{s->Gp, s->norm, s->yplus, s->n, q.Mx * q.Mz, q.ny}, s->Y, c->st));
+  if ((rc = les_fits(q, true))) return rc;
+  hipLaunchKernelGGL(k_les_tau, dim3(q.ny + 1, 6), dim3(GT), tau_lds(q), c->st, s->Y, q, s->norm, s->twz, s->phxT, s->T);
   LCHK(hipGetLastError());
   if (!c->F0) {
     if ((rc = lmal(&c->F0, 3 * (size_t)q.Ny * q.ps))) return rc;

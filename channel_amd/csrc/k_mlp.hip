@@ -4,20 +4,23 @@
 // counterpart; the network maps box-filtered velocity gradients to the six
 // subgrid stresses.
 //
-// Matrix-core fragments (16x16x32, one wavefront):
-//   A (16 x 32): lane l holds A[l % 16][8 (l / 16) + j], j = 0..7
-//   B (32 x 16): lane l holds B[8 (l / 16) + j][l % 16]
-//   D (16 x 16): lane l holds D[4 (l / 16) + i][l % 16], i = 0..3
-// Layers are padded to 64 inputs (46 features + zeros) and 16 outputs (6 +
-// zeros).  Weights are kept twice in BF16: Woi[l][out][in] feeds the forward
-// pass (8 consecutive inputs per lane), Wio[l][in][out] the backward data
-// pass; biases stay FP32.
+// Matrix-core fragments (16x16x32, one wavefront, lane l, q = l / 16):
+//   A (16 x 32): A[l % 16][8 q + j], j = 0..7
+//   B (32 x 16): B[8 q + j][l % 16]
+//   D (16 x 16): D[4 q + i][l % 16], i = 0..3
+// Samples sit in the columns (B and D), units in the rows: a layer is D =
+// W^T B with the weights as A fragments, which a wave keeps in registers for
+// all its samples, and four swaps of register pairs with lane rows turn the D
+// layout of one layer into the B layout of the next (next_operand), so that
+// activations never leave the registers between layers.  Layers are padded to
+// 64 inputs (46 features + zeros) and 16 outputs (6 + zeros).  Weights are kept
+// twice in BF16: Woi[l][out][in] feeds the forward pass (8 consecutive inputs
+// per lane), Wio[l][in][out] the backward data pass; biases stay FP32.
 //
-// Kernels: k_mlp_fwd (inference, or training forward storing activations and
-// the loss gradient), k_mlp_bwd (dz of one layer from the next), k_mlp_wgrad
-// (weight and bias gradients of one layer as per-block partial sums over
-// samples), k_mlp_reduce (sum of the partials in block order: deterministic)
-// and k_mlp_adam (Adam on FP32 master weights, refreshing the BF16 copies).
+// Kernels: k_mlp_fwd, k_mlp_fwd_les (inference from BF16 or FP32 rows, from the
+// closure's gradients), k_mlp_grad (forward, backward and weight gradients of a minibatch
+// in one pass, per-block partial sums) and k_mlp_update (sums the partials in a
+// fixed order, then Adam on the FP32 master weights, refreshing the BF16 copies).
 #include "chan_internal.hpp"
 #include "mlp_internal.hpp"
 
@@ -31,12 +34,6 @@ __device__ __forceinline__ f32x4 mma(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __device__ __forceinline__ bf16x8 load8(const __bf16 *p) { return *reinterpret_cast<const bf16x8 *>(p); }
 __device__ __forceinline__ bf16x8 zero8() {
   bf16x8 z;
@@ -45,239 +42,454 @@ __device__ __forceinline__ bf16x8 zero8() {
   return z;
 }
 
-// ------------------------------------------------------------ forward --
-// One wave per 16-sample tile.  TRAIN: stores the hidden activations act[l]
-// ([N][64] BF16, l = 0..2 for layers 1..3) and dy = 2 (y - t) / (6 N) as BF16
-// [N][16], and the block's squared-error sum; otherwise stores y [N][6].
-template <bool TRAIN>
-__global__ __launch_bounds__(256) void k_mlp_fwd(Weights w, const __bf16 *__restrict__ X, const float *__restrict__ Tg,
-                                                 int n, float inv_count, float *__restrict__ Y,
-                                                 __bf16 *__restrict__ act, __bf16 *__restrict__ dy,
-                                                 float *__restrict__ loss_part) {
-  __shared__ __align__(16) __bf16 woi[WSIZE];
-  __shared__ __align__(16) __bf16 tile[4][16 * 64];
-  __shared__ float lred[4];
-  for (int i = threadIdx.x; i < WSIZE / 8; i += 256)
-    reinterpret_cast<bf16x8 *>(woi)[i] = reinterpret_cast<const bf16x8 *>(w.woi)[i];
-  __syncthreads();
-  const int wv = threadIdx.x / 64, l = threadIdx.x % 64, c16 = l % 16, q = l / 16;
-  __bf16 *tl = tile[wv];
-  float lsum = 0.0f;
-  const int ntile = (n + 15) / 16;
-  for (int tt = blockIdx.x * 4 + wv; tt < ntile; tt += gridDim.x * 4) {
-    const int s0 = tt * 16;
-    // input fragments straight from global memory (rows past n read row n-1, masked later)
-    bf16x8 a[2];
-    {
-      const int row = min(s0 + c16, n - 1);
-      a[0] = load8(X + (size_t)row * KP + 8 * q);
-      a[1] = load8(X + (size_t)row * KP + 32 + 8 * q);
+// The next layer's B fragments from this layer's outputs: P[mt][h] packs the
+// outputs mt*16 + 4q + 2h, + 1 of the lane's sample.  Lane row q needs the units
+// ks*32 + 8q + j, which lane rows 2 (q & 1) + (j >> 2) hold for mt = 2 ks + (q >> 1):
+// exchanging the register pair with the upper half of the wave and then with the
+// odd rows puts them there.
+__device__ __forceinline__ void next_operand(const unsigned (&P)[4][2], bf16x8 (&b)[2]) {
+#pragma unroll
+  for (int ks = 0; ks < 2; ks++) {
+    unsigned r[4];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const auto u = __builtin_amdgcn_permlane32_swap(P[2 * ks][h], P[2 * ks + 1][h], false, false);
+      const auto v = __builtin_amdgcn_permlane16_swap(u[0], u[1], false, false);
+      r[h] = v[0];
+      r[2 + h] = v[1];
     }
-#pragma unroll
-    for (int L = 0; L < 4; L++) {
-      const int nout = L < 3 ? H : OP;
-      const __bf16 *W = woi + WOFF[L];  // [out][64]
-      const float *b = w.bias + BOFF[L];
-      f32x4 acc[4];
-#pragma unroll
-      for (int nt = 0; nt < 4; nt++) {
-        if (nt * 16 >= nout) break;
-        acc[nt] = f32x4{0, 0, 0, 0};
-#pragma unroll
-        for (int ks = 0; ks < 2; ks++) acc[nt] = mma(a[ks], load8(W + (nt * 16 + c16) * KP + ks * 32 + 8 * q), acc[nt]);
-      }
-      if (L < 3) {
-        // bias, ReLU, BF16; the tile goes through LDS into the A layout
-#pragma unroll
-        for (int nt = 0; nt < 4; nt++) {
-          const int col = nt * 16 + c16;
-#pragma unroll
-          for (int i = 0; i < 4; i++) {
-            const float z = acc[nt][i] + b[col];
-            tl[(4 * q + i) * 64 + col] = (__bf16)(z > 0.0f ? z : 0.0f);
-          }
-        }
-        wave_sync();
-        a[0] = load8(tl + c16 * 64 + 8 * q);
-        a[1] = load8(tl + c16 * 64 + 32 + 8 * q);
-        if constexpr (TRAIN) {
-          const int row = s0 + c16;
-          if (row < n) {
-            __bf16 *dst = act + ((size_t)L * n + row) * KP;
-            *reinterpret_cast<bf16x8 *>(dst + 8 * q) = a[0];
-            *reinterpret_cast<bf16x8 *>(dst + 32 + 8 * q) = a[1];
-          }
-        }
-        wave_sync();
-      } else {
-        // output layer: lane holds y[4q + i][c16]
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const int row = s0 + 4 * q + i;
-          const float y = acc[0][i] + b[c16];
-          if (row < n && c16 < OUT) {
-            if constexpr (TRAIN) {
-              const float d = y - Tg[(size_t)row * OUT + c16];
-              lsum += d * d;
-              dy[(size_t)row * OP + c16] = (__bf16)(2.0f * d * inv_count);
-            } else {
-              Y[(size_t)row * OUT + c16] = y;
-            }
-          } else if (TRAIN && row < n) {
-            dy[(size_t)row * OP + c16] = (__bf16)0.0f;
-          }
-        }
-      }
-    }
-  }
-  if constexpr (TRAIN) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off, 64);
-    if (l == 0) lred[wv] = lsum;
-    __syncthreads();
-    if (threadIdx.x == 0) loss_part[blockIdx.x] = (lred[0] + lred[1]) + (lred[2] + lred[3]);
+    __builtin_memcpy(&b[ks], r, sizeof r);
   }
 }
 
-// ------------------------------------------------------ backward (data) --
-// dz of hidden layer L (0..2): dh = dz_next W_next^T, masked by act_L > 0.
-// dz_next is dy ([N][16]) for L = 2, else dz of layer L+1 ([N][64]).
-__global__ __launch_bounds__(256) void k_mlp_bwd(Weights w, int L, int n, const __bf16 *__restrict__ act,
-                                                 const __bf16 *__restrict__ dnext, __bf16 *__restrict__ dz) {
-  __shared__ __align__(16) __bf16 wio[64 * 64];
-  const int Lw = L + 1;                    // the layer whose weights carry the gradient back
-  const int kout = Lw < 3 ? H : OP;        // its outputs: the K of this product
-  for (int i = threadIdx.x; i < 64 * kout / 8; i += 256)
-    reinterpret_cast<bf16x8 *>(wio)[i] = reinterpret_cast<const bf16x8 *>(w.wio + WOFF[Lw])[i];  // [in][kout]
-  __syncthreads();
-  const int wv = threadIdx.x / 64, l = threadIdx.x % 64, c16 = l % 16, q = l / 16;
-  const int ntile = (n + 15) / 16;
-  const int dstride = Lw < 3 ? KP : OP;
-  for (int tt = blockIdx.x * 4 + wv; tt < ntile; tt += gridDim.x * 4) {
-    const int s0 = tt * 16;
-    const int row = min(s0 + c16, n - 1);
-    bf16x8 a[2];
-    a[0] = 8 * q < kout ? load8(dnext + (size_t)row * dstride + 8 * q) : zero8();
-    a[1] = kout > 32 ? load8(dnext + (size_t)row * dstride + 32 + 8 * q) : zero8();
-#pragma unroll
-    for (int nt = 0; nt < 4; nt++) {
-      const int col = nt * 16 + c16;  // input of layer Lw = output of layer L
-      f32x4 acc = {0, 0, 0, 0};
-      acc = mma(a[0], 8 * q < kout ? load8(wio + col * kout + 8 * q) : zero8(), acc);
-      if (kout > 32) acc = mma(a[1], load8(wio + col * kout + 32 + 8 * q), acc);
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int r = s0 + 4 * q + i;
-        if (r < n) {
-          const float h = (float)act[((size_t)L * n + r) * KP + col];
-          dz[(size_t)r * KP + col] = (__bf16)(h > 0.0f ? acc[i] : 0.0f);
-        }
-      }
-    }
-  }
+__device__ __forceinline__ unsigned pack2(__bf16 x, __bf16 y) {
+  unsigned short u, v;
+  __builtin_memcpy(&u, &x, 2);
+  __builtin_memcpy(&v, &y, 2);
+  return (unsigned)u | (unsigned)v << 16;
 }
 
-// ---------------------------------------------------- weight gradients --
-// dW_L = in_L^T dz_L and db_L = sum dz_L over the block's samples, with
-// in_0 = X and in_L = act_(L-1); dz_3 = dy.  Each block writes its partial
-// sums (dW [64][nout] then db [nout]) to part + blockIdx.x * PSIZE(L).
-__global__ __launch_bounds__(256) void k_mlp_wgrad(int L, int n, const __bf16 *__restrict__ X,
-                                                   const __bf16 *__restrict__ act, const __bf16 *__restrict__ dz,
-                                                   float *__restrict__ part, int chunk) {
-  __shared__ __align__(16) __bf16 tin[4][32 * 64];   // [sample][in] per wave
-  __shared__ __align__(16) __bf16 tdz[4][64 * 32];   // [out][sample] per wave
-  __shared__ float red[64 * 64 + 64];
-  const int nout = L < 3 ? H : OP, dstride = L < 3 ? KP : OP;
-  const __bf16 *in = L == 0 ? X : act + (size_t)(L - 1) * n * KP;
-  const int wv = threadIdx.x / 64, l = threadIdx.x % 64, c16 = l % 16, q = l / 16;
-  const int NT = nout / 16;
-  f32x4 acc[4][4];
+// The weights of the forward pass as A fragments, 104 registers, and the biases
+// in LDS.
+struct Layers {
+  bf16x8 h[3][4][2], o[2];
+  __device__ __forceinline__ void load(const Weights &w, int c16, int q) {
 #pragma unroll
-  for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-    for (int nt = 0; nt < 4; nt++) acc[mt][nt] = f32x4{0, 0, 0, 0};
-  float bsum = 0.0f;  // lane l < nout: sum of dz[.][l]
-  const int s_begin = blockIdx.x * chunk, s_end = min(n, s_begin + chunk);
-  for (int s0 = s_begin + wv * 32; s0 < s_end; s0 += 4 * 32) {
-    // stage 32 samples: inputs row-major, dz transposed; rows past the chunk are zero
-    for (int e = l; e < 32 * 8; e += 64) {
-      const int r = e / 8, k8 = (e % 8) * 8, s = s0 + r;
-      *reinterpret_cast<bf16x8 *>(&tin[wv][r * 64 + k8]) = s < s_end ? load8(in + (size_t)s * KP + k8) : zero8();
-    }
-    for (int e = l; e < 32 * nout; e += 64) {
-      const int r = e / nout, o = e % nout, s = s0 + r;
-      const __bf16 v = s < s_end ? dz[(size_t)s * dstride + o] : (__bf16)0.0f;
-      tdz[wv][o * 32 + r] = v;
-    }
-    wave_sync();
-    // A[m = in][k = sample] = tin[k][m]; B[k = sample][n = out] = tdz[n][k]
-#pragma unroll
-    for (int mt = 0; mt < 4; mt++) {
-      bf16x8 a;
-#pragma unroll
-      for (int j = 0; j < 8; j++) a[j] = tin[wv][(8 * q + j) * 64 + mt * 16 + c16];
-#pragma unroll
-      for (int nt = 0; nt < 4; nt++) {
-        if (nt >= NT) break;
-        acc[mt][nt] = mma(a, load8(&tdz[wv][(nt * 16 + c16) * 32 + 8 * q]), acc[mt][nt]);
-      }
-    }
-    if (l < nout) {
-      float s = 0.0f;
-#pragma unroll
-      for (int r = 0; r < 32; r++) s += (float)tdz[wv][l * 32 + r];
-      bsum += s;
-    }
-    wave_sync();
-  }
-  // block reduction of the four waves' sums, in wave order
-  for (int i = threadIdx.x; i < 64 * 64 + 64; i += 256) red[i] = 0.0f;
-  __syncthreads();
-  for (int w2 = 0; w2 < 4; w2++) {
-    if (wv == w2) {
+    for (int L = 0; L < 3; L++)
 #pragma unroll
       for (int mt = 0; mt < 4; mt++)
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++) {
-          if (nt >= NT) break;
+        for (int ks = 0; ks < 2; ks++) h[L][mt][ks] = load8(w.woi + WOFF[L] + (mt * 16 + c16) * KP + ks * 32 + 8 * q);
 #pragma unroll
-          for (int i = 0; i < 4; i++) red[(mt * 16 + 4 * q + i) * nout + nt * 16 + c16] += acc[mt][nt][i];
+    for (int ks = 0; ks < 2; ks++) o[ks] = load8(w.woi + WOFF[3] + c16 * KP + ks * 32 + 8 * q);
+  }
+};
+
+// z of one hidden layer: D tile mt of W^T b, plus bias
+__device__ __forceinline__ f32x4 dense(const bf16x8 (&A)[2], const bf16x8 (&b)[2]) {
+  f32x4 acc = {0, 0, 0, 0};
+  acc = mma(A[0], b[0], acc);
+  return mma(A[1], b[1], acc);
+}
+__device__ __forceinline__ f32x4 bias4(const float *b) { return *reinterpret_cast<const f32x4 *>(b); }
+
+// Output of one 16-sample tile from its B fragments: lane (q, c16) returns
+// y[4q + i] of sample c16.
+__device__ __forceinline__ f32x4 forward_tile(const Layers &W, const float *bias, bf16x8 (&b)[2], int q) {
+#pragma unroll
+  for (int L = 0; L < 3; L++) {
+    unsigned P[4][2];
+#pragma unroll
+    for (int mt = 0; mt < 4; mt++) {
+      const f32x4 acc = dense(W.h[L][mt], b), bb = bias4(bias + BOFF[L] + mt * 16 + 4 * q);
+      __bf16 v[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const float z = acc[i] + bb[i];
+        v[i] = (__bf16)(z > 0.0f ? z : 0.0f);
+      }
+      P[mt][0] = pack2(v[0], v[1]);
+      P[mt][1] = pack2(v[2], v[3]);
+    }
+    next_operand(P, b);
+  }
+  return dense(W.o, b) + bias4(bias + BOFF[3] + 4 * q);
+}
+__device__ __forceinline__ void store_tile(float *__restrict__ Y, const f32x4 &y, int row, int n, int q) {
+  if (row >= n) return;
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    if (4 * q + i < OUT) Y[(size_t)row * OUT + 4 * q + i] = y[i];
+}
+
+// ------------------------------------------------------------ forward --
+// Sources of input rows: raw(row) starts the loads of lane row q's features of a
+// sample, operand(raw) forms its B fragments.
+struct FromBf16 {  // BF16 rows [n][64]
+  const __bf16 *X;
+  struct Raw {
+    bf16x8 v[2];
+  };
+  __device__ __forceinline__ Raw raw(int row, int q) const {
+    return Raw{{load8(X + (size_t)row * KP + 8 * q), load8(X + (size_t)row * KP + 32 + 8 * q)}};
+  }
+  __device__ __forceinline__ void operand(const Raw &r, bf16x8 (&b)[2]) const {
+    b[0] = r.v[0];
+    b[1] = r.v[1];
+  }
+};
+struct FromFloat {  // FP32 rows [n][46], any alignment of a float
+  const float *X;
+  struct Raw {
+    float v[2][8];
+  };
+  __device__ __forceinline__ Raw raw(int row, int q) const {
+    Raw r;
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const int f = 32 * k + 8 * q + j;
+        r.v[k][j] = f < IN ? X[(size_t)row * IN + f] : 0.0f;
+      }
+    return r;
+  }
+  __device__ __forceinline__ void operand(const Raw &r, bf16x8 (&b)[2]) const {
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+#pragma unroll
+      for (int j = 0; j < 8; j++) b[k][j] = (__bf16)r.v[k][j];
+  }
+};
+
+// y [N][6] of 16-sample tiles, one wave each, the weights in registers.  With
+// the weights read from LDS per tile and the activations turned through LDS
+// between layers, 599040 BF16 rows took 58 us, now 41; 65536 FP32 rows 8.9 us
+// with a conversion pass before it.
+template <class Src>
+__global__ __launch_bounds__(256, 2) void k_mlp_fwd(Weights w, Src src, int n, float *__restrict__ Y) {
+  __shared__ __align__(16) float bias[BSIZE];
+  for (int i = threadIdx.x; i < BSIZE; i += 256) bias[i] = w.bias[i];
+  const int wv = threadIdx.x / 64, l = threadIdx.x % 64, c16 = l % 16, q = l / 16;
+  const int ntile = (n + 15) / 16, stride = gridDim.x * 4;
+  Layers W;
+  W.load(w, c16, q);
+  __syncthreads();
+  int tt = blockIdx.x * 4 + wv;
+  if (tt >= ntile) return;
+  auto next = src.raw(min(tt * 16 + c16, n - 1), q);
+  for (; tt < ntile; tt += stride) {
+    const auto cur = next;
+    next = src.raw(min((tt + stride) * 16 + c16, n - 1), q);  // rows past n read row n-1
+    bf16x8 b[2];
+    src.operand(cur, b);
+    store_tile(Y, forward_tile(W, bias, b, q), tt * 16 + c16, n, q);
+  }
+}
+
+// The same for the closure's normalised features, formed straight from the
+// velocity gradients G[9][n] (LesSource): feature 9 k + j of a sample is gradient
+// j of the row dy[k] = 0, -2, -1, 1, 2 away (clamped to 0..ny), the last one y+.
+// A wave takes 64 samples, one per lane, so that every load is contiguous and
+// the means and scales are wave-uniform, and turns them into fragments through
+// LDS.  (x - mean) / scale is rounded as the division rounds it: one product with
+// the rounded reciprocal and one exact-remainder correction.
+constexpr int FROW = 72;  // BF16 values per sample in LDS, padded
+__global__ __launch_bounds__(256, 2) void k_mlp_fwd_les(Weights w, LesSource s, const float *__restrict__ norm,
+                                                        const double *__restrict__ yplus, float *__restrict__ Y) {
+  __shared__ __align__(16) float bias[BSIZE];
+  __shared__ __align__(16) __bf16 rows[4][64 * FROW];
+  for (int i = threadIdx.x; i < BSIZE; i += 256) bias[i] = w.bias[i];
+  const int wv = threadIdx.x / 64, l = threadIdx.x % 64, c16 = l % 16, q = l / 16, n = s.n;
+  const int ngrp = (n + 63) / 64, stride = gridDim.x * 4;
+  Layers W;
+  W.load(w, c16, q);
+  __syncthreads();
+  int grp = blockIdx.x * 4 + wv;
+  if (grp >= ngrp) return;
+  __bf16 *mine = rows[wv] + l * FROW;
+  float f[IN];
+  auto fetch = [&](int g) {
+    const int sm = min(g * 64 + l, n - 1), iy = sm / s.plane, o = sm - iy * s.plane;
+    const int dy[5] = {0, -2, -1, 1, 2};
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+      const int at = min(max(iy + dy[k], 0), s.ny) * s.plane + o;
+#pragma unroll
+      for (int j = 0; j < 9; j++) f[9 * k + j] = s.G[(size_t)j * n + at];
+    }
+    f[IN - 1] = (float)yplus[iy];
+  };
+  for (; grp < ngrp; grp += stride) {
+    fetch(grp);
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+      bf16x8 v = zero8();
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const int k = 8 * c + j;
+        if (k < IN) {
+          const float d = norm[IN + k], x = f[k] - norm[k], rd = norm[NORM_RECIP + k], t = x * rd;
+          v[j] = (__bf16)fmaf(fmaf(-t, d, x), rd, t);
         }
-      if (l < nout) red[64 * nout + l] += bsum;
+      }
+      *reinterpret_cast<bf16x8 *>(mine + 8 * c) = v;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll 1
+    for (int t = 0; t < 4; t++) {
+      const __bf16 *r = rows[wv] + (16 * t + c16) * FROW + 8 * q;
+      bf16x8 b[2] = {load8(r), load8(r + 32)};
+      store_tile(Y, forward_tile(W, bias, b, q), grp * 64 + 16 * t + c16, n, q);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+}
+
+// ------------------------------------------------------------- gradient --
+// Loss and gradient of a minibatch.  The samples are cut into chunks of C * 128
+// and a chunk into four slots: slot w takes the 32-sample sets at w * 32 + 128 k.
+// A slot's weight gradients accumulate on the matrix cores set after set, a
+// chunk's are the sum of its slots in order, the minibatch's the sum of its
+// chunks in order: this fixes every rounding, so that training does not depend on
+// how the work is spread.  A block takes `per` slots of one chunk and passes over
+// two sets, 64 samples, at a time: each wave runs 16 samples forward and back in
+// registers, leaving inputs, activations and dz of every layer in LDS as
+// [unit][sample]; then wave L adds the sets' weight gradient of layer L.  With per
+// = 4 the block writes its chunk's sum, with per = 2 (few chunks: twice the blocks
+// at work) each slot's.  8192 samples take 14 us in this one launch, where separate
+// forward, three backward and four weight-gradient kernels through memory took 97.
+constexpr int SP = 72;  // samples per LDS row, padded: 16-byte rows, spread over the banks
+struct GradLds {
+  __bf16 in[4][64 * SP];   // inputs of the layers: X, act 1..3
+  __bf16 dz[3][64 * SP];   // dz of the hidden layers
+  __bf16 dy[OP * SP];
+  float bias[BSIZE];
+  float red[4];
+};
+__global__ __launch_bounds__(256) void k_mlp_grad(Weights w, const __bf16 *__restrict__ X, const float *__restrict__ Tg,
+                                                  int n, float inv_count, int chunk, int per,
+                                                  float *__restrict__ part, float *__restrict__ loss_part) {
+  extern __shared__ __align__(16) char smem[];
+  GradLds &S = *reinterpret_cast<GradLds *>(smem);
+  for (int i = threadIdx.x; i < BSIZE; i += 256) S.bias[i] = w.bias[i];
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), l = threadIdx.x % 64, c16 = l % 16, q = l / 16;
+  const int sc = wv * 16 + c16;  // the lane's sample in the group
+  __syncthreads();
+  const int nout = wv < 3 ? H : OP, NT = nout / 16;  // of the layer whose weight gradient this wave forms
+  const __bf16 *tz = wv < 3 ? S.dz[wv] : S.dy;
+  const int split = 4 / per, ch = blockIdx.x / split, w0 = (blockIdx.x % split) * per, C = chunk / 128;
+  const int begin = ch * chunk, end = min(n, begin + chunk);
+  f32x4 acc[4][4], g[4][4];  // of the current slot; of the chunk
+#pragma unroll
+  for (int mt = 0; mt < 4; mt++)
+#pragma unroll
+    for (int nt = 0; nt < 4; nt++) acc[mt][nt] = g[mt][nt] = f32x4{0, 0, 0, 0};
+  float bacc = 0.0f, bsum = 0.0f, lsum = 0.0f;
+  auto store = [&](const f32x4(&v)[4][4], float bias, int at) {
+    float *dst = part + (size_t)at * GSIZE + GOFF[wv];
+#pragma unroll
+    for (int nt = 0; nt < 4; nt++) {
+      if (nt >= NT) break;
+#pragma unroll
+      for (int mt = 0; mt < 4; mt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) dst[(mt * 16 + 4 * q + i) * nout + nt * 16 + c16] = v[mt][nt][i];
+    }
+    if (l < nout) dst[64 * nout + l] = bias;
+  };
+  for (int t0 = w0 * C; t0 < (w0 + per) * C; t0 += 2) {
+    const int ts = t0 + (wv >> 1);  // this wave's set: slot ts / C, its set ts % C
+    const int row = begin + (ts / C) * 32 + (ts % C) * 128 + (wv & 1) * 16 + c16;
+    const bool valid = row < end;
+    const size_t rc = (size_t)min(row, n - 1);
+    Layers W;
+    W.load(w, c16, q);
+    bf16x8 b[2];
+    b[0] = load8(X + rc * KP + 8 * q);
+    b[1] = load8(X + rc * KP + 32 + 8 * q);
+    float tg[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) tg[i] = 4 * q + i < OUT ? Tg[rc * OUT + 4 * q + i] : 0.0f;
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+      for (int j = 0; j < 8; j++) S.in[0][(ks * 32 + 8 * q + j) * SP + sc] = b[ks][j];
+    unsigned mask[3];
+#pragma unroll
+    for (int L = 0; L < 3; L++) {
+      unsigned P[4][2];
+      mask[L] = 0;
+#pragma unroll
+      for (int mt = 0; mt < 4; mt++) {
+        const f32x4 h = dense(W.h[L][mt], b), bb = bias4(S.bias + BOFF[L] + mt * 16 + 4 * q);
+        __bf16 v[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const float z = h[i] + bb[i];
+          v[i] = (__bf16)(z > 0.0f ? z : 0.0f);
+          mask[L] |= (float)v[i] > 0.0f ? 1u << (4 * mt + i) : 0u;
+          S.in[L + 1][(mt * 16 + 4 * q + i) * SP + sc] = v[i];
+        }
+        P[mt][0] = pack2(v[0], v[1]);
+        P[mt][1] = pack2(v[2], v[3]);
+      }
+      next_operand(P, b);
+    }
+    {
+      const f32x4 o = dense(W.o, b), bb = bias4(S.bias + BOFF[3] + 4 * q);
+      __bf16 dv[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        float d = o[i] + bb[i] - tg[i];
+        if (!valid || 4 * q + i >= OUT) d = 0.0f;
+        lsum += d * d;
+        dv[i] = (__bf16)(2.0f * d * inv_count);
+        S.dy[(4 * q + i) * SP + sc] = dv[i];
+      }
+      // dy as a B fragment: only the outputs 0..7, lane row 0, are not zero
+      const unsigned p0 = pack2(dv[0], dv[1]), p1 = pack2(dv[2], dv[3]);
+      unsigned r[4] = {p0, p1, (unsigned)__shfl((int)p0, c16 + 16, 64), (unsigned)__shfl((int)p1, c16 + 16, 64)};
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        if (q) r[k] = 0;
+      __builtin_memcpy(&b[0], r, sizeof r);
+    }
+    // back: dh = W dz_next, masked by the activation
+#pragma unroll
+    for (int L = 2; L >= 0; L--) {
+      unsigned P[4][2];
+#pragma unroll
+      for (int mt = 0; mt < 4; mt++) {
+        f32x4 h = {0, 0, 0, 0};
+        const __bf16 *A = w.wio + WOFF[L + 1] + (size_t)(mt * 16 + c16) * (L == 2 ? OP : H);
+        if (L == 2) {
+          h = mma(q < 2 ? load8(A + 8 * q) : zero8(), b[0], h);
+        } else {
+          h = mma(load8(A + 8 * q), b[0], h);
+          h = mma(load8(A + 32 + 8 * q), b[1], h);
+        }
+        __bf16 v[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          v[i] = (__bf16)((mask[L] >> (4 * mt + i)) & 1 ? h[i] : 0.0f);
+          S.dz[L][(mt * 16 + 4 * q + i) * SP + sc] = v[i];
+        }
+        P[mt][0] = pack2(v[0], v[1]);
+        P[mt][1] = pack2(v[2], v[3]);
+      }
+      if (L > 0) next_operand(P, b);
     }
     __syncthreads();
+    // dW[in][out] of layer wv, one 32-sample set after the other
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) {
+      bf16x8 A[4];
+#pragma unroll
+      for (int mt = 0; mt < 4; mt++) A[mt] = load8(&S.in[wv][(mt * 16 + c16) * SP + ks * 32 + 8 * q]);
+#pragma unroll
+      for (int nt = 0; nt < 4; nt++) {
+        if (nt >= NT) break;
+        const bf16x8 B = load8(tz + (nt * 16 + c16) * SP + ks * 32 + 8 * q);
+#pragma unroll
+        for (int mt = 0; mt < 4; mt++) acc[mt][nt] = mma(A[mt], B, acc[mt][nt]);
+      }
+      if (l < nout) {
+        float s = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const bf16x8 v = load8(tz + l * SP + ks * 32 + 8 * k);
+#pragma unroll
+          for (int j = 0; j < 8; j++) s += (float)v[j];
+        }
+        bacc += s;
+      }
+      if ((t0 + ks) % C == C - 1) {  // the slot is done
+        if (per == 2) {
+          store(acc, bacc, ch * 4 + (t0 + ks) / C);
+        } else {
+#pragma unroll
+          for (int mt = 0; mt < 4; mt++)
+#pragma unroll
+            for (int nt = 0; nt < 4; nt++) g[mt][nt] += acc[mt][nt];
+          bsum += bacc;
+        }
+#pragma unroll
+        for (int mt = 0; mt < 4; mt++)
+#pragma unroll
+          for (int nt = 0; nt < 4; nt++) acc[mt][nt] = f32x4{0, 0, 0, 0};
+        bacc = 0.0f;
+      }
+    }
+    __syncthreads();  // the next pass reuses the tiles
   }
-  float *dst = part + (size_t)blockIdx.x * (64 * nout + nout);
-  for (int i = threadIdx.x; i < 64 * nout + nout; i += 256) dst[i] = red[i];
+  if (per == 4) store(g, bsum, ch);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off, 64);
+  if (l == 0) S.red[wv] = lsum;
+  __syncthreads();
+  if (threadIdx.x == 0) loss_part[blockIdx.x] = (S.red[0] + S.red[1]) + (S.red[2] + S.red[3]);
 }
 
-// sum of nblk partial vectors of length len, in block order
-__global__ __launch_bounds__(256) void k_mlp_reduce(const float *__restrict__ part, int nblk, int len,
-                                                    float *__restrict__ out) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= len) return;
-  float s = 0.0f;
-  for (int b = 0; b < nblk; b++) s += part[(size_t)b * len + i];
-  out[i] = s;
-}
-
-// --------------------------------------------------------------- Adam --
-// master/m/v/g in the padded kernel layout (GSIZE floats); refreshes the
-// BF16 weight copies in both orientations and the FP32 biases.  Padding
-// entries have zero gradient and stay zero.
-__global__ __launch_bounds__(256) void k_mlp_adam(float *__restrict__ master, float *__restrict__ m1,
-                                                  float *__restrict__ m2, const float *__restrict__ g, Weights w,
-                                                  float lr, float b1, float b2, float eps, float c1, float c2) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
+// --------------------------------------------------------------- update --
+// Gradient g = sum of the chunks' gradients in order (SLOTS: each the sum of its
+// four slots in order), 64 loads in flight; ADAM then updates master/m/v
+// (padded kernel layout) and refreshes the BF16 weight copies in both orientations
+// and the FP32 biases.  Padding entries have zero gradient and stay zero.  The
+// last block sums the loss partials.
+struct AdamArgs {
+  float *master, *m1, *m2;
+  float lr, b1, b2, eps, c1, c2;
+};
+template <bool ADAM, bool SLOTS>
+__global__ __launch_bounds__(64) void k_mlp_update(const float *__restrict__ part, const float *__restrict__ loss_part,
+                                                   int nchunk, int nloss, float *__restrict__ g, float *__restrict__ loss,
+                                                   AdamArgs a, Weights w) {
+  if (blockIdx.x == gridDim.x - 1) {
+    float s = 0.0f;
+    for (int b = threadIdx.x; b < nloss; b += 64) s += loss_part[b];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if (threadIdx.x == 0) *loss = s;
+    return;
+  }
+  const int i = blockIdx.x * 64 + threadIdx.x;
   if (i >= GSIZE) return;
-  const float gi = g[i];
-  const float mi = b1 * m1[i] + (1.0f - b1) * gi;
-  const float vi = b2 * m2[i] + (1.0f - b2) * gi * gi;
-  m1[i] = mi;
-  m2[i] = vi;
-  const float p = master[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-  master[i] = p;
-  write_param(w, i, p);
+  constexpr int V = SLOTS ? 4 : 1, U = 64 / V;  // vectors per chunk, chunks per round
+  float gi = 0.0f;
+  auto chunk_sum = [&](const float *v) {
+    if constexpr (SLOTS) return ((v[0] + v[1]) + v[2]) + v[3];
+    else return v[0];
+  };
+  int c = 0;
+  for (; c + U <= nchunk; c += U) {
+    float v[64];
+#pragma unroll
+    for (int k = 0; k < 64; k++) v[k] = part[((size_t)c * V + k) * GSIZE + i];
+#pragma unroll
+    for (int k = 0; k < U; k++) gi += chunk_sum(v + k * V);
+  }
+  for (; c < nchunk; c++) {
+    float v[V];
+#pragma unroll
+    for (int k = 0; k < V; k++) v[k] = part[((size_t)c * V + k) * GSIZE + i];
+    gi += chunk_sum(v);
+  }
+  if constexpr (ADAM) {
+    const float mi = a.b1 * a.m1[i] + (1.0f - a.b1) * gi;
+    const float vi = a.b2 * a.m2[i] + (1.0f - a.b2) * gi * gi;
+    a.m1[i] = mi;
+    a.m2[i] = vi;
+    const float p = a.master[i] - a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
+    a.master[i] = p;
+    write_param(w, i, p);
+  } else {
+    g[i] = gi;
+  }
 }
 
 // copies the padded FP32 master to the BF16 / bias arrays (after set_params)
@@ -292,7 +504,7 @@ __global__ __launch_bounds__(256) void k_mlp_refresh(const float *__restrict__ m
 // ================================================================ C-ABI ==
 #include <chrono>
 #include <cstring>
-#include <mutex>
+#include <algorithm>
 #include <vector>
 
 #include "../../include/channel_closure.h"
@@ -306,52 +518,27 @@ static_assert(NPARAM == CHAN_MLP_NPARAM, "canonical parameter count");
 struct chan_mlp {
   int64_t cap = 0, n = 0;
   int dev = 0;                // device the model lives on
+  int ncu = 256;              // its compute units
   hipStream_t st = nullptr;
   __bf16 *X = nullptr;        // [cap][64]
   float *T = nullptr;         // [cap][6]
-  __bf16 *act = nullptr;      // [3][cap][64]
-  __bf16 *dz = nullptr;       // [3][cap][64]
-  __bf16 *dy = nullptr;       // [cap][16]
+  float *Xf = nullptr;        // [cap][46] host rows on their way in, made on first use
   float *Y = nullptr;         // [cap][6]
   float *master = nullptr, *m1 = nullptr, *m2 = nullptr, *g = nullptr;  // [GSIZE]
-  float *part = nullptr;      // wgrad partials
-  float *lpart = nullptr;     // loss partials
+  float *part = nullptr;      // gradient partials [gvec][GSIZE]
+  float *lpart = nullptr;     // loss partials [GBLK], then the loss of chan_mlp_grad
   float *losses = nullptr;    // per training step
   __bf16 *woi = nullptr, *wio = nullptr;
   float *bias = nullptr;
   int64_t adam_t = 0;
   int losses_cap = 0;
+  int gvec = 0;               // gradient partials
 };
-
-// Staging of chan_mlp_forward_noalloc: the BF16 inputs [CHAN_MLP_NOALLOC_MAX][64]
-// (8 MiB), one copy per GPU for the life of the process.  Host code never
-// passes this name to a kernel: it holds a host-side stand-in, and the device
-// address comes from hipGetSymbolAddress (noalloc_scratch below).
-static __device__ __align__(256) __bf16 scratch[(size_t)CHAN_MLP_NOALLOC_MAX * KP];
 
 namespace {
 
-constexpr int MAXDEV = 64;
-std::mutex g_scratch_mu;
-void *g_scratch[MAXDEV] = {};  // device address of `scratch` per device
-
-// Resolves the address of `scratch` on the current device, once per device
-// (called by chan_mlp_create with the model's device current).
-int noalloc_scratch(int dev, void **out) {
-  if (dev < 0 || dev >= MAXDEV) return set_error(CHAN_E_ARG, "device %d beyond the %d the library tracks", dev, MAXDEV);
-  std::lock_guard<std::mutex> lk(g_scratch_mu);
-  if (!g_scratch[dev]) {
-    void *ptr = nullptr;
-    hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
-    if (e != hipSuccess || !ptr) return set_error((int)(e != hipSuccess ? e : hipErrorInvalidSymbol), "hipGetSymbolAddress of the staging array failed: %s", hipGetErrorString(e));
-    g_scratch[dev] = ptr;
-  }
-  *out = g_scratch[dev];
-  return 0;
-}
-
-constexpr int MAXBLK = 1024;  // blocks of the per-sample kernels
-constexpr int WBLK = 256;     // blocks of the weight-gradient kernels
+// most chunks of a minibatch, and most partial vectors
+constexpr int GBLK = 256;
 
 #define MCHK(expr)                                                                                          \
   do {                                                                                                      \
@@ -376,43 +563,55 @@ __global__ void k_to_bf16(const float *__restrict__ x, __bf16 *__restrict__ xb, 
   xb[i] = (__bf16)(c < IN ? x[r * IN + c] : 0.0f);
 }
 
-int nblk_rows(int64_t n) { return (int)std::min<int64_t>(MAXBLK, std::max<int64_t>(1, ((n + 15) / 16 + 3) / 4)); }
+// Blocks of k_mlp_fwd: its waves keep the weights in registers, so each takes
+// several tiles (two waves per SIMD are resident).
+int fwd_blocks(const chan_mlp *m, int64_t n) {
+  return (int)std::min<int64_t>(2 * (int64_t)m->ncu, std::max<int64_t>(1, ((n + 15) / 16 + 3) / 4));
+}
 
-// gradient of the minibatch [first, first+count) into m->g; loss partials in m->lpart
-int grad_pass(chan_mlp *m, int64_t first, int count) {
-  const Weights w = weights(m);
-  const __bf16 *X = m->X + first * KP;
-  const float *T = m->T + first * OUT;
-  const int nb = nblk_rows(count);
-  hipLaunchKernelGGL((k_mlp_fwd<true>), dim3(nb), dim3(256), 0, m->st, w, X, T, count, 1.0f / (6.0f * count),
-                     (float *)nullptr, m->act, m->dy, m->lpart);
+template <class Src>
+hipError_t launch_fwd(chan_mlp *m, const Src &src, int64_t n, float *Y, hipStream_t st) {
+  hipLaunchKernelGGL((k_mlp_fwd<Src>), dim3(fwd_blocks(m, n)), dim3(256), 0, st, weights(m), src, (int)n, Y);
+  return hipGetLastError();
+}
+
+// Gradient of the minibatch [first, first+count): partials, then their sum into
+// m->g or, with `adam`, straight into the weights; the loss sum goes to *loss.
+// Chunks are whole multiples of 128 samples, at most GBLK of them; up to GBLK / 4
+// chunks are worked on slot by slot, by two blocks each.
+int grad_pass(chan_mlp *m, int64_t first, int count, const AdamArgs *adam, float *loss) {
+  const int wb = (int)std::min<int64_t>(GBLK, ((int64_t)count + 127) / 128);
+  const int chunk = (int)((((int64_t)count + wb - 1) / wb + 127) / 128 * 128);
+  const int nchunk = (count + chunk - 1) / chunk;
+  const bool slots = nchunk <= GBLK / 4;
+  const int nb = slots ? 2 * nchunk : nchunk;
+  hipLaunchKernelGGL(k_mlp_grad, dim3(nb), dim3(256), sizeof(GradLds), m->st, weights(m), m->X + first * KP,
+                     m->T + first * OUT, count, 1.0f / (6.0f * count), chunk, slots ? 2 : 4, m->part, m->lpart);
   MCHK(hipGetLastError());
-  for (int L = 2; L >= 0; L--) {
-    const __bf16 *dn = L == 2 ? m->dy : m->dz + (size_t)(L + 1) * m->cap * KP;
-    hipLaunchKernelGGL(k_mlp_bwd, dim3(nb), dim3(256), 0, m->st, w, L, count, m->act, dn,
-                       m->dz + (size_t)L * m->cap * KP);
-    MCHK(hipGetLastError());
-  }
-  // weight gradients: chunks of whole 128-sample groups
-  const int wb = (int)std::min<int64_t>(WBLK, (count + 127) / 128);
-  const int chunk = (int)(((count + wb - 1) / wb + 127) / 128 * 128);
-  for (int L = 0; L < 4; L++) {
-    const __bf16 *dzL = L == 3 ? m->dy : m->dz + (size_t)L * m->cap * KP;
-    hipLaunchKernelGGL(k_mlp_wgrad, dim3(wb), dim3(256), 0, m->st, L, count, X, m->act, dzL, m->part, chunk);
-    MCHK(hipGetLastError());
-    const int len = psize(L);
-    hipLaunchKernelGGL(k_mlp_reduce, dim3((len + 255) / 256), dim3(256), 0, m->st, m->part, wb, len, m->g + goff(L));
-    MCHK(hipGetLastError());
-  }
+  auto update = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((GSIZE + 63) / 64 + 1), dim3(64), 0, m->st, m->part, m->lpart, nchunk, nb, m->g, loss,
+                       adam ? *adam : AdamArgs{}, weights(m));
+    return hipGetLastError();
+  };
+  if (adam)
+    MCHK(slots ? update(k_mlp_update<true, true>) : update(k_mlp_update<true, false>));
+  else
+    MCHK(slots ? update(k_mlp_update<false, true>) : update(k_mlp_update<false, false>));
+  return 0;
+}
+
+int row_workspace(chan_mlp *m) {
+  int rc;
+  if (!m->Xf && (rc = mal(&m->Xf, (size_t)m->cap * IN))) return rc;
   return 0;
 }
 
 }  // namespace
 
-hipError_t chan::mlp::forward_device(chan_mlp *m, const __bf16 *X, int64_t n, float *Y, hipStream_t st) {
-  if (n < 1 || n > ((int64_t)1 << 31) / KP) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_mlp_fwd<false>), dim3(nblk_rows(n)), dim3(256), 0, st, weights(m), X, (const float *)nullptr,
-                     (int)n, 0.0f, Y, (__bf16 *)nullptr, (__bf16 *)nullptr, (float *)nullptr);
+hipError_t chan::mlp::forward_gradients(chan_mlp *m, const LesSource &s, float *Y, hipStream_t st) {
+  if (s.n < 1 || s.n > ((int64_t)1 << 31) / KP) return hipErrorInvalidValue;
+  const int nb = (int)std::min<int64_t>(2 * (int64_t)m->ncu, ((int64_t)s.n + 255) / 256);
+  hipLaunchKernelGGL(k_mlp_fwd_les, dim3(nb), dim3(256), 0, st, weights(m), s, s.norm, s.yplus, Y);
   return hipGetLastError();
 }
 
@@ -425,23 +624,23 @@ int chan_mlp_create(int64_t capacity, chan_mlp **out) {
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1) return set_error(CHAN_E_NODEV, "no HIP device");
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return set_error(CHAN_E_NODEV, "no current HIP device");
-  void *scr = nullptr;
-  int rc = noalloc_scratch(dev, &scr);  // once per device, at set-up
-  if (rc) return rc;
-  (void)scr;
+  int rc = 0;
   chan_mlp *m = new chan_mlp();
   m->cap = capacity;
   m->dev = dev;
+  if (hipDeviceGetAttribute(&m->ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || m->ncu < 1) m->ncu = 256;
+  // gradient vectors: four slots of each of GBLK / 4 chunks, or GBLK chunks
+  m->gvec = (int)std::min<int64_t>(GBLK, (capacity + 127) / 128 * 4);
   auto bail = [&](int code) {
     chan_mlp_destroy(m);
     return code;
   };
   if (hipStreamCreate(&m->st) != hipSuccess) return bail(set_error(CHAN_E_STATE, "hipStreamCreate failed"));
   const size_t c = (size_t)capacity;
-  if ((rc = mal(&m->X, c * KP)) || (rc = mal(&m->T, c * OUT)) || (rc = mal(&m->act, 3 * c * KP)) ||
-      (rc = mal(&m->dz, 3 * c * KP)) || (rc = mal(&m->dy, c * OP)) || (rc = mal(&m->Y, c * OUT)) ||
+  if ((rc = mal(&m->X, c * KP)) || (rc = mal(&m->T, c * OUT)) || (rc = mal(&m->Y, c * OUT)) ||
       (rc = mal(&m->master, GSIZE)) || (rc = mal(&m->m1, GSIZE)) || (rc = mal(&m->m2, GSIZE)) ||
-      (rc = mal(&m->g, GSIZE)) || (rc = mal(&m->part, (size_t)WBLK * psize(0))) || (rc = mal(&m->lpart, MAXBLK)) ||
+      (rc = mal(&m->g, GSIZE)) || (rc = mal(&m->part, (size_t)m->gvec * GSIZE)) ||
+      (rc = mal(&m->lpart, (size_t)GBLK + 1)) ||
       (rc = mal(&m->woi, WSIZE)) || (rc = mal(&m->wio, WSIZE)) || (rc = mal(&m->bias, BSIZE)))
     return bail(rc);
   if (hipMemset(m->master, 0, sizeof(float) * GSIZE) != hipSuccess ||
@@ -456,7 +655,7 @@ int chan_mlp_create(int64_t capacity, chan_mlp **out) {
 int chan_mlp_destroy(chan_mlp *m) {
   if (!m) return 0;
   if (m->st) hipStreamSynchronize(m->st);
-  void *bufs[] = {m->X, m->T, m->act, m->dz, m->dy, m->Y, m->master, m->m1, m->m2, m->g, m->part, m->lpart,
+  void *bufs[] = {m->X, m->T, m->Xf, m->Y, m->master, m->m1, m->m2, m->g, m->part, m->lpart,
                   m->losses, m->woi, m->wio, m->bias};
   for (void *b : bufs)
     if (b) hipFree(b);
@@ -487,19 +686,17 @@ int chan_mlp_get_params(chan_mlp *m, float *params) {
 
 int chan_mlp_set_data(chan_mlp *m, const float *X, const float *T, int64_t n) {
   if (!m || !X || !T || n < 1 || n > m->cap) return set_error(CHAN_E_ARG, "bad argument");
-  float *tmp = nullptr;
   int rc;
-  if ((rc = mal(&tmp, (size_t)n * IN))) return rc;
-  hipError_t e = hipMemcpyAsync(tmp, X, sizeof(float) * n * IN, hipMemcpyHostToDevice, m->st);
+  if ((rc = row_workspace(m))) return rc;
+  hipError_t e = hipMemcpyAsync(m->Xf, X, sizeof(float) * n * IN, hipMemcpyHostToDevice, m->st);
   if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_to_bf16, dim3((unsigned)((n * KP + 255) / 256)), dim3(256), 0, m->st, tmp, m->X, n);
+    hipLaunchKernelGGL(k_to_bf16, dim3((unsigned)((n * KP + 255) / 256)), dim3(256), 0, m->st, m->Xf, m->X, n);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipMemcpyAsync(m->T, T, sizeof(float) * n * OUT, hipMemcpyHostToDevice, m->st);
   if (e == hipSuccess) e = hipMemsetAsync(m->m1, 0, sizeof(float) * GSIZE, m->st);
   if (e == hipSuccess) e = hipMemsetAsync(m->m2, 0, sizeof(float) * GSIZE, m->st);
   if (e == hipSuccess) e = hipStreamSynchronize(m->st);
-  hipFree(tmp);
   if (e != hipSuccess) return set_error((int)e, "set_data: %s", hipGetErrorString(e));
   m->n = n;
   m->adam_t = 0;
@@ -508,25 +705,12 @@ int chan_mlp_set_data(chan_mlp *m, const float *X, const float *T, int64_t n) {
 
 int chan_mlp_forward(chan_mlp *m, const float *X, int64_t n, float *Y) {
   if (!m || !X || !Y || n < 1 || n > m->cap) return set_error(CHAN_E_ARG, "bad argument");
-  float *tmp = nullptr;
   int rc;
-  if ((rc = mal(&tmp, (size_t)n * IN))) return rc;
-  // the inputs go through the activation buffer, leaving the resident data alone
-  __bf16 *xb = m->act;
-  hipError_t e = hipMemcpyAsync(tmp, X, sizeof(float) * n * IN, hipMemcpyHostToDevice, m->st);
-  if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_to_bf16, dim3((unsigned)((n * KP + 255) / 256)), dim3(256), 0, m->st, tmp, xb, n);
-    e = hipGetLastError();
-  }
-  if (e == hipSuccess) {
-    hipLaunchKernelGGL((k_mlp_fwd<false>), dim3(nblk_rows(n)), dim3(256), 0, m->st, weights(m), xb,
-                       (const float *)nullptr, (int)n, 0.0f, m->Y, (__bf16 *)nullptr, (__bf16 *)nullptr,
-                       (float *)nullptr);
-    e = hipGetLastError();
-  }
+  if ((rc = row_workspace(m))) return rc;
+  hipError_t e = hipMemcpyAsync(m->Xf, X, sizeof(float) * n * IN, hipMemcpyHostToDevice, m->st);
+  if (e == hipSuccess) e = launch_fwd(m, FromFloat{m->Xf}, n, m->Y, m->st);
   if (e == hipSuccess) e = hipMemcpyAsync(Y, m->Y, sizeof(float) * n * OUT, hipMemcpyDeviceToHost, m->st);
   if (e == hipSuccess) e = hipStreamSynchronize(m->st);
-  hipFree(tmp);
   if (e != hipSuccess) return set_error((int)e, "forward: %s", hipGetErrorString(e));
   return 0;
 }
@@ -534,23 +718,13 @@ int chan_mlp_forward(chan_mlp *m, const float *X, int64_t n, float *Y) {
 int chan_mlp_forward_noalloc(chan_mlp *m, const float *dX, int64_t n, float *dY) {
   if (!m || !dX || !dY || n < 1) return set_error(CHAN_E_ARG, "bad argument");
   if (n > CHAN_MLP_NOALLOC_MAX)
-    return set_error(CHAN_E_ARG, "chan_mlp_forward_noalloc: %lld rows exceed its staging of %d rows; split the call",
+    return set_error(CHAN_E_ARG, "chan_mlp_forward_noalloc: %lld rows exceed its limit of %d rows; split the call",
                      (long long)n, CHAN_MLP_NOALLOC_MAX);
   int dev = -1;
   MCHK(hipGetDevice(&dev));
   if (dev != m->dev) return set_error(CHAN_E_STATE, "chan_mlp_forward_noalloc: device %d is current, the model lives on %d", dev, m->dev);
-  __bf16 *xb = nullptr;
-  {
-    std::lock_guard<std::mutex> lk(g_scratch_mu);
-    xb = static_cast<__bf16 *>(g_scratch[dev]);
-  }
-  if (!xb) return set_error(CHAN_E_STATE, "chan_mlp_forward_noalloc: no staging address for device %d", dev);
-  // the same two kernels and launch shapes as chan_mlp_forward
-  hipLaunchKernelGGL(k_to_bf16, dim3((unsigned)((n * KP + 255) / 256)), dim3(256), 0, m->st, dX, xb, n);
-  MCHK(hipGetLastError());
-  hipLaunchKernelGGL((k_mlp_fwd<false>), dim3(nblk_rows(n)), dim3(256), 0, m->st, weights(m), xb,
-                     (const float *)nullptr, (int)n, 0.0f, dY, (__bf16 *)nullptr, (__bf16 *)nullptr, (float *)nullptr);
-  MCHK(hipGetLastError());
+  // the same kernel and launch shape as chan_mlp_forward
+  MCHK(launch_fwd(m, FromFloat{dX}, n, dY, m->st));
   MCHK(hipStreamSynchronize(m->st));
   return 0;
 }
@@ -558,16 +732,14 @@ int chan_mlp_forward_noalloc(chan_mlp *m, const float *dX, int64_t n, float *dY)
 int chan_mlp_grad(chan_mlp *m, int64_t first, int64_t count, float *grad, double *loss) {
   if (!m || !grad || !loss || first < 0 || count < 1 || first + count > m->n) return set_error(CHAN_E_ARG, "bad argument");
   int rc;
-  if ((rc = grad_pass(m, first, (int)count))) return rc;
-  std::vector<float> pad(GSIZE), lp(MAXBLK);
-  const int nb = nblk_rows(count);
+  if ((rc = grad_pass(m, first, (int)count, nullptr, m->lpart + GBLK))) return rc;
+  std::vector<float> pad(GSIZE);
+  float lsum = 0.0f;
   MCHK(hipMemcpyAsync(pad.data(), m->g, sizeof(float) * GSIZE, hipMemcpyDeviceToHost, m->st));
-  MCHK(hipMemcpyAsync(lp.data(), m->lpart, sizeof(float) * nb, hipMemcpyDeviceToHost, m->st));
+  MCHK(hipMemcpyAsync(&lsum, m->lpart + GBLK, sizeof lsum, hipMemcpyDeviceToHost, m->st));
   MCHK(hipStreamSynchronize(m->st));
   for (int c = 0; c < NPARAM; c++) grad[c] = pad[canon_to_padded(c)];
-  double s = 0.0;
-  for (int b = 0; b < nb; b++) s += lp[b];
-  *loss = s / (6.0 * (double)count);
+  *loss = (double)lsum / (6.0 * (double)count);
   return 0;
 }
 
@@ -587,18 +759,13 @@ int chan_mlp_train(chan_mlp *m, int32_t steps, int32_t batch, float lr, float *l
   int64_t off = 0;
   for (int s = 0; s < steps; s++) {
     if (off + batch > m->n) off = 0;
-    int rc;
-    if ((rc = grad_pass(m, off, batch))) return rc;
-    const int nb = nblk_rows(batch);
-    hipLaunchKernelGGL(k_mlp_reduce, dim3(1), dim3(256), 0, m->st, m->lpart, nb, 1, m->losses + s);
-    MCHK(hipGetLastError());
     m->adam_t++;
     const float b1 = 0.9f, b2 = 0.999f;
     const float c1 = 1.0f - (float)std::pow((double)b1, (double)m->adam_t);
     const float c2 = 1.0f - (float)std::pow((double)b2, (double)m->adam_t);
-    hipLaunchKernelGGL(k_mlp_adam, dim3((GSIZE + 255) / 256), dim3(256), 0, m->st, m->master, m->m1, m->m2, m->g,
-                       weights(m), lr, b1, b2, 1e-8f, c1, c2);
-    MCHK(hipGetLastError());
+    const AdamArgs adam = {m->master, m->m1, m->m2, lr, b1, b2, 1e-8f, c1, c2};
+    int rc;
+    if ((rc = grad_pass(m, off, batch, &adam, m->losses + s))) return rc;
     off += batch;
   }
   MCHK(hipEventRecord(e1, m->st));
@@ -622,12 +789,9 @@ int chan_mlp_bench_forward(chan_mlp *m, int32_t reps, double *ms) {
   MCHK(hipEventCreate(&e0));
   MCHK(hipEventCreate(&e1));
   const int n = (int)m->n;
-  hipLaunchKernelGGL((k_mlp_fwd<false>), dim3(nblk_rows(n)), dim3(256), 0, m->st, weights(m), m->X,
-                     (const float *)nullptr, n, 0.0f, m->Y, (__bf16 *)nullptr, (__bf16 *)nullptr, (float *)nullptr);
+  MCHK(launch_fwd(m, FromBf16{m->X}, n, m->Y, m->st));
   MCHK(hipEventRecord(e0, m->st));
-  for (int r = 0; r < reps; r++)
-    hipLaunchKernelGGL((k_mlp_fwd<false>), dim3(nblk_rows(n)), dim3(256), 0, m->st, weights(m), m->X,
-                       (const float *)nullptr, n, 0.0f, m->Y, (__bf16 *)nullptr, (__bf16 *)nullptr, (float *)nullptr);
+  for (int r = 0; r < reps; r++) MCHK(launch_fwd(m, FromBf16{m->X}, n, m->Y, m->st));
   MCHK(hipEventRecord(e1, m->st));
   MCHK(hipEventSynchronize(e1));
   float t = 0;

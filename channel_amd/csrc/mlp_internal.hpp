@@ -23,6 +23,7 @@ constexpr int WSIZE = woff(4);
 constexpr int boff(int L) { return L == 0 ? 0 : boff(L - 1) + nout_of(L - 1); }
 constexpr int BSIZE = boff(4);
 __device__ constexpr int WOFF[5] = {woff(0), woff(1), woff(2), woff(3), woff(4)};
+__device__ constexpr int GOFF[5] = {goff(0), goff(1), goff(2), goff(3), goff(4)};
 __device__ constexpr int BOFF[5] = {boff(0), boff(1), boff(2), boff(3), boff(4)};
 
 struct Weights {
@@ -65,8 +66,17 @@ inline int canon_to_padded(int c) {
 struct chan_mlp;
 namespace chan {
 namespace mlp {
-// inference of model m on n resident BF16 rows X[n][64] -> Y[n][6] FP32,
-// enqueued on stream st (k_mlp.hip)
-hipError_t forward_device(chan_mlp *m, const __bf16 *X, int64_t n, float *Y, hipStream_t st);
+// The velocity gradients of a closure grid: G[9][n] on rows 0..ny of `plane`
+// points each (n = (ny + 1) plane), y+ per row, and the normalisation
+// [46 mean][46 scale][12 of the stresses][46 reciprocal scales].
+constexpr int NORM_RECIP = 2 * IN + 2 * OUT;
+struct LesSource {
+  const float *G, *norm;
+  const double *yplus;
+  int n, plane, ny;
+};
+// inference of model m on the features of s -> Y[n][6] FP32, enqueued on stream
+// st (k_mlp.hip)
+hipError_t forward_gradients(chan_mlp *m, const LesSource &s, float *Y, hipStream_t st);
 }  // namespace mlp
 }  // namespace chan
