@@ -341,12 +341,20 @@ int chan_create(const chan_params *p, chan_ctx **out) {
   const size_t esz = c->split ? sizeof(cx<float>) : sizeof(cx<double>);
   if ((rc = dalloc_bytes(&c->old, 2 * (size_t)(g.ny - 1) * plane * esz))) return bail(rc);
   // B doubles as the staging area of the field and rhs transposes, which
-  // needs 3*Ny*npair complex FP64 <= 6*Ny*slab*esz
+  // needs 3*Ny*npair complex FP64 <= NPROD*Ny*slab*esz (nzd >= 3 nz), P as the
+  // device layout of a force, 3*Ny*ps complex FP64
   if ((rc = dalloc_bytes(&c->A, 3 * (size_t)g.Ny * slab * esz))) return bail(rc);
-  if ((rc = dalloc_bytes(&c->B, 6 * (size_t)g.Ny * slab * esz))) return bail(rc);
-  if ((rc = dalloc_bytes(&c->P, 6 * NyP * esz))) return bail(rc);
+  if ((rc = dalloc_bytes(&c->B, NPROD * (size_t)g.Ny * slab * esz))) return bail(rc);
+  if ((rc = dalloc_bytes(&c->P, NyP * (NPROD * esz > 48 ? NPROD * esz : 48)))) return bail(rc);
   if ((rc = dalloc_bytes(&c->twz, (size_t)fft::tw_table_size(g.nzd) * esz))) return bail(rc);
   if ((rc = dalloc_bytes(&c->twx, (size_t)fft::tw_table_size(2 * g.nxd) * esz))) return bail(rc);
+  // no mode that is kept may alias: more than 3 nz points in z; 3 (nx + 1) in x,
+  // which the x pass's slots need
+  c->nzs = alias_free_size(3 * g.nz + 1, g.nzd);
+  c->mxs = alias_free_size(3 * g.Nx, 2 * g.nxd);
+  if ((rc = dalloc_bytes(&c->twzs, (size_t)fft::tw_table_size(c->nzs) * esz)) ||
+      (rc = dalloc_bytes(&c->twxs, (size_t)fft::tw_table_size(c->mxs) * esz)))
+    return bail(rc);
   if ((rc = dalloc(&c->der, (size_t)(g.ny - 1) * 20))) return bail(rc);
   if ((rc = dalloc(&c->derT, (size_t)g.Ny * 20)) || (rc = dalloc(&c->derF, (size_t)g.Ny * 10)) ||
       (rc = dalloc(&c->tab, (size_t)(g.ny - 1) * SROW))) return bail(rc);
@@ -362,6 +370,10 @@ int chan_create(const chan_params *p, chan_ctx **out) {
     if (hipMemcpy(c->twz, tw.data(), tw.size() * sizeof(tw[0]), hipMemcpyHostToDevice) != hipSuccess) return 1;
     twiddles_x(tw, 2 * g.nxd);
     if (hipMemcpy(c->twx, tw.data(), tw.size() * sizeof(tw[0]), hipMemcpyHostToDevice) != hipSuccess) return 1;
+    twiddles(tw, c->nzs);
+    if (hipMemcpy(c->twzs, tw.data(), tw.size() * sizeof(tw[0]), hipMemcpyHostToDevice) != hipSuccess) return 1;
+    twiddles_x(tw, c->mxs);
+    if (hipMemcpy(c->twxs, tw.data(), tw.size() * sizeof(tw[0]), hipMemcpyHostToDevice) != hipSuccess) return 1;
     return 0;
   };
   if (c->split ? upload_tw(cx<float>{}) : upload_tw(cx<double>{})) return bail(fail(CHAN_E_STATE, "upload failed"));
@@ -419,7 +431,7 @@ int chan_destroy(chan_ctx *c) {
     hipEventDestroy(r.b);
   }
   for (auto e : c->pool) hipEventDestroy(e);
-  void *bufs[] = {c->V, c->old, c->rhs, c->L, c->col00, c->A, c->B, c->P, c->twz, c->twx,
+  void *bufs[] = {c->V, c->old, c->rhs, c->L, c->col00, c->A, c->B, c->P, c->twz, c->twx, c->twzs, c->twxs,
                   c->der, c->derT, c->derF, c->tab, c->d0fac, c->y, c->dy, c->sc, c->stat, c->F0, c->gain, c->Fkeep};
   for (void *b : bufs)
     if (b) hipFree(b);
@@ -645,24 +657,30 @@ extern "C++" {
 // in the split mode)
 template <typename R>
 static int products_t(chan_ctx *c, int plane0, int nplanes, bool prods, int cfl) {
-  const Geom &g = c->g;
+  // the physical grid where a CFL maximum is taken over it, else the alias-free one
+  const bool small = prods && !cfl;
+  Geom g = c->g;
   const HostSetup &h = c->hs;
+  const int M = small ? c->mxs : 2 * g.nxd;
+  if (small) g.nzd = c->nzs;
   // the transform kernels index A and B from the launch's first plane: the
   // base pointers are offset so that every plane keeps its own slices
   const size_t slab = (size_t)g.nzd * g.Nx;
   cx<R> *A = static_cast<cx<R> *>(c->A) + (size_t)plane0 * 3 * slab;
-  cx<R> *B = static_cast<cx<R> *>(c->B) + (size_t)plane0 * 6 * slab;
+  cx<R> *B = static_cast<cx<R> *>(c->B) + (size_t)plane0 * NPROD * slab;
   cx<R> *P = static_cast<cx<R> *>(c->P);
-  const cx<R> *twz = static_cast<const cx<R> *>(c->twz), *twx = static_cast<const cx<R> *>(c->twx);
+  const cx<R> *twz = static_cast<const cx<R> *>(small ? c->twzs : c->twz);
+  const cx<R> *twx = static_cast<const cx<R> *>(small ? c->twxs : c->twx);
+  const R factor = small ? (R)(1.0 / ((double)M * g.nzd)) : (R)h.factor;
   int rc;
-  if ((rc = timed(c, "zinv", [&] { return launch_zinv<R>(g.nzd, c->st, c->V, A, twz, g, plane0, nplanes); }))) return rc;
-  if ((rc = timed(c, prods ? "xpass" : "xpass_cfl", [&] {
-         return launch_xpass<R>(2 * g.nxd, c->st, A, B, twx, g, plane0, nplanes, prods, cfl, c->dy, h.dx, h.dz,
-                                (R)h.factor, &c->sc->cfl_bits);
+  if ((rc = timed(c, small ? "zinv" : "zinv_cfl", [&] { return launch_zinv<R>(g.nzd, c->st, c->V, A, twz, g, plane0, nplanes); }))) return rc;
+  if ((rc = timed(c, small ? "xpass" : (prods ? "xpass_cfl" : "cfl"), [&] {
+         return launch_xpass<R>(M, c->st, A, B, twx, g, plane0, nplanes, prods, cfl, c->dy, h.dx, h.dz, factor,
+                                &c->sc->cfl_bits);
        })))
     return rc;
   if (prods)
-    if ((rc = timed(c, "zfwd", [&] { return launch_zfwd<R>(g.nzd, c->st, B, P, twz, g, plane0, nplanes); }))) return rc;
+    if ((rc = timed(c, small ? "zfwd" : "zfwd_cfl", [&] { return launch_zfwd<R>(g.nzd, c->st, B, P, twz, g, plane0, nplanes); }))) return rc;
   return 0;
 }
 

@@ -16,6 +16,9 @@ namespace chan {
 // contiguous bytes per x-mode.
 constexpr int ZB = 4;
 
+// Product fields: uu - ww, vv - ww, uv, vw, uw (k_fft.hip).
+constexpr int NPROD = 5;
+
 // Geometry passed by value to kernels.
 struct Geom {
   int nx, ny, nz;   // dns.in sizes
@@ -49,7 +52,7 @@ __device__ __forceinline__ double div_by(double x, double d, double r) {
 // ---------------------------------------------------------- kernel args --
 template <typename R>
 struct RhsArgs {
-  const cx<R> *P;        // [6][Ny][ps] products
+  const cx<R> *P;        // [NPROD][Ny][ps] products
   const cx<double> *V;   // [3][Ny][ps]
   cx<R> *old;            // [2][ny-1][ps] previous explicit terms (eta, d2v); in the split
                          // mode FP32, as the products they are formed from
@@ -121,6 +124,7 @@ int set_error(int code, const char *fmt, ...);
 
 // ----------------------------------------------------------- launchers --
 int fft_size_supported(int N);
+int alias_free_size(int need, int below);
 template <typename R>
 hipError_t launch_zinv(int NZ, hipStream_t st, const cx<double> *V, cx<R> *A, const cx<R> *tw, const Geom &g, int plane0,
                        int nplanes);

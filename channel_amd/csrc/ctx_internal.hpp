@@ -26,6 +26,10 @@ struct chan_ctx {
   // the split mode
   bool split = false;
   void *A = nullptr, *B = nullptr, *P = nullptr, *twz = nullptr, *twx = nullptr;
+  // the alias-free grid of substeps without a CFL maximum: sizes and twiddles
+  // (the physical grid's own where there is no smaller size)
+  int nzs = 0, mxs = 0;
+  void *twzs = nullptr, *twxs = nullptr;
   double *der = nullptr, *derT = nullptr, *derF = nullptr, *tab = nullptr, *d0fac = nullptr, *y = nullptr, *dy = nullptr;
   double *stat = nullptr;  // statistics: [3][ny+1] mean in, [7][ny+1] profiles out
   // body force: static field [3][Ny][ps] and feedback gains [3][Ny][Nz+1]

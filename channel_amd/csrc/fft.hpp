@@ -5,8 +5,8 @@
 // Slot convention: a team of T threads transforms N = E*T points; thread t
 // holds "slot" s (0 <= s < E) = element t + T*s both on input and on output,
 // so loads from and stores to global memory by consecutive threads are
-// contiguous.  Sizes N = 3*2^k use E = 12, N = 2^k use E = 16; every radix
-// divides E, so each pass maps whole butterflies onto each thread.
+// contiguous.  Sizes N = 3*2^k and 9*2^k use E = 12, N = 2^k use E = 16; every
+// radix divides E, so each pass maps whole butterflies onto each thread.
 //
 // Conventions match FFTW's (ffts.f90:70-75): sign -1 forward
 // X_k = sum_j x_j e^{-2 pi i jk/N}, sign +1 backward, both unnormalised.
@@ -53,9 +53,16 @@ namespace fft {
 // most one radix-2 pass and a final radix-3 pass (fewer live registers, one
 // more LDS exchange).  The plan is a set of constexpr functions so that the
 // host builds the twiddle tables from the same definition.
+//
+// N = 9*2^k: radix 12, then a second radix 12 (or 3 for 36 and 72), then radix 4
+// and 2; both plans are the same.
 constexpr bool plan_pow2(int N) { return (N & (N - 1)) == 0; }
+constexpr bool plan_nine(int N) { return N % 9 == 0; }
+constexpr int nine_second(int N) { return N / 12 % 12 == 0 ? 12 : 3; }
 constexpr int plan_E(int N) { return plan_pow2(N) ? 16 : 12; }
-constexpr int plan_rest(int N, bool big) { return big ? N / plan_E(N) : (plan_pow2(N) ? N : N / 3); }
+constexpr int plan_rest(int N, bool big) {
+  return plan_nine(N) ? N / 12 / nine_second(N) : big ? N / plan_E(N) : (plan_pow2(N) ? N : N / 3);
+}
 constexpr int plan_n4(int N, bool big) {
   int r = plan_rest(N, big), n = 0;
   while (r % 4 == 0) {
@@ -70,9 +77,11 @@ constexpr bool plan_has2(int N, bool big) {
   return r == 2;
 }
 constexpr int plan_npass(int N, bool big) {
+  if (plan_nine(N)) return 2 + plan_n4(N, big) + (plan_has2(N, big) ? 1 : 0);
   return (big ? 1 : (plan_pow2(N) ? 0 : 1)) + plan_n4(N, big) + (plan_has2(N, big) ? 1 : 0);
 }
 constexpr int plan_radix(int N, bool big, int p) {
+  if (plan_nine(N)) return p == 0 ? 12 : (p == 1 ? nine_second(N) : (p < 2 + plan_n4(N, big) ? 4 : 2));
   if (big) return p == 0 ? plan_E(N) : (p <= plan_n4(N, big) ? 4 : 2);
   return p < plan_n4(N, big) ? 4 : ((p == plan_n4(N, big) && plan_has2(N, big)) ? 2 : 3);
 }
@@ -126,10 +135,11 @@ inline void build_twiddles(cx<T> *w, int N) {
 }
 
 // team-level LDS synchronisation: a team within one wavefront only needs the
-// wave's LDS operations ordered; larger teams use the workgroup barrier.
+// wave's LDS operations ordered; teams of several wavefronts, and those that
+// straddle them (T = 3*2^k), use the workgroup barrier.
 template <int T>
 __device__ __forceinline__ void team_sync() {
-  if constexpr (T <= 64) {
+  if constexpr (64 % T == 0) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -290,16 +300,33 @@ __device__ __forceinline__ void run_pass(cx<R> (&v)[Plan<N>::E], R *lds, const c
 #pragma unroll
   for (int m = 0; m < NB; m++) {
     if constexpr (NS > 1) {
-      // one table load per butterfly; higher powers by multiplication
+      // one table load per butterfly; higher powers by multiplication (for
+      // radix 12 from those of 1, 2, 3, 4 and 8, at most four products deep)
       const int j = t + m * T;
       const int k = j % NS;
       cx<R> w1 = tw[PL::tw_base(P) + k];
       if constexpr (S > 0) w1.y = -w1.y;
-      cx<R> wr = w1;
+      if constexpr (RAD == 12) {
+        cx<R> *x = &v[m * RAD];
+        const cx<R> w2 = mul(w1, w1), w3 = mul(w2, w1), w4 = mul(w2, w2), w8 = mul(w4, w4);
+        x[1] = mul(x[1], w1);
+        x[2] = mul(x[2], w2);
+        x[3] = mul(x[3], w3);
+        x[4] = mul(x[4], w4);
+        x[5] = mul(x[5], mul(w4, w1));
+        x[6] = mul(x[6], mul(w4, w2));
+        x[7] = mul(x[7], mul(w4, w3));
+        x[8] = mul(x[8], w8);
+        x[9] = mul(x[9], mul(w8, w1));
+        x[10] = mul(x[10], mul(w8, w2));
+        x[11] = mul(x[11], mul(w8, w3));
+      } else {
+        cx<R> wr = w1;
 #pragma unroll
-      for (int r = 1; r < RAD; r++) {
-        v[m * RAD + r] = mul(v[m * RAD + r], wr);
-        if (r + 1 < RAD) wr = mul(wr, w1);
+        for (int r = 1; r < RAD; r++) {
+          v[m * RAD + r] = mul(v[m * RAD + r], wr);
+          if (r + 1 < RAD) wr = mul(wr, w1);
+        }
       }
     }
     dft<RAD, S>(&v[m * RAD]);

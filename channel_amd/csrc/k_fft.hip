@@ -4,10 +4,22 @@
 //   K1 k_zinv : V(iy,iz,ix,c) -> zero-pad z to nzd, backward c2c FFT in z
 //               (IFT, ffts.f90:93-96)  -> A[plane][c][zb][ix][ZB]
 //   K2 k_xpass: per physical-z row: Hermitian c2r in x (RFT, zero modes
-//               nx+1..nxd), CFL maximum, the six products, r2c in x keeping
+//               nx+1..nxd), CFL maximum, the products, r2c in x keeping
 //               modes 0..nx (HFT), times `factor`       -> B[plane][q][zb][ix][ZB]
 //   K3 k_zfwd : forward c2c FFT in z, keep modes -nz..nz (FFT + izd)
 //                                                       -> P[q][plane][pair]
+//
+// Products.  Five fields stand for the reference's six: uu - ww, vv - ww, uv, vw,
+// uw.  The v-eta right-hand sides do not change when one field is added to uu, vv
+// and ww alike (the divergence of an isotropic stress is a gradient; the compact
+// stencils keep this exactly, k_rhs.hip), so ww is taken out of all three: one
+// sixth less to write, transform in z and read.
+//
+// Grids.  The physical grid is the reference's (fftFIT, sizes 2^k and 3*2^k) where
+// the CFL maximum is taken over its points.  The kept modes of the products are
+// the same sums on every grid of more than 3 nz points in z and 3 nx in x, so
+// where no CFL is asked for, the smallest supported size that large is used:
+// 9*2^k where it is smaller than fftFIT's (576 for 768, 288 for 384, 144 for 192).
 //
 // The reference's pencil transposes (zTOx / xTOz, mpi_transpose.f90:50-117)
 // are the layout changes between K1/K2 and K2/K3: both sides move ZB*16
@@ -41,19 +53,29 @@ constexpr int stage_stride() {
 // hold an FP64 block to three waves per SIMD and an FP32 block to six (four
 // and eight with the two rounds: the FP64 step 1.5% and the FP32 z kernels
 // 4-9% faster)
+// x modes per block of the z kernels, and its threads: 256, or 192 where the team
+// size is 3*2^k (N = 9*2^k)
+template <int NZ>
+constexpr int zteams() {
+  return (fft::plan_nine(NZ) ? 192 : 256) / fft::Plan<NZ>::T;
+}
+template <int NZ>
+constexpr int zthreads() {
+  return zteams<NZ>() * fft::Plan<NZ>::T;
+}
 template <int NZ, typename R>
 constexpr int zbuf_reals() {
-  constexpr int G = 256 / fft::Plan<NZ>::T;
+  constexpr int G = zteams<NZ>();
   constexpr int fftr = G * fft::lds_reals<NZ, ZXCH>();
   constexpr int stg = z_staged<NZ, R>() ? G * stage_stride<NZ>() : 0;
   return fftr > stg ? fftr : stg;
 }
 
 template <int NZ, typename R>
-__global__ __launch_bounds__(256) void k_zinv(const cx<double> *__restrict__ V, cx<R> *__restrict__ A,
+__global__ __launch_bounds__(zthreads<NZ>()) void k_zinv(const cx<double> *__restrict__ V, cx<R> *__restrict__ A,
                                               const cx<R> *__restrict__ tw, Geom g, int plane0) {
   using PL = fft::Plan<NZ>;
-  constexpr int T = PL::T, E = PL::E, G = 256 / T, SP = stage_stride<NZ>();
+  constexpr int T = PL::T, E = PL::E, G = zteams<NZ>(), NT = zthreads<NZ>(), SP = stage_stride<NZ>();
   __shared__ __align__(16) R lds[zbuf_reals<NZ, R>()];
   const int team = threadIdx.x / T, t = threadIdx.x % T;
   const int nxg = (g.Nx + G - 1) / G;
@@ -86,14 +108,14 @@ __global__ __launch_bounds__(256) void k_zinv(const cx<double> *__restrict__ V, 
       __syncthreads();
 #pragma unroll
       for (int i = 0; i < E; i++) {
-        const int el = (int)threadIdx.x + 256 * i;  // G*NZ = 256*E elements per block
+        const int el = (int)threadIdx.x + NT * i;  // G*NZ = NT*E elements per block
         const int zb = el / (G * ZB), w = el % (G * ZB), tm = w / ZB, r = w % ZB;
         out[h][i] = lds[min(tm, nact - 1) * SP + zb * ZB + r];
       }
     }
 #pragma unroll
     for (int i = 0; i < E; i++) {
-      const int el = (int)threadIdx.x + 256 * i;
+      const int el = (int)threadIdx.x + NT * i;
       const int zb = el / (G * ZB), w = el % (G * ZB), tm = w / ZB;
       if (tm < nact) dst[((size_t)zb * g.Nx + ix0) * ZB + w] = cx<R>{out[0][i], out[1][i]};
     }
@@ -141,6 +163,17 @@ __device__ __forceinline__ void block_max_atomic(double m, double *red, unsigned
   // integers (NaN above +Inf above every finite value)
   if (threadIdx.x == 0) atomicMax(out, (unsigned long long)__double_as_longlong(r));
 }
+
+// Product pairs: fields 0 uu-ww, 1 vv-ww, 2 uv, 3 vw, 4 uw as the real and
+// imaginary parts of three complex sequences.
+template <typename R>
+__device__ __forceinline__ cx<R> product_pair(const int pp, R u, R v, R w) {
+  if (pp == 0) return cx<R>{u * u - w * w, u * v};
+  if (pp == 1) return cx<R>{u * w, v * v - w * w};
+  return cx<R>{v * w, R(0)};
+}
+__device__ constexpr int pair_first(int pp) { return pp == 0 ? 0 : (pp == 1 ? 4 : 3); }
+__device__ constexpr int pair_second(int pp) { return pp == 0 ? 2 : 1; }
 
 // x modes per thread of the x pass: nxd >= 3(nx+1)/2 bounds Nx by M/3
 template <int E>
@@ -395,34 +428,24 @@ __global__ __launch_bounds__((xteams<M, R>() * fft::Plan<M>::T), 2) void k_xpass
   }
 
   if constexpr (PRODUCTS) {
-    // pairs (uu,uv), (uw,vv), (vw,ww) share one forward transform each; in
-    // this order u is dead once the second pair is formed, and v and w once
-    // the third is.  Product indices: 0 uu, 1 vv, 2 ww, 3 uv, 4 vw, 5 uw.
+    // pairs (uu-ww, uv) and (uw, vv-ww) share one forward transform each, vw has
+    // its own; in this order u is dead once the second pair is formed, and v and
+    // w once vw is
     auto form = [&](const int pp, cx<R>(&e)[E]) {
 #pragma unroll
-      for (int s = 0; s < E; s++) {
-        R a, b;
-        if (pp == 0) {
-          a = u[s] * u[s];
-          b = u[s] * v[s];
-        } else if (pp == 1) {
-          a = u[s] * w[s];
-          b = v[s] * v[s];
-        } else {
-          a = v[s] * w[s];
-          b = w[s] * w[s];
-        }
-        e[s] = cx<R>{a, b};
-      }
+      for (int s = 0; s < E; s++) e[s] = product_pair(pp, u[s], v[s], w[s]);
     };
     // A_k = (Z_k + conj Z_{M-k})/2, B_k = (Z_k - conj Z_{M-k})/(2i), k=0..nx,
     // with the transform's normalisation factor applied here, once per mode
     auto emit = [&](const int pp, const cx<R>(&e)[E]) {
-      const int qa = pp == 0 ? 0 : (pp == 1 ? 5 : 4), qb = pp == 0 ? 3 : (pp == 1 ? 1 : 2);
-      cx<R> *da = B + ((size_t)(pl * 6 + qa) * NZB + zb) * Nx * ZB + zi;
-      cx<R> *db = B + ((size_t)(pl * 6 + qb) * NZB + zb) * Nx * ZB + zi;
+      cx<R> *da = B + ((size_t)(pl * NPROD + pair_first(pp)) * NZB + zb) * Nx * ZB + zi;
+      cx<R> *db = B + ((size_t)(pl * NPROD + pair_second(pp)) * NZB + zb) * Nx * ZB + zi;
       const R hf = R(0.5) * factor;
       auto put = [&](int k, cx<R> z, cx<R> q) {
+        if (pp == 2) {  // a real sequence alone
+          da[(size_t)k * ZB] = cx<R>{z.x * factor, z.y * factor};
+          return;
+        }
         da[(size_t)k * ZB] = cx<R>{(z.x + q.x) * hf, (z.y - q.y) * hf};
         db[(size_t)k * ZB] = cx<R>{(z.y + q.y) * hf, (q.x - z.x) * hf};
       };
@@ -441,7 +464,7 @@ __global__ __launch_bounds__((xteams<M, R>() * fft::Plan<M>::T), 2) void k_xpass
         fft::team_sync<T>();  // the rows are the next transform's exchange area
       } else {
         cx<R> mz[MO];
-        mirror_pairs<T, E, MO, R>(e, mz, t, nx + 1);
+        if (pp < 2) mirror_pairs<T, E, MO, R>(e, mz, t, nx + 1);
 #pragma unroll
         for (int s = 0; s < MO; s++) {
           const int k = t + T * s;
@@ -476,29 +499,140 @@ __global__ __launch_bounds__((xteams<M, R>() * fft::Plan<M>::T), 2) void k_xpass
   }
 }
 
+// ------------------------------------------------------------ K2, 9*2^k --
+// The x pass of the 9*2^k grids (no CFL): a block of 192 threads holds RW rows in
+// teams of T = M/12 lanes, which straddle the wavefronts, so that the block
+// synchronises as a whole; four rows are a z block.  As it does so anyway, it
+// moves its global data through the teams' exchange areas: thread (mode, row) of
+// a whole run reads and writes contiguous memory, the Hermitian extension and the
+// mode split read their partners from LDS.
+//
+// Bound by the latency of its exchanges and barriers: three waves per SIMD in FP64
+// (33 spilled registers) take 2.04 ms at 191x384x189 (576 x 576 points, 5.5 GB),
+// two without spills 2.38; k_xpass on the 768 x 768 grid 2.49.  FP32 1.10 ms.  At
+// 95x128x95 (288 x 288 for 384 x 384) FP64 175 for 256 us, FP32 87 for 145.
+template <int M>
+constexpr int xrows() {
+  return 192 / fft::Plan<M>::T < ZB ? ZB : 192 / fft::Plan<M>::T;
+}
+template <int M, typename R>
+__global__ __launch_bounds__((xrows<M>() * fft::Plan<M>::T), (sizeof(R) == 8 ? 3 : 4)) void k_xpass_blk(
+    const cx<R> *__restrict__ A, cx<R> *__restrict__ B, const cx<R> *__restrict__ tw, Geom g, R factor, int nplanes) {
+  using PL = fft::Plan<M>;
+  constexpr int T = PL::T, E = PL::E, RW = xrows<M>(), NT = RW * T, MO = xmodes<E>(), MM = T * MO;  // MM modes at most
+  constexpr int ROW = fft::xch_len<M, fft::XCH_PAD>();  // complex values of a row's area; 3 MM <= M
+  constexpr int NTW = fft::plan_tw_size(M, true), ZPB = RW / ZB;  // twiddles, z blocks per block
+  __shared__ __align__(16) cx<R> lds[RW * ROW];
+  __shared__ __align__(16) cx<R> twl[NTW > 0 ? NTW : 1];
+  const int Nx = g.Nx, nx = g.nx, NZB = g.nzd / ZB, ntile = NZB * nplanes;
+  const int tid = threadIdx.x, t = tid % T, team = tid / T;
+  cx<R> *mine = lds + team * ROW;
+  R *fr = reinterpret_cast<R *>(mine);
+  for (int i = tid; i < NTW; i += NT) twl[i] = tw[i];
+  // modes 0..nx of u, v, w of every row: [row][c][MM]
+  for (int zz = 0; zz < ZPB; zz++) {
+    const int z = min((int)blockIdx.x * ZPB + zz, ntile - 1), pl = z / NZB, zb = z % NZB;
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      const cx<R> *src = A + ((size_t)(pl * 3 + c) * NZB + zb) * Nx * ZB;
+      cx<R> *dst = lds + zz * ZB * ROW + c * MM;
+#pragma unroll
+      for (int j = 0; j < (ZB * MM + NT - 1) / NT; j++) {
+        const int i = tid + NT * j;
+        if (i < ZB * Nx) dst[(i % ZB) * ROW + i / ZB] = src[i];
+      }
+    }
+  }
+  __syncthreads();
+  R u[E], v[E], w[E];
+  {
+    cx<R> e[E], f[E];
+#pragma unroll
+    for (int s = 0; s < E; s++) {
+      e[s] = f[s] = cx<R>{0, 0};
+      if (s >= MO && s < E - MO) continue;
+      const int k = t + T * s, m = s < MO ? k : M - k;
+      if (m > nx) continue;
+      cx<R> a = mine[m], b = mine[MM + m], c = mine[2 * MM + m];
+      if (s >= MO) {
+        a.y = -a.y;
+        b.y = -b.y;
+        c.y = -c.y;
+      }
+      if (k == 0) a.y = b.y = c.y = 0;  // as c2r does
+      e[s] = cx<R>{a.x - b.y, a.y + b.x};  // U + iV
+      f[s] = c;
+    }
+    __syncthreads();
+    fft::fft_slots<M, +1, true, fft::XCH_CPLX | fft::XCH_PAD>(e, fr, twl, t);
+    fft::fft_slots<M, +1, true, fft::XCH_CPLX | fft::XCH_PAD>(f, fr, twl, t);
+#pragma unroll
+    for (int s = 0; s < E; s++) {
+      u[s] = e[s].x;
+      v[s] = e[s].y;
+      w[s] = f[s].x;
+    }
+  }
+#pragma unroll
+  for (int pp = 0; pp < 3; pp++) {
+    cx<R> e[E];
+#pragma unroll
+    for (int s = 0; s < E; s++) e[s] = product_pair(pp, u[s], v[s], w[s]);
+    fft::fft_slots<M, -1, true, fft::XCH_CPLX | fft::XCH_PAD>(e, fr, twl, t);
+    // the modes to LDS in natural order, then A_k = (Z_k + conj Z_{M-k})/2,
+    // B_k = (Z_k - conj Z_{M-k})/(2i), k = 0..nx, times `factor`
+#pragma unroll
+    for (int s = 0; s < E; s++)
+      if (s < MO || (pp < 2 && s >= E - MO)) mine[t + T * s] = e[s];
+    __syncthreads();
+    const R hf = R(0.5) * factor;
+    for (int zz = 0; zz < ZPB; zz++) {
+      const int z = (int)blockIdx.x * ZPB + zz, pl = z / NZB, zb = z % NZB;
+      if (z >= ntile) break;
+      cx<R> *da = B + ((size_t)(pl * NPROD + pair_first(pp)) * NZB + zb) * Nx * ZB;
+      cx<R> *db = B + ((size_t)(pl * NPROD + pair_second(pp)) * NZB + zb) * Nx * ZB;
+#pragma unroll
+      for (int j = 0; j < (ZB * MM + NT - 1) / NT; j++) {
+        const int i = tid + NT * j, k = i / ZB;
+        if (i >= ZB * Nx) continue;
+        const cx<R> *row = lds + (zz * ZB + i % ZB) * ROW;
+        const cx<R> z0 = row[k];
+        if (pp == 2) {
+          da[i] = cx<R>{z0.x * factor, z0.y * factor};
+        } else {
+          const cx<R> q = row[k ? M - k : 0];
+          da[i] = cx<R>{(z0.x + q.x) * hf, (z0.y - q.y) * hf};
+          db[i] = cx<R>{(z0.y + q.y) * hf, (q.x - z0.x) * hf};
+        }
+      }
+    }
+    __syncthreads();
+  }
+}
+
 // ------------------------------------------------------------------- K3 --
 template <int NZ, typename R>
-__global__ __launch_bounds__(256) void k_zfwd(const cx<R> *__restrict__ B, cx<R> *__restrict__ P,
+__global__ __launch_bounds__(zthreads<NZ>()) void k_zfwd(const cx<R> *__restrict__ B, cx<R> *__restrict__ P,
                                               const cx<R> *__restrict__ tw, Geom g, int plane0) {
   using PL = fft::Plan<NZ>;
-  constexpr int T = PL::T, E = PL::E, G = 256 / T, SP = stage_stride<NZ>();
+  constexpr int T = PL::T, E = PL::E, G = zteams<NZ>(), NT = zthreads<NZ>(), SP = stage_stride<NZ>();
   __shared__ __align__(16) R lds[zbuf_reals<NZ, R>()];
   const int team = threadIdx.x / T, t = threadIdx.x % T;
   const int nxg = (g.Nx + G - 1) / G;
   int b = blockIdx.x;
   const int xg = b % nxg;
   b /= nxg;
-  const int q = b % 6, pl = b / 6;
+  const int q = b % NPROD, pl = b / NPROD;
   const int ix = xg * G + team;
   const bool act = ix < g.Nx;
-  const cx<R> *src = B + (size_t)(pl * 6 + q) * NZ * g.Nx;
+  const cx<R> *src = B + (size_t)(pl * NPROD + q) * NZ * g.Nx;
   cx<R> e[E];
   if constexpr (z_staged<NZ, R>()) {
     const int ix0 = xg * G, nact = min(G, g.Nx - ix0);
     cx<R> v[E];
 #pragma unroll
     for (int i = 0; i < E; i++) {  // all loads in flight together, clamped into the block's runs
-      const int el = (int)threadIdx.x + 256 * i;
+      const int el = (int)threadIdx.x + NT * i;
       const int zb = el / (G * ZB), w = el % (G * ZB);
       v[i] = src[((size_t)zb * g.Nx + ix0) * ZB + min(w, nact * ZB - 1)];
     }
@@ -506,7 +640,7 @@ __global__ __launch_bounds__(256) void k_zfwd(const cx<R> *__restrict__ B, cx<R>
     for (int h = 0; h < 2; h++) {
 #pragma unroll
       for (int i = 0; i < E; i++) {
-        const int el = (int)threadIdx.x + 256 * i;
+        const int el = (int)threadIdx.x + NT * i;
         const int zb = el / (G * ZB), w = el % (G * ZB), tm = w / ZB, r = w % ZB;
         lds[tm * SP + zb * ZB + r] = tm < nact ? (h ? v[i].y : v[i].x) : R(0);
       }
@@ -664,6 +798,7 @@ hipError_t launch_fft_bench(int N, int sign, int variant, const cx<double> *in, 
 }
 
 // ------------------------------------------------------------ launchers --
+#define CHAN_FOR_NINES(X) X(36) X(72) X(144) X(288) X(576) X(1152)
 #define CHAN_FOR_SIZES(X) X(12) X(24) X(48) X(96) X(192) X(384) X(768) X(1536) X(16) X(32) X(64) X(128) X(256) X(512) X(1024)
 
 template <typename R>
@@ -672,12 +807,13 @@ hipError_t launch_zinv(int NZ, hipStream_t st, const cx<double> *V, cx<R> *A, co
   switch (NZ) {
 #define X(N)                                                                              \
   case N: {                                                                               \
-    constexpr int G = 256 / fft::Plan<N>::T;                                              \
+    constexpr int G = zteams<N>();                                                        \
     dim3 grid((unsigned)(((g.Nx + G - 1) / G) * 3 * nplanes));                            \
-    hipLaunchKernelGGL((k_zinv<N, R>), grid, dim3(256), 0, st, V, A, tw, g, plane0);      \
+    hipLaunchKernelGGL((k_zinv<N, R>), grid, dim3(zthreads<N>()), 0, st, V, A, tw, g, plane0); \
     return hipGetLastError();                                                             \
   }
     CHAN_FOR_SIZES(X)
+    CHAN_FOR_NINES(X)
 #undef X
   }
   return hipErrorInvalidValue;
@@ -709,6 +845,16 @@ hipError_t launch_xpass(int M, hipStream_t st, const cx<R> *A, cx<R> *B, const c
   }
     CHAN_FOR_SIZES(X)
 #undef X
+#define X(N)                                                                                                          \
+  case N: {                                                                                                           \
+    if (!products || cfl_on) break;                                                                                   \
+    constexpr int RW = xrows<N>();                                                                                    \
+    hipLaunchKernelGGL((k_xpass_blk<N, R>), dim3((ntile + RW / ZB - 1) / (RW / ZB)), dim3(RW * fft::Plan<N>::T), 0, \
+                       st, A, B, tw, g, factor, nplanes);                                                             \
+    return hipGetLastError();                                                                                         \
+  }
+    CHAN_FOR_NINES(X)
+#undef X
   }
   return hipErrorInvalidValue;
 }
@@ -719,12 +865,13 @@ hipError_t launch_zfwd(int NZ, hipStream_t st, const cx<R> *B, cx<R> *P, const c
   switch (NZ) {
 #define X(N)                                                                         \
   case N: {                                                                          \
-    constexpr int G = 256 / fft::Plan<N>::T;                                         \
-    dim3 grid((unsigned)(((g.Nx + G - 1) / G) * 6 * nplanes));                       \
-    hipLaunchKernelGGL((k_zfwd<N, R>), grid, dim3(256), 0, st, B, P, tw, g, plane0); \
+    constexpr int G = zteams<N>();                                                   \
+    dim3 grid((unsigned)(((g.Nx + G - 1) / G) * NPROD * nplanes));                   \
+    hipLaunchKernelGGL((k_zfwd<N, R>), grid, dim3(zthreads<N>()), 0, st, B, P, tw, g, plane0); \
     return hipGetLastError();                                                        \
   }
     CHAN_FOR_SIZES(X)
+    CHAN_FOR_NINES(X)
 #undef X
   }
   return hipErrorInvalidValue;
@@ -746,6 +893,15 @@ hipError_t launch_fft_test(int N, int sign, hipStream_t st, cx<double> *data, co
 #undef X
   }
   return hipErrorInvalidValue;
+}
+
+// the smallest size of the form 9*2^k in [need, below), or `below` when none is
+int alias_free_size(int need, int below) {
+#define X(N) \
+  if (N >= need && N < below) return N;
+  CHAN_FOR_NINES(X)
+#undef X
+  return below;
 }
 
 int fft_size_supported(int N) {

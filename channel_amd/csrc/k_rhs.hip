@@ -2,10 +2,12 @@
 // interior row and wavenumber pair (buildrhs, dnsdata.f90:611-673).
 //
 // With kx = al, kz = be, k2 = kx^2 + kz^2, the explicit terms of the D2v and
-// eta equations (:637-661) are stencils of four combinations of the six
-// products, formed once per row and pair:
+// eta equations (:637-661) are stencils of four combinations of the products,
+// formed once per row and pair:
 //   G1 = k2 vv - kx^2 uu - 2 kx kz uw - kz^2 ww,  G2 = i kx uv + i kz vw
 //   G3 = kx kz (uu - ww) + (kz^2 - kx^2) uw,      G4 = i kx vw - i kz uv
+// which hold uu, vv and ww only as a = uu - ww and b = vv - ww: G1 = k2 b - kx^2 a
+// - 2 kx kz uw, G3 = kx kz a + (kz^2 - kx^2) uw.
 //   D2v: D1(G1) + D2(G2) + k2 D0(G2),             eta: D0(G3) + D1(G4)
 // (the (0,0) mode's eta slot carries the mean flow: G4 = -(Re uv + i Re vw)).
 // The implicit operators OS/SQ (:476-477) and the time derivative are one
@@ -14,8 +16,8 @@
 // One thread per (pair, chunk of rows) walks y and adds each row, as it is
 // read, to the sums of the five output rows whose stencils reach it: four
 // complex sums per pending row (explicit and implicit part of each equation),
-// 80 FP64 registers' worth, where a five-row window of the nine fields that
-// are read would be 90 complex values.  It then finishes the oldest row with
+// 80 FP64 registers' worth, where a five-row window of the eight fields that
+// are read would be 40 complex values.  It then finishes the oldest row with
 // the CN-RK3 time scheme (:486), writes the new rhs and replaces the stored
 // explicit term.  The stencil coefficients come transposed (row r's weights
 // in the five rows r-2..r+2), wave-uniform through the scalar cache.
@@ -105,14 +107,14 @@ __global__ __launch_bounds__(RHS_BLOCK) void k_rhs(RhsArgs<R> a, ForceArgs fa, c
   const size_t rs = (size_t)(g.ny - 1) * ps;  // component stride of old/rhs
 
   // the row being read; all loads are unconditional, with the row clamped
-  cx<R> np[6];
+  cx<R> np[NPROD];
   cx<double> nv[3], nold[2] = {{0.0, 0.0}, {0.0, 0.0}};
   cx<double> nf[3];  // static force
   double ng[3];      // feedback gains
   auto load = [&](int r) {  // row r (its plane is r + 1)
     const size_t off = (size_t)(r + 1) * ps + p;
 #pragma unroll
-    for (int q = 0; q < 6; q++) np[q] = a.P[q * pstride + off];
+    for (int q = 0; q < NPROD; q++) np[q] = a.P[q * pstride + off];
 #pragma unroll
     for (int c = 0; c < 3; c++) nv[c] = a.V[c * pstride + off];
     if constexpr (FORCE) {
@@ -137,7 +139,7 @@ __global__ __launch_bounds__(RHS_BLOCK) void k_rhs(RhsArgs<R> a, ForceArgs fa, c
   load(y0 - 2);
   for (int r = y0 - 2; r <= y1 + 2; r++) {
     const auto D = [](cx<R> v) { return cx<double>{(double)v.x, (double)v.y}; };
-    const cx<double> uu = D(np[0]), vv = D(np[1]), ww = D(np[2]), uv = D(np[3]), vw = D(np[4]), uw = D(np[5]);
+    const cx<double> pa = D(np[0]), pb = D(np[1]), uv = D(np[2]), vw = D(np[3]), uw = D(np[4]);
     const cx<double> u = nv[0], v = nv[1], w = nv[2], old_e = nold[0], old_v = nold[1];
     cx<double> F[3];
     if constexpr (FORCE) {
@@ -155,11 +157,11 @@ __global__ __launch_bounds__(RHS_BLOCK) void k_rhs(RhsArgs<R> a, ForceArgs fa, c
     }
     load(min(r + 1, g.ny + 1));
     cx<double> G1, G2, G3, G4, eta;
-    G1.x = k2 * vv.x - al2 * uu.x - be2 * ww.x - 2.0 * albe * uw.x;
-    G1.y = k2 * vv.y - al2 * uu.y - be2 * ww.y - 2.0 * albe * uw.y;
+    G1.x = k2 * pb.x - al2 * pa.x - 2.0 * albe * uw.x;
+    G1.y = k2 * pb.y - al2 * pa.y - 2.0 * albe * uw.y;
     G2 = cx<double>{-(al * uv.y + be * vw.y), al * uv.x + be * vw.x};
-    G3.x = albe * (uu.x - ww.x) + (be2 - al2) * uw.x;
-    G3.y = albe * (uu.y - ww.y) + (be2 - al2) * uw.y;
+    G3.x = albe * pa.x + (be2 - al2) * uw.x;
+    G3.y = albe * pa.y + (be2 - al2) * uw.y;
     G4 = cx<double>{be * uv.y - al * vw.y, al * vw.x - be * uv.x};
     eta = cx<double>{al * w.y - be * u.y, be * u.x - al * w.x};
     if (mean) {
