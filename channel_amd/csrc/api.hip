@@ -90,19 +90,25 @@ __global__ __launch_bounds__(TT * 8) void k_to_host(const cx<double> *__restrict
   }
 }
 
-// outstats staging: the (0,0) columns of all three components as out[c][row],
-// then a copy of the device scalars; the running CFL maximum restarts at 0.
-__global__ void k_gather00(const cx<double> *__restrict__ V, cx<double> *__restrict__ out, DevScalars *sc, Geom g) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r == 0) {
-    DevScalars *stash = reinterpret_cast<DevScalars *>(out + 3 * g.Ny);
-    *stash = *sc;
+// What outstats reads on the host: five rows of u's and w's (0,0) columns at each
+// wall and the device scalars.  Pinned memory that the kernel writes itself, so
+// that a step ends with one launch and a wait: a copy engine's transfer to
+// pageable memory took 20 us more, of 250 for a step of a 15x32x15 field.
+struct StepRow {
+  double lo[2][5], hi[2][5];
+  DevScalars sc;
+};
+// The running CFL maximum restarts at 0.
+__global__ void k_step_row(const cx<double> *__restrict__ V, StepRow *__restrict__ out, DevScalars *sc, Geom g) {
+  const int t = threadIdx.x;
+  if (t == 0) {
+    out->sc = *sc;
     sc->cfl_bits = 0ull;
   }
-  if (r >= g.Ny) return;
-  for (int c = 0; c < 3; c++) out[c * g.Ny + r] = V[((size_t)c * g.Ny + r) * g.ps + g.nz];
+  if (t >= 20) return;
+  const int comp = t / 5 % 2, j = t % 5, r = t < 10 ? j : g.Ny - 5 + j;
+  (t < 10 ? out->lo : out->hi)[comp][j] = V[((size_t)2 * comp * g.Ny + r) * g.ps + g.nz].x;
 }
-constexpr size_t STASH = (sizeof(DevScalars) + sizeof(cx<double>) - 1) / sizeof(cx<double>);
 
 // grid-stride streaming copy of n 32-byte elements
 __global__ __launch_bounds__(256) void k_copy(const double4 *__restrict__ a, double4 *__restrict__ b, size_t n) {
@@ -337,7 +343,8 @@ int chan_create(const chan_params *p, chan_ctx **out) {
   if ((rc = dalloc(&c->V, 3 * NyP))) return bail(rc);
   if ((rc = dalloc(&c->rhs, 2 * (size_t)(g.ny - 1) * plane))) return bail(rc);
   if ((rc = dalloc(&c->L, 2 * (size_t)(g.ny - 1) * plane))) return bail(rc);
-  if ((rc = dalloc(&c->col00, 3 * (size_t)g.Ny + STASH))) return bail(rc);
+  if (hipHostMalloc(&c->step_row, sizeof(StepRow), hipHostMallocDefault) != hipSuccess)
+    return bail(fail(CHAN_E_STATE, "hipHostMalloc failed"));
   const size_t esz = c->split ? sizeof(cx<float>) : sizeof(cx<double>);
   if ((rc = dalloc_bytes(&c->old, 2 * (size_t)(g.ny - 1) * plane * esz))) return bail(rc);
   // B doubles as the staging area of the field and rhs transposes, which
@@ -426,12 +433,14 @@ int chan_destroy(chan_ctx *c) {
   if (!c) return 0;
   if (c->st) hipStreamSynchronize(c->st);
   if (c->les) les_free(c->les);
+  c->stage.free();
+  if (c->step_row) hipHostFree(c->step_row);
   for (auto &r : c->pend) {
     hipEventDestroy(r.a);
     hipEventDestroy(r.b);
   }
   for (auto e : c->pool) hipEventDestroy(e);
-  void *bufs[] = {c->V, c->old, c->rhs, c->L, c->col00, c->A, c->B, c->P, c->twz, c->twx, c->twzs, c->twxs,
+  void *bufs[] = {c->V, c->old, c->rhs, c->L, c->A, c->B, c->P, c->twz, c->twx, c->twzs, c->twxs,
                   c->der, c->derT, c->derF, c->tab, c->d0fac, c->y, c->dy, c->sc, c->stat, c->F0, c->gain, c->Fkeep};
   for (void *b : bufs)
     if (b) hipFree(b);
@@ -485,7 +494,7 @@ int chan_set_field(chan_ctx *c, const double *V) {
   if (!c || !V) return fail(CHAN_E_ARG, "null argument");
   const size_t n = (size_t)3 * c->g.npair * c->g.Ny;
   cx<double> *stage = static_cast<cx<double> *>(c->B);
-  HIPCHK(hipMemcpyAsync(stage, V, n * sizeof(cx<double>), hipMemcpyHostToDevice, c->st));
+  HIPCHK(copy_to_device(c->stage, stage, V, n * sizeof(cx<double>), c->st));
   HIPCHK(launch_to_device_layout(c->st, stage, c->V, c->g));
   HIPCHK(hipStreamSynchronize(c->st));
   c->field_set = true;
@@ -497,8 +506,7 @@ int chan_get_field(chan_ctx *c, double *V) {
   const size_t n = (size_t)3 * c->g.npair * c->g.Ny;
   cx<double> *stage = static_cast<cx<double> *>(c->B);
   HIPCHK(launch_to_host_layout(c->st, c->V, stage, c->g));
-  HIPCHK(hipMemcpyAsync(V, stage, n * sizeof(cx<double>), hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipStreamSynchronize(c->st));
+  HIPCHK(copy_to_host(c->stage, V, stage, n * sizeof(cx<double>), c->st));
   return 0;
 }
 
@@ -514,7 +522,7 @@ int chan_set_body_force(chan_ctx *c, const double *F) {
   if (!c->F0 && (rc = dalloc(&c->F0, 3 * (size_t)c->g.Ny * c->g.ps))) return rc;
   const size_t n = (size_t)3 * c->g.npair * c->g.Ny;
   cx<double> *stage = static_cast<cx<double> *>(c->B);
-  HIPCHK(hipMemcpyAsync(stage, F, n * sizeof(cx<double>), hipMemcpyHostToDevice, c->st));
+  HIPCHK(copy_to_device(c->stage, stage, F, n * sizeof(cx<double>), c->st));
   HIPCHK(launch_to_device_layout(c->st, stage, c->F0, c->g));
   HIPCHK(hipStreamSynchronize(c->st));
   return 0;
@@ -559,8 +567,7 @@ int chan_get_body_force(chan_ctx *c, double *F) {
   a.out = dev;
   HIPCHK(launch_force(c->st, a));
   HIPCHK(launch_to_host_layout(c->st, dev, stage, c->g));
-  HIPCHK(hipMemcpyAsync(F, stage, n * sizeof(cx<double>), hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipStreamSynchronize(c->st));
+  HIPCHK(copy_to_host(c->stage, F, stage, n * sizeof(cx<double>), c->st));
   return 0;
 }
 
@@ -589,8 +596,7 @@ int chan_get_applied_body_force(chan_ctx *c, double *F) {
   }
   cx<double> *stage = static_cast<cx<double> *>(c->B);
   HIPCHK(launch_to_host_layout(c->st, c->Fkeep, stage, c->g));
-  HIPCHK(hipMemcpyAsync(F, stage, n * sizeof(cx<double>), hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipStreamSynchronize(c->st));
+  HIPCHK(copy_to_host(c->stage, F, stage, n * sizeof(cx<double>), c->st));
   return 0;
 }
 
@@ -609,8 +615,7 @@ int chan_get_rhs(chan_ctx *c, double *R) {
                        stage + (size_t)k * g1.npair * g1.Ny, g1);
     HIPCHK(hipGetLastError());
   }
-  HIPCHK(hipMemcpyAsync(R, stage, sizeof(cx<double>) * 2 * (size_t)g.npair * g.Ny, hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipStreamSynchronize(c->st));
+  HIPCHK(copy_to_host(c->stage, R, stage, sizeof(cx<double>) * 2 * (size_t)g.npair * g.Ny, c->st));
   return 0;
 }
 
@@ -828,31 +833,28 @@ int chan_stats(chan_ctx *c, const double *avg, double *out) {
 int chan_outstats(chan_ctx *c, double row[11]) {
   if (!c || !row) return fail(CHAN_E_ARG, "null argument");
   const Geom &g = c->g;
-  std::vector<cx<double>> col(3 * (size_t)g.Ny + STASH);
-  DevScalars d;
-  // one kernel stages the columns and scalars and resets the running CFL
-  // maximum (cfl=0 in outstats); one copy brings them back
-  hipLaunchKernelGGL(k_gather00, dim3((g.Ny + 127) / 128), dim3(128), 0, c->st, c->V, c->col00, c->sc, g);
+  // one kernel writes the rows and scalars and resets the running CFL maximum
+  // (cfl=0 in outstats)
+  StepRow *const row0 = static_cast<StepRow *>(c->step_row);
+  hipLaunchKernelGGL(k_step_row, dim3(1), dim3(64), 0, c->st, c->V, row0, c->sc, g);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(col.data(), c->col00, col.size() * sizeof(col[0]), hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));
-  std::memcpy(&d, col.data() + 3 * (size_t)g.Ny, sizeof d);
+  const StepRow s = *row0;
+  const DevScalars &d = s.sc;
   const double rg = cfl_value(d);
   if (!std::isfinite(rg)) return fail(CHAN_E_NOTFINITE, "CFL maximum is not finite (%g): the field holds NaN or Inf", rg);
   if (c->prm.cflmax > 0) c->deltat = c->prm.cflmax / rg;
   const double *b140 = c->hs.bnd[B_D140], *b14n = c->hs.bnd[B_D14N];
-  const int ny = g.ny;
-  auto re = [&](int comp, int iy) { return col[(size_t)comp * g.Ny + iy + 1].x; };
   double d11 = 0, d21 = 0, d12 = 0, d22 = 0;
   for (int j = 0; j < 5; j++) {
-    d12 += b14n[j] * re(0, ny - 3 + j);
-    d22 += b14n[j] * re(2, ny - 3 + j);
+    d12 += b14n[j] * s.hi[0][j];
+    d22 += b14n[j] * s.hi[1][j];
   }
   d12 = -d12;
   d22 = -d22;
   for (int j = 0; j < 5; j++) {
-    d11 += b140[j] * re(0, -1 + j);
-    d21 += b140[j] * re(2, -1 + j);
+    d11 += b140[j] * s.lo[0][j];
+    d21 += b140[j] * s.lo[1][j];
   }
   row[0] = c->time;
   row[1] = d11;

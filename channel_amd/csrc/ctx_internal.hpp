@@ -6,6 +6,7 @@
 
 #include "../../include/channel_hip.h"
 #include "chan_internal.hpp"
+#include "host_copy.hpp"
 
 namespace chan {
 struct LesState;
@@ -19,7 +20,8 @@ struct chan_ctx {
   chan::Geom g;
   hipStream_t st = nullptr;
   // device state
-  chan::cx<double> *V = nullptr, *rhs = nullptr, *col00 = nullptr;
+  chan::cx<double> *V = nullptr, *rhs = nullptr;
+  void *step_row = nullptr;  // pinned: what a step's end reads on the host
   void *old = nullptr;  // explicit terms: complex FP64, or FP32 in the split mode
   double2 *L = nullptr;
   // transform intermediates and twiddles: complex FP64, or complex FP32 in
@@ -41,6 +43,7 @@ struct chan_ctx {
   chan::cx<double> *Fkeep = nullptr;
   int kept_state = 0;
   chan::DevScalars *sc = nullptr;
+  chan::HostStage stage;  // of fields on their way to and from the host
   // host scalars
   double time = 0, deltat = 0;
   bool field_set = false;

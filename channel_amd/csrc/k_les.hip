@@ -466,8 +466,7 @@ int chan_les_features(chan_ctx *c, float *X) {
   if ((rc = les_gradients(c, s))) return rc;
   hipLaunchKernelGGL(k_les_features, dim3((s->n + 255) / 256), dim3(256), 0, c->st, s->Gp, les_geom(c), s->yplus, s->Xf);
   LCHK(hipGetLastError());
-  LCHK(hipMemcpyAsync(X, s->Xf, sizeof(float) * 46 * (size_t)s->n, hipMemcpyDeviceToHost, c->st));
-  LCHK(hipStreamSynchronize(c->st));
+  LCHK(copy_to_host(c->stage, X, s->Xf, sizeof(float) * 46 * (size_t)s->n, c->st));
   return 0;
 }
 

@@ -509,6 +509,7 @@ __global__ __launch_bounds__(256) void k_mlp_refresh(const float *__restrict__ m
 
 #include "../../include/channel_closure.h"
 #include "../../include/channel_hip.h"
+#include "host_copy.hpp"
 
 using namespace chan;
 using namespace chan::mlp;
@@ -533,6 +534,7 @@ struct chan_mlp {
   int64_t adam_t = 0;
   int losses_cap = 0;
   int gvec = 0;               // gradient partials
+  HostStage stage;            // of rows on their way to and from the host
 };
 
 namespace {
@@ -655,6 +657,7 @@ int chan_mlp_create(int64_t capacity, chan_mlp **out) {
 int chan_mlp_destroy(chan_mlp *m) {
   if (!m) return 0;
   if (m->st) hipStreamSynchronize(m->st);
+  m->stage.free();
   void *bufs[] = {m->X, m->T, m->Xf, m->Y, m->master, m->m1, m->m2, m->g, m->part, m->lpart,
                   m->losses, m->woi, m->wio, m->bias};
   for (void *b : bufs)
@@ -688,12 +691,12 @@ int chan_mlp_set_data(chan_mlp *m, const float *X, const float *T, int64_t n) {
   if (!m || !X || !T || n < 1 || n > m->cap) return set_error(CHAN_E_ARG, "bad argument");
   int rc;
   if ((rc = row_workspace(m))) return rc;
-  hipError_t e = hipMemcpyAsync(m->Xf, X, sizeof(float) * n * IN, hipMemcpyHostToDevice, m->st);
+  hipError_t e = copy_to_device(m->stage, m->Xf, X, sizeof(float) * n * IN, m->st);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_to_bf16, dim3((unsigned)((n * KP + 255) / 256)), dim3(256), 0, m->st, m->Xf, m->X, n);
     e = hipGetLastError();
   }
-  if (e == hipSuccess) e = hipMemcpyAsync(m->T, T, sizeof(float) * n * OUT, hipMemcpyHostToDevice, m->st);
+  if (e == hipSuccess) e = copy_to_device(m->stage, m->T, T, sizeof(float) * n * OUT, m->st);
   if (e == hipSuccess) e = hipMemsetAsync(m->m1, 0, sizeof(float) * GSIZE, m->st);
   if (e == hipSuccess) e = hipMemsetAsync(m->m2, 0, sizeof(float) * GSIZE, m->st);
   if (e == hipSuccess) e = hipStreamSynchronize(m->st);
@@ -707,10 +710,9 @@ int chan_mlp_forward(chan_mlp *m, const float *X, int64_t n, float *Y) {
   if (!m || !X || !Y || n < 1 || n > m->cap) return set_error(CHAN_E_ARG, "bad argument");
   int rc;
   if ((rc = row_workspace(m))) return rc;
-  hipError_t e = hipMemcpyAsync(m->Xf, X, sizeof(float) * n * IN, hipMemcpyHostToDevice, m->st);
+  hipError_t e = copy_to_device(m->stage, m->Xf, X, sizeof(float) * n * IN, m->st);
   if (e == hipSuccess) e = launch_fwd(m, FromFloat{m->Xf}, n, m->Y, m->st);
-  if (e == hipSuccess) e = hipMemcpyAsync(Y, m->Y, sizeof(float) * n * OUT, hipMemcpyDeviceToHost, m->st);
-  if (e == hipSuccess) e = hipStreamSynchronize(m->st);
+  if (e == hipSuccess) e = copy_to_host(m->stage, Y, m->Y, sizeof(float) * n * OUT, m->st);
   if (e != hipSuccess) return set_error((int)e, "forward: %s", hipGetErrorString(e));
   return 0;
 }
