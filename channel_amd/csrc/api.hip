@@ -98,11 +98,32 @@ struct StepRow {
   double lo[2][5], hi[2][5];
   DevScalars sc;
 };
+// The largest of the CFL_SLOTS running maxima and before, which start again at 0;
+// called by one whole wave.
+__device__ __forceinline__ unsigned long long take_cfl(unsigned long long *slots, unsigned long long before) {
+  static_assert(CFL_SLOTS == 64, "a slot per lane");
+  unsigned long long *mine = slots + threadIdx.x * CFL_STRIDE, m = *mine;
+  *mine = 0ull;
+  m = m > before ? m : before;
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1) {
+    const unsigned long long o = __shfl_xor(m, s, 64);
+    m = o > m ? o : m;
+  }
+  return m;
+}
+__global__ void k_fold_cfl(unsigned long long *slots, DevScalars *sc) {
+  const unsigned long long m = take_cfl(slots, sc->cfl_bits);
+  if (threadIdx.x == 0) sc->cfl_bits = m;
+}
 // The running CFL maximum restarts at 0.
-__global__ void k_step_row(const cx<double> *__restrict__ V, StepRow *__restrict__ out, DevScalars *sc, Geom g) {
+__global__ void k_step_row(const cx<double> *__restrict__ V, StepRow *__restrict__ out, DevScalars *sc,
+                           unsigned long long *cfl_max, Geom g) {
   const int t = threadIdx.x;
+  DevScalars s = *sc;
+  s.cfl_bits = take_cfl(cfl_max, s.cfl_bits);
   if (t == 0) {
-    out->sc = *sc;
+    out->sc = s;
     sc->cfl_bits = 0ull;
   }
   if (t >= 20) return;
@@ -368,7 +389,7 @@ int chan_create(const chan_params *p, chan_ctx **out) {
   if ((rc = dalloc(&c->d0fac, (size_t)(g.ny + 1) * 5))) return bail(rc);
   if ((rc = dalloc(&c->y, (size_t)g.Ny))) return bail(rc);
   if ((rc = dalloc(&c->dy, (size_t)g.ny + 1))) return bail(rc);
-  if ((rc = dalloc(&c->sc, 1))) return bail(rc);
+  if ((rc = dalloc(&c->sc, 1)) || (rc = dalloc(&c->cfl_max, CFL_SLOTS * CFL_STRIDE))) return bail(rc);
   if ((rc = dalloc(&c->stat, (size_t)10 * (g.ny + 1)))) return bail(rc);
 
   auto upload_tw = [&](auto proto) {
@@ -420,7 +441,9 @@ int chan_create(const chan_params *p, chan_ctx **out) {
   std::memset(&s0, 0, sizeof s0);
   s0.meanpx = p->meanpx;
   s0.meanpz = p->meanpz;
-  if (hipMemcpy(c->sc, &s0, sizeof s0, hipMemcpyHostToDevice) != hipSuccess) return bail(fail(CHAN_E_STATE, "upload failed"));
+  if (hipMemcpy(c->sc, &s0, sizeof s0, hipMemcpyHostToDevice) != hipSuccess ||
+      hipMemset(c->cfl_max, 0, sizeof(unsigned long long) * CFL_SLOTS * CFL_STRIDE) != hipSuccess)
+    return bail(fail(CHAN_E_STATE, "upload failed"));
   // stored explicit terms start at zero (ODE3 = 0 in the first substep)
   if (hipMemset(c->old, 0, esz * 2 * (g.ny - 1) * plane) != hipSuccess ||
       hipMemset(c->V, 0, sizeof(cx<double>) * 3 * NyP) != hipSuccess)
@@ -441,7 +464,7 @@ int chan_destroy(chan_ctx *c) {
   }
   for (auto e : c->pool) hipEventDestroy(e);
   void *bufs[] = {c->V, c->old, c->rhs, c->L, c->A, c->B, c->P, c->twz, c->twx, c->twzs, c->twxs,
-                  c->der, c->derT, c->derF, c->tab, c->d0fac, c->y, c->dy, c->sc, c->stat, c->F0, c->gain, c->Fkeep};
+                  c->der, c->derT, c->derF, c->tab, c->d0fac, c->y, c->dy, c->sc, c->cfl_max, c->stat, c->F0, c->gain, c->Fkeep};
   for (void *b : bufs)
     if (b) hipFree(b);
   if (c->st) hipStreamDestroy(c->st);
@@ -622,6 +645,8 @@ int chan_get_rhs(chan_ctx *c, double *R) {
 int chan_get_scalars(chan_ctx *c, chan_scalars *s) {
   if (!c || !s) return fail(CHAN_E_ARG, "null argument");
   DevScalars d;
+  hipLaunchKernelGGL(k_fold_cfl, dim3(1), dim3(64), 0, c->st, c->cfl_max, c->sc);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(&d, c->sc, sizeof d, hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));
   s->time = c->time;
@@ -652,6 +677,8 @@ int chan_set_scalars(chan_ctx *c, const chan_scalars *s) {
   std::memcpy(&d.cfl_bits, &cf, sizeof cf);
   c->time = s->time;
   c->deltat = s->deltat;
+  hipLaunchKernelGGL(k_fold_cfl, dim3(1), dim3(64), 0, c->st, c->cfl_max, c->sc);  // empties the slots
+  HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(c->sc, &d, sizeof d, hipMemcpyHostToDevice, c->st));
   HIPCHK(hipStreamSynchronize(c->st));
   return 0;
@@ -681,7 +708,7 @@ static int products_t(chan_ctx *c, int plane0, int nplanes, bool prods, int cfl)
   if ((rc = timed(c, small ? "zinv" : "zinv_cfl", [&] { return launch_zinv<R>(g.nzd, c->st, c->V, A, twz, g, plane0, nplanes); }))) return rc;
   if ((rc = timed(c, small ? "xpass" : (prods ? "xpass_cfl" : "cfl"), [&] {
          return launch_xpass<R>(M, c->st, A, B, twx, g, plane0, nplanes, prods, cfl, c->dy, h.dx, h.dz, factor,
-                                &c->sc->cfl_bits);
+                                c->cfl_max);
        })))
     return rc;
   if (prods)
@@ -836,7 +863,7 @@ int chan_outstats(chan_ctx *c, double row[11]) {
   // one kernel writes the rows and scalars and resets the running CFL maximum
   // (cfl=0 in outstats)
   StepRow *const row0 = static_cast<StepRow *>(c->step_row);
-  hipLaunchKernelGGL(k_step_row, dim3(1), dim3(64), 0, c->st, c->V, row0, c->sc, g);
+  hipLaunchKernelGGL(k_step_row, dim3(1), dim3(64), 0, c->st, c->V, row0, c->sc, c->cfl_max, g);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(c->st));
   const StepRow s = *row0;

@@ -43,6 +43,7 @@ struct chan_ctx {
   chan::cx<double> *Fkeep = nullptr;
   int kept_state = 0;
   chan::DevScalars *sc = nullptr;
+  unsigned long long *cfl_max = nullptr;  // CFL_SLOTS running maxima
   chan::HostStage stage;  // of fields on their way to and from the host
   // host scalars
   double time = 0, deltat = 0;

@@ -153,15 +153,17 @@ __device__ __forceinline__ void block_max_atomic(double m, double *red, unsigned
     red[threadIdx.x] = m;
     __syncthreads();
 #pragma unroll
-    for (int s = NT / 2; s > 0; s >>= 1) {
-      if ((int)threadIdx.x < s) red[threadIdx.x] = mx(red[threadIdx.x], red[threadIdx.x + s]);
+    for (int n = NT; n > 1; n = (n + 1) / 2) {
+      const int h = (n + 1) / 2;
+      if ((int)threadIdx.x + h < n) red[threadIdx.x] = mx(red[threadIdx.x], red[threadIdx.x + h]);
       __syncthreads();
     }
     r = red[0];
   }
   // values are >= 0 or NaN, so their bit patterns order as unsigned
   // integers (NaN above +Inf above every finite value)
-  if (threadIdx.x == 0) atomicMax(out, (unsigned long long)__double_as_longlong(r));
+  if (threadIdx.x == 0)
+    atomicMax(out + (blockIdx.x % CFL_SLOTS) * CFL_STRIDE, (unsigned long long)__double_as_longlong(r));
 }
 
 // Product pairs: fields 0 uu-ww, 1 vv-ww, 2 uv, 3 vw, 4 uw as the real and
@@ -223,7 +225,7 @@ template <int M, typename R, bool PRODUCTS, int MO_ = xmodes<fft::Plan<M>::E>(),
 __global__ __launch_bounds__((xteams<M, R>() * fft::Plan<M>::T), 2) void k_xpass(const cx<R> *__restrict__ A, cx<R> *__restrict__ B,
                                                                 const cx<R> *__restrict__ tw, Geom g, int plane0,
                                                                 int cfl_on, const double *__restrict__ dy, double dx,
-                                                                double dz, R factor, unsigned long long *__restrict__ cfl_bits,
+                                                                double dz, R factor, unsigned long long *__restrict__ cfl_max,
                                                                 int nplanes) {
   using PL = fft::Plan<M>;
   constexpr int TB = xteams<M, R>();
@@ -424,7 +426,7 @@ __global__ __launch_bounds__((xteams<M, R>() * fft::Plan<M>::T), 2) void k_xpass
         m = (c > m || c != c) ? c : m;
       }
     }
-    block_max_atomic<NT>(m, red, cfl_bits);
+    block_max_atomic<NT>(m, red, cfl_max);
   }
 
   if constexpr (PRODUCTS) {
@@ -607,6 +609,100 @@ __global__ __launch_bounds__((xrows<M>() * fft::Plan<M>::T), (sizeof(R) == 8 ? 3
       }
     }
     __syncthreads();
+  }
+}
+
+// -------------------------------------------------------- K2, few rows --
+// The x pass of short rows, whose teams of less than 16 lanes leave k_xpass's waves
+// half empty, and of few rows: three teams per row, one for each field on the way
+// in and one for each product pair on the way out, so that a row's chain is two
+// transforms instead of five.  They meet in LDS: the samples and the products' modes
+// of a z block's rows, which its threads then write out as whole runs.
+//
+// Bound by that chain where the rows are few: 15x32x15 (rows of 48) 8.9 for 13.0 us,
+// 31x64x31 (96) 19.8 for 22.0, 23x64x31 (72) 18.8 for 23.4.
+template <int M, typename R>
+__global__ __launch_bounds__(3 * ZB * fft::Plan<M>::T) void k_xpass_few(const cx<R> *__restrict__ A, cx<R> *__restrict__ B,
+                                                                        const cx<R> *__restrict__ tw, Geom g, int plane0,
+                                                                        int cfl_on, const double *__restrict__ dy, double dx,
+                                                                        double dz, R factor,
+                                                                        unsigned long long *__restrict__ cfl_max) {
+  using PL = fft::Plan<M>;
+  constexpr int T = PL::T, E = PL::E, MO = xmodes<E>(), NT = 3 * ZB * T, XC = fft::XCH_CPLX | fft::XCH_PAD;
+  constexpr int ROW = fft::xch_len<M, fft::XCH_PAD>(), NTW = fft::plan_tw_size(M, true);
+  __shared__ __align__(16) cx<R> lds[3 * ZB * ROW];
+  __shared__ __align__(16) cx<R> twl[NTW > 0 ? NTW : 1];
+  __shared__ double red[NT];
+  const int nx = g.nx, Nx = g.Nx, NZB = g.nzd / ZB, zb = blockIdx.x % NZB, pl = blockIdx.x / NZB, iy = plane0 + pl - 1;
+  const int tid = threadIdx.x, t = tid % T, zi = tid / T % ZB, c = tid / (T * ZB);
+  cx<R> *mine = lds + (c * ZB + zi) * ROW;
+  R *fr = reinterpret_cast<R *>(mine);
+  cx<R> e[E];
+  {
+    const cx<R> *src = A + ((size_t)(pl * 3 + c) * NZB + zb) * Nx * ZB + zi;
+#pragma unroll
+    for (int s = 0; s < E; s++) {
+      e[s] = cx<R>{0, 0};
+      if (s >= MO && s < E - MO) continue;
+      const int k = t + T * s, m = s < MO ? k : M - k;
+      if (m <= nx) e[s] = src[(size_t)m * ZB];
+      if (s >= MO) e[s].y = -e[s].y;
+      if (k == 0) e[s].y = 0;  // as c2r does
+    }
+  }
+  for (int i = tid; i < NTW; i += NT) twl[i] = tw[i];
+  __syncthreads();
+  fft::fft_slots<M, +1, true, XC>(e, fr, twl, t);
+#pragma unroll
+  for (int s = 0; s < E; s++) fr[t + T * s] = e[s].x;
+  __syncthreads();
+  const R *u = reinterpret_cast<const R *>(lds + zi * ROW), *v = u + 2 * ZB * ROW, *w = v + 2 * ZB * ROW;
+  // the CFL maximum as k_xpass takes it, a third of the samples per team
+  if (cfl_on && iy >= 1 && iy <= g.ny - 1) {
+    const double dyv = dy[iy];
+    const double rx = 1.0 / dx, ry = 1.0 / dyv, rz = 1.0 / dz;
+    double m = 0.0;
+#pragma unroll
+    for (int j = 0; j < (E + 2) / 3; j++) {
+      const int n = t + T * (3 * j + c);
+      if (n >= M) continue;
+      const double au = fabs((double)u[n]), av = fabs((double)v[n]), aw = fabs((double)w[n]);
+      const double q = sizeof(R) == 4 ? au * rx + av * ry + aw * rz
+                                      : div_by(au, dx, rx) + div_by(av, dyv, ry) + div_by(aw, dz, rz);
+      m = (q > m || q != q) ? q : m;
+    }
+    block_max_atomic<NT>(m, red, cfl_max);
+  }
+#pragma unroll
+  for (int s = 0; s < E; s++) {
+    const int n = t + T * s;
+    const R a = u[n], b = v[n], d = w[n];
+    e[s].x = c == 0 ? a * a - d * d : (c == 1 ? a * d : b * d);  // product_pair(c, a, b, d)
+    e[s].y = c == 0 ? a * b : (c == 1 ? b * b - d * d : R(0));
+  }
+  __syncthreads();
+  fft::fft_slots<M, -1, true, XC>(e, fr, twl, t);
+#pragma unroll
+  for (int s = 0; s < E; s++)
+    if (s < MO || s >= E - MO) mine[t + T * s] = e[s];
+  __syncthreads();
+  const R hf = R(0.5) * factor;
+  const int first = c == 0 ? pair_first(0) : (c == 1 ? pair_first(1) : pair_first(2));
+  cx<R> *da = B + ((size_t)(pl * NPROD + first) * NZB + zb) * Nx * ZB;
+  cx<R> *db = B + ((size_t)(pl * NPROD + pair_second(c)) * NZB + zb) * Nx * ZB;
+#pragma unroll
+  for (int j = 0; j < MO; j++) {
+    const int i = zi * T + t + ZB * T * j, k = i / ZB;
+    if (i >= ZB * Nx) continue;
+    const cx<R> *row = lds + (c * ZB + i % ZB) * ROW;
+    const cx<R> z0 = row[k];
+    if (c == 2) {
+      da[i] = cx<R>{z0.x * factor, z0.y * factor};
+    } else {
+      const cx<R> q = row[k ? M - k : 0];
+      da[i] = cx<R>{(z0.x + q.x) * hf, (z0.y - q.y) * hf};
+      db[i] = cx<R>{(z0.y + q.y) * hf, (q.x - z0.x) * hf};
+    }
   }
 }
 
@@ -801,6 +897,19 @@ hipError_t launch_fft_bench(int N, int sign, int variant, const cx<double> *in, 
 #define CHAN_FOR_NINES(X) X(36) X(72) X(144) X(288) X(576) X(1152)
 #define CHAN_FOR_SIZES(X) X(12) X(24) X(48) X(96) X(192) X(384) X(768) X(1536) X(16) X(32) X(64) X(128) X(256) X(512) X(1024)
 
+#define CHAN_FOR_FEW(X) X(12) X(24) X(48) X(96) X(16) X(32) X(64) X(128) X(36) X(72)
+// sizes whose products k_xpass_few always forms: it does six transforms for five,
+// but in full waves (31x128x31 28.9 for 34.5 us; 11x128x95, rows of 36 that
+// k_xpass_blk could take, 26.5 for 32.8)
+template <int M>
+constexpr bool few_always() {
+  return M == 36 || (M % 9 != 0 && fft::Plan<M>::T < 16);
+}
+// rows of 72 points fill k_xpass_blk's waves too: k_xpass_few has them while its
+// blocks of two waves are all resident, at four waves per SIMD (23x64x31, 1608 blocks,
+// 18.8 for 23.4 us; 23x128x95, 9432 blocks, 56.1 for 51.9)
+static bool use_few(int M, unsigned ntile, int ncu) { return M != 72 || ntile <= 8u * (unsigned)ncu; }
+
 template <typename R>
 hipError_t launch_zinv(int NZ, hipStream_t st, const cx<double> *V, cx<R> *A, const cx<R> *tw, const Geom &g, int plane0,
                        int nplanes) {
@@ -822,25 +931,42 @@ hipError_t launch_zinv(int NZ, hipStream_t st, const cx<double> *V, cx<R> *A, co
 template <typename R>
 hipError_t launch_xpass(int M, hipStream_t st, const cx<R> *A, cx<R> *B, const cx<R> *tw, const Geom &g, int plane0,
                         int nplanes, bool products, int cfl_on, const double *dy, double dx, double dz, R factor,
-                        unsigned long long *cfl_bits) {
+                        unsigned long long *cfl_max) {
   const unsigned ntile = (unsigned)((g.nzd / ZB) * nplanes);
+  if (products && use_few(M, ntile, g.ncu)) switch (M) {
+#define X(N)                                                                                                         \
+  case N:                                                                                                            \
+    hipLaunchKernelGGL((k_xpass_few<N, R>), dim3(ntile), dim3(3 * ZB * fft::Plan<N>::T), 0, st, A, B, tw, g, plane0, \
+                       cfl_on, dy, dx, dz, factor, cfl_max);                                                         \
+    return hipGetLastError();
+      CHAN_FOR_FEW(X)
+#undef X
+    }
   switch (M) {
 #define X(N)                                                                                                          \
   case N: {                                                                                                           \
     dim3 blk(xteams<N, R>() * fft::Plan<N>::T);                                                                       \
     dim3 grid(xteams<N, R>() < ZB ? 16 * ((ntile + 7) / 8) : ntile);                                                  \
-    if (products && N == 768 && g.nx + 1 == 192)                                                                      \
-      hipLaunchKernelGGL((k_xpass<N, R, true, (N == 768 ? 3 : xmodes<fft::Plan<N>::E>()), true>), grid, blk, 0, st, A, \
-                         B, tw, g, plane0, cfl_on, dy, dx, dz, factor, cfl_bits, nplanes);                            \
-    else if (products && N == 768 && g.nx + 1 <= 192)                                                                 \
-      hipLaunchKernelGGL((k_xpass<N, R, true, (N == 768 ? 3 : xmodes<fft::Plan<N>::E>())>), grid, blk, 0, st, A, B, tw, \
-                         g, plane0, cfl_on, dy, dx, dz, factor, cfl_bits, nplanes);                                   \
-    else if (products)                                                                                                \
-      hipLaunchKernelGGL((k_xpass<N, R, true>), grid, blk, 0, st, A, B, tw, g, plane0, cfl_on, dy, dx, dz, factor,    \
-                         cfl_bits, nplanes);                                                                          \
-    else                                                                                                              \
-      hipLaunchKernelGGL((k_xpass<N, R, false>), grid, blk, 0, st, A, B, tw, g, plane0, cfl_on, dy, dx, dz, factor,   \
-                         cfl_bits, nplanes);                                                                          \
+    if constexpr (!few_always<N>()) {                                                                                 \
+      if constexpr (N == 768) {                                                                                       \
+        if (products && g.nx + 1 <= 192) {                                                                            \
+          if (g.nx + 1 == 192)                                                                                        \
+            hipLaunchKernelGGL((k_xpass<N, R, true, 3, true>), grid, blk, 0, st, A, B, tw, g, plane0, cfl_on, dy, dx, \
+                               dz, factor, cfl_max, nplanes);                                                         \
+          else                                                                                                        \
+            hipLaunchKernelGGL((k_xpass<N, R, true, 3>), grid, blk, 0, st, A, B, tw, g, plane0, cfl_on, dy, dx, dz,   \
+                               factor, cfl_max, nplanes);                                                             \
+          return hipGetLastError();                                                                                   \
+        }                                                                                                             \
+      }                                                                                                               \
+      if (products) {                                                                                                 \
+        hipLaunchKernelGGL((k_xpass<N, R, true>), grid, blk, 0, st, A, B, tw, g, plane0, cfl_on, dy, dx, dz, factor,  \
+                           cfl_max, nplanes);                                                                         \
+        return hipGetLastError();                                                                                     \
+      }                                                                                                               \
+    }                                                                                                                 \
+    hipLaunchKernelGGL((k_xpass<N, R, false>), grid, blk, 0, st, A, B, tw, g, plane0, cfl_on, dy, dx, dz, factor,     \
+                       cfl_max, nplanes);                                                                             \
     return hipGetLastError();                                                                                         \
   }
     CHAN_FOR_SIZES(X)
@@ -849,8 +975,9 @@ hipError_t launch_xpass(int M, hipStream_t st, const cx<R> *A, cx<R> *B, const c
   case N: {                                                                                                           \
     if (!products || cfl_on) break;                                                                                   \
     constexpr int RW = xrows<N>();                                                                                    \
-    hipLaunchKernelGGL((k_xpass_blk<N, R>), dim3((ntile + RW / ZB - 1) / (RW / ZB)), dim3(RW * fft::Plan<N>::T), 0, \
-                       st, A, B, tw, g, factor, nplanes);                                                             \
+    if constexpr (!few_always<N>())                                                                                   \
+      hipLaunchKernelGGL((k_xpass_blk<N, R>), dim3((ntile + RW / ZB - 1) / (RW / ZB)), dim3(RW * fft::Plan<N>::T), 0, \
+                         st, A, B, tw, g, factor, nplanes);                                                           \
     return hipGetLastError();                                                                                         \
   }
     CHAN_FOR_NINES(X)
