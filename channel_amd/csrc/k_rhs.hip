@@ -33,10 +33,11 @@
 // by a kernel of their own and read back, 34 for 155 us per substep at
 // 63x96x47, 1.19 for 2.23 ms at 191x384x189.
 //
-// Bound by HBM on large grids: 5.8 GB per launch at 191x384x189 (FP64) in 1.21
-// ms, 4.8 TB/s, where a five-row window of the nine fields in two waves per
-// SIMD and 48-row chunks took 1.39; by the length of the walk on small ones
-// (31x64x31: 11.8 us, 61 before).
+// Bound by HBM and the memory-side cache on large grids: at 191x384x189 (FP64)
+// 1.13 ms with five product fields, 7.0 GB of counted traffic at 6.2 TB/s (1.21
+// with six, where a five-row window of the nine fields in two waves per SIMD and
+// 48-row chunks took 1.39); by the length of the walk on small ones (31x64x31:
+// 11.3 us, 61 before).
 #include "chan_internal.hpp"
 
 namespace chan {
@@ -265,7 +266,7 @@ hipError_t launch_force(hipStream_t st, const ForceArgs &a) {
 // one front, whose shared rows the memory-side cache still holds
 // (191x384x189: 1.21 ms with 8 rows, 1.30 with 48 or 96; 191x128x189 418 and
 // 445 us; 127x384x127, 510 blocks, 602 and 594 us, 578 with 96; with a body
-// force 1.19 and 1.29 ms at 191x384x189).
+// force 1.19 and 1.29 ms at 191x384x189; all with six product fields).
 static int rhs_chunk(const Geom &g) {
   const int blocks = (g.npair + RHS_BLOCK - 1) / RHS_BLOCK;
   if (blocks >= 1024) return 8;
