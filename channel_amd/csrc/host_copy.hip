@@ -29,12 +29,22 @@ void HostStage::free() {
 namespace {
 
 constexpr int MOVE_BLOCKS = 64;
-// Where staging begins.  To the host it wins from the first transfer that is worth
-// its threads (0.1 ms): 9 MB take 0.5 ms, 0.7 directly.  To the device the runtime
+// Where staging begins.  To the host it wins from the first size that is worth its
+// threads (0.1 ms): 9 MB take 0.5 ms, 0.7 directly.  To the device the runtime
 // pins the caller's pages and moves 29 GB/s, so the line lies where a first
 // transfer, which also pins the slots, is no slower: 115 MB first 3.7 ms, then 2.6,
 // directly 3.9; 75 MB first 4.0, then 1.8, directly 2.9 and 2.6; 12 MB the same 0.5.
 constexpr size_t TO_HOST_MIN = 8u << 20, TO_DEVICE_MIN = 96u << 20;
+
+// To the host an owner's first transfers go directly until they have moved what the
+// slots hold: what they lose by it (0.07 ms/MB) is then what pinning the slots costs
+// (2 to 3 ms), so that a short-lived owner does not pay for slots it will not use
+// (a first 15 MB took 2.0 ms with the pinning, 1.4 without).
+bool to_host_staged(HostStage &s, size_t bytes) {
+  if (s.ev[0]) return true;
+  s.direct += bytes;
+  return s.direct > STAGE_SLOTS * STAGE_CHUNK;
+}
 
 // Makes slot i, in the thread that uses it: pinning all at once takes twice the time.
 hipError_t make_slot(HostStage &s, int i) {
@@ -135,13 +145,15 @@ hipError_t staged(HostStage &s, char *host, char *device, size_t bytes, hipStrea
 
 template <bool TO_HOST>
 hipError_t copy(HostStage &s, void *host, void *device, size_t bytes, hipStream_t st) {
-  if (bytes >= (TO_HOST ? TO_HOST_MIN : TO_DEVICE_MIN) && pageable(host)) {
+  if (bytes >= (TO_HOST ? TO_HOST_MIN : TO_DEVICE_MIN) && pageable(host) && (!TO_HOST || to_host_staged(s, bytes))) {
     if (staged<TO_HOST>(s, static_cast<char *>(host), static_cast<char *>(device), bytes, st) == hipSuccess)
       return hipSuccess;
     (void)hipGetLastError();  // no pinned memory left, or a fault that the plain copy meets again
   }
-  const hipError_t e = TO_HOST ? hipMemcpyAsync(host, device, bytes, hipMemcpyDeviceToHost, st)
-                               : hipMemcpyAsync(device, host, bytes, hipMemcpyHostToDevice, st);
+  // to the device the caller's next wait serves as well: a wait of its own here took 7
+  // of 42 us from a small closure forward
+  if (!TO_HOST) return hipMemcpyAsync(device, host, bytes, hipMemcpyHostToDevice, st);
+  const hipError_t e = hipMemcpyAsync(host, device, bytes, hipMemcpyDeviceToHost, st);
   return e != hipSuccess ? e : hipStreamSynchronize(st);
 }
 

@@ -15,11 +15,13 @@ constexpr int STAGE_THREADS = 8, STAGE_SLOTS = 2 * STAGE_THREADS;
 struct HostStage {
   char *buf[STAGE_SLOTS] = {};
   hipEvent_t ev[STAGE_SLOTS] = {};
+  size_t direct = 0;  // bytes that went to the host without it
   void free();
 };
 
-// Copies `bytes` (a multiple of 4, device side aligned to 16) on the stream and
-// returns when they have arrived.  Large pageable buffers go through the stage in
+// Copies `bytes` (a multiple of 4, device side aligned to 16) on the stream.  To the
+// host it returns when they have arrived; to the device the stream may still be
+// copying, and the caller waits for it before it returns to its own.  Large pageable buffers go through the stage in
 // chunks, each of a few host threads filling or emptying its two slots while the
 // others' are on the bus; smaller ones and pinned memory are copied directly.
 hipError_t copy_to_host(HostStage &s, void *dst, const void *src, size_t bytes, hipStream_t st);
