@@ -80,7 +80,7 @@ def algorithmic_bytes(cfg, nxd, nzd, c=16):
 
 def cpu_threads():
     """Threads for the oracle: the CPUs this process may run on, capped by
-    OMP_NUM_THREADS when that is set (the GPU box sets it to the host share
+    OMP_NUM_THREADS when that is set (a launcher sets it to the host share
     that goes with one GPU)."""
     try:
         avail = len(os.sched_getaffinity(0))
