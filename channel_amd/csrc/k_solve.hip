@@ -731,10 +731,24 @@ __device__ __forceinline__ void lds_sweeps(const SolveArgs &a, const Band &band,
   }
 }
 
-// dv/dy of the v columns x, in place
+// Orders a wave's LDS accesses where its lanes exchange data.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// dv/dy of the v columns x, in place.  The stencils of the innermost rows reach
+// three rows of the other half, which its lanes of the same wave overwrite: they
+// are taken between two fences, before either half starts.
 __device__ __forceinline__ void lds_dv(const UwArgs &uw, const Half h, const double *T, double *x, const int ny) {
   const int m = (ny - 1) / 2;
   const bool more = ((ny - 1) & 1) && !h.up;
+  wave_sync();
+  double vo[3];  // v of the rows m + 1 .. m + 3
+#pragma unroll
+  for (int j = 0; j < 3; j++) vo[j] = x[h.x0 + (m + 1 + j) * h.xs];
+  wave_sync();
   // one-sided derivatives at the wall (fw) and the ghost row (fg): the window
   // w[j] = v of row k + 2 - j in the mirrored frame, here at k = 1
   double w[5], fw = 0.0, fg = 0.0;
@@ -747,15 +761,17 @@ __device__ __forceinline__ void lds_dv(const UwArgs &uw, const Half h, const dou
   constexpr int U = 4;
   double x1 = 0.0, x2 = 0.0, vr[U], dr[U][8];  // v of row k + 3, d1 and the factors D[2..4] of the rows ahead
   auto fetch = [&](int k, int u) {
-    vr[u] = x[h.x0 + min(k + 3, m + 3) * h.xs];
+    vr[u] = x[h.x0 + min(k + 3, m) * h.xs];
     const double *t = T + h.t0 + min(k, m + 1) * h.ts;
 #pragma unroll
     for (int j = 0; j < 5; j++) dr[u][j] = t[15 + j];
 #pragma unroll
     for (int j = 0; j < 3; j++) dr[u][5 + j] = t[22 + j];
   };
-  auto in = [&](int k, int u, double g) {
-    const double vnext = vr[u];
+  auto in = [&](auto inner, int k, int u, double g) {
+    double vnext = vr[u];
+    if constexpr (decltype(inner)::value)
+      if (k + 3 > m) vnext = k + 2 == m ? vo[0] : (k + 1 == m ? vo[1] : vo[2]);
     double d[8];
 #pragma unroll
     for (int j = 0; j < 8; j++) d[j] = dr[u][j];
@@ -775,13 +791,16 @@ __device__ __forceinline__ void lds_dv(const UwArgs &uw, const Half h, const dou
   const double *t1 = T + h.t0 + h.ts;
   const double g1 = t1[3] * fw + t1[4] * fg, g2 = t1[h.ts + 4] * fw;
   int k = 1;
-  for (; k + (U - 1) <= m; k += U) {
+  for (; k + (U - 1) <= m - 3; k += U) {  // rows whose stencils stay in this half
 #pragma unroll
-    for (int u = 0; u < U; u++) in(k + u, u, u == 0 ? (k == 1 ? g1 : 0.0) : (u == 1 && k == 1 ? g2 : 0.0));
+    for (int u = 0; u < U; u++) in(std::false_type{}, k + u, u, u == 0 ? (k == 1 ? g1 : 0.0) : (u == 1 && k == 1 ? g2 : 0.0));
   }
+#pragma unroll 1
+  for (; k <= m; k += U) {
 #pragma unroll
-  for (int u = 0; u < U; u++)
-    if (k + u <= m) in(k + u, u, k + u == 1 ? g1 : (k + u == 2 ? g2 : 0.0));
+    for (int u = 0; u < U; u++)
+      if (k + u <= m) in(std::true_type{}, k + u, u, k + u == 1 ? g1 : (k + u == 2 ? g2 : 0.0));
+  }
   if (more) {
     double d[5], D[3];
     const double *t = T + h.t0 + (m + 1) * h.ts;
