@@ -485,12 +485,16 @@ int chan_les_closure_force(chan_ctx *c, chan_mlp *m, const float *norm) {
   for (int j = 0; j < 46; j++)
     if (!(norm[46 + j] > 0.0f)) return set_error(CHAN_E_ARG, "feature scale %d is not positive", j);
   float nv[mlp::NORM_RECIP + 46];
+  bool quick = true;
   std::memcpy(nv, norm, sizeof(float) * mlp::NORM_RECIP);
-  for (int j = 0; j < 46; j++) nv[mlp::NORM_RECIP + j] = 1.0f / norm[46 + j];
+  for (int j = 0; j < 46; j++) {
+    nv[mlp::NORM_RECIP + j] = 1.0f / norm[46 + j];
+    quick = quick && norm[46 + j] >= 1.0f / mlp::SPAN_D && norm[46 + j] <= mlp::SPAN_D;
+  }
   LCHK(hipMemcpyAsync(s->norm, nv, sizeof nv, hipMemcpyHostToDevice, c->st));
   if ((rc = les_gradients(c, s))) return rc;
   const LesGeom q = les_geom(c);
-  LCHK(mlp::forward_gradients(m, mlp::LesSource{s->Gp, s->norm, s->yplus, s->n, q.Mx * q.Mz, q.ny}, s->Y, c->st));
+  LCHK(mlp::forward_gradients(m, mlp::LesSource{s->Gp, s->norm, s->yplus, s->n, q.Mx * q.Mz, q.ny, quick}, s->Y, c->st));
   if ((rc = les_fits(q, true))) return rc;
   hipLaunchKernelGGL(k_les_tau, dim3(q.ny + 1, 6), dim3(GT), tau_lds(q), c->st, s->Y, q, s->norm, s->twz, s->phxT, s->T);
   LCHK(hipGetLastError());

@@ -68,12 +68,15 @@ namespace chan {
 namespace mlp {
 // The velocity gradients of a closure grid: G[9][n] on rows 0..ny of `plane`
 // points each (n = (ny + 1) plane), y+ per row, and the normalisation
-// [46 mean][46 scale][12 of the stresses][46 reciprocal scales].
+// [46 mean][46 scale][12 of the stresses][46 reciprocal scales].  quick: every scale
+// is in [1 / SPAN_D, SPAN_D], where quotients may be formed from the reciprocals.
 constexpr int NORM_RECIP = 2 * IN + 2 * OUT;
+constexpr float SPAN_D = 0x1p26f;
 struct LesSource {
   const float *G, *norm;
   const double *yplus;
   int n, plane, ny;
+  bool quick;
 };
 // inference of model m on the features of s -> Y[n][6] FP32, enqueued on stream
 // st (k_mlp.hip)

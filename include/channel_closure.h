@@ -91,7 +91,9 @@ int chan_les_features(chan_ctx *c, float *X);
 /* Sets the context's static body force (the F0 of chan_set_body_force) to
  * -div(tau), tau = MLP(m) of the normalised features of the resident field:
  * inputs (X - xmean) / xscale, stresses tau = Y * tscale + tmean, with
- * norm = [46 xmean][46 xscale][6 tmean][6 tscale].  Everything stays on the
+ * norm = [46 xmean][46 xscale][6 tmean][6 tscale]; the scales are positive,
+ * infinite ones mask their features (the quotients are IEEE division's), others
+ * are refused with CHAN_E_ARG.  Everything stays on the
  * device; the next chan_step / chan_buildrhs applies the force with the
  * wall treatment of chan_set_body_force. */
 int chan_les_closure_force(chan_ctx *c, chan_mlp *m, const float *norm);
