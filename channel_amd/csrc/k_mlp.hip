@@ -542,7 +542,7 @@ struct chan_mlp {
   __bf16 *X = nullptr;        // [cap][64]
   float *T = nullptr;         // [cap][6]
   float *Xf = nullptr;        // [cap][46] host rows on their way in, made on first use
-  float *Y = nullptr;         // [cap][6]
+  float *Y = nullptr;         // [cap][6], at least [CHAN_MLP_NOALLOC_MAX][6]
   float *master = nullptr, *m1 = nullptr, *m2 = nullptr, *g = nullptr;  // [GSIZE]
   float *part = nullptr;      // gradient partials [gvec][GSIZE]
   float *lpart = nullptr;     // loss partials [GBLK], then the loss of chan_mlp_grad
@@ -581,6 +581,10 @@ __global__ void k_to_bf16(const float *__restrict__ x, __bf16 *__restrict__ xb, 
   const int64_t r = i / KP;
   const int c = (int)(i % KP);
   xb[i] = (__bf16)(c < IN ? x[r * IN + c] : 0.0f);
+}
+
+__global__ __launch_bounds__(256) void k_move_outputs(const float *__restrict__ a, float *__restrict__ b, int n) {
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) b[i] = a[i];
 }
 
 // Blocks of k_mlp_fwd: its waves keep the weights in registers, so each takes
@@ -657,7 +661,7 @@ int chan_mlp_create(int64_t capacity, chan_mlp **out) {
   };
   if (hipStreamCreate(&m->st) != hipSuccess) return bail(set_error(CHAN_E_STATE, "hipStreamCreate failed"));
   const size_t c = (size_t)capacity;
-  if ((rc = mal(&m->X, c * KP)) || (rc = mal(&m->T, c * OUT)) || (rc = mal(&m->Y, c * OUT)) ||
+  if ((rc = mal(&m->X, c * KP)) || (rc = mal(&m->T, c * OUT)) || (rc = mal(&m->Y, std::max(c, (size_t)CHAN_MLP_NOALLOC_MAX) * OUT)) ||
       (rc = mal(&m->master, GSIZE)) || (rc = mal(&m->m1, GSIZE)) || (rc = mal(&m->m2, GSIZE)) ||
       (rc = mal(&m->g, GSIZE)) || (rc = mal(&m->part, (size_t)m->gvec * GSIZE)) ||
       (rc = mal(&m->lpart, (size_t)GBLK + 1)) ||
@@ -743,8 +747,17 @@ int chan_mlp_forward_noalloc(chan_mlp *m, const float *dX, int64_t n, float *dY)
   int dev = -1;
   MCHK(hipGetDevice(&dev));
   if (dev != m->dev) return set_error(CHAN_E_STATE, "chan_mlp_forward_noalloc: device %d is current, the model lives on %d", dev, m->dev);
-  // the same kernel and launch shape as chan_mlp_forward
-  MCHK(launch_fwd(m, FromFloat{dX}, n, dY, m->st));
+  // the same kernel and launch shape as chan_mlp_forward.  Its waves store outputs
+  // while others still read rows: buffers that overlap go through the model's own
+  // output rows.
+  const uintptr_t x = (uintptr_t)dX, y = (uintptr_t)dY;
+  const bool overlap = x < y + (size_t)n * OUT * sizeof(float) && y < x + (size_t)n * IN * sizeof(float);
+  MCHK(launch_fwd(m, FromFloat{dX}, n, overlap ? m->Y : dY, m->st));
+  if (overlap) {
+    hipLaunchKernelGGL(k_move_outputs, dim3((unsigned)std::min<int64_t>(256, (n * OUT + 255) / 256)), dim3(256), 0, m->st,
+                       m->Y, dY, (int)(n * OUT));
+    MCHK(hipGetLastError());
+  }
   MCHK(hipStreamSynchronize(m->st));
   return 0;
 }

@@ -20,7 +20,7 @@ CHAN_E_NOTFINITE = -3
 CHAN_E_CPITYPE = -4
 CHAN_E_STATE = -5
 CHAN_E_NODEV = -6
-# rows that chan_mlp_forward_noalloc stages (include/channel_closure.h)
+# rows that chan_mlp_forward_noalloc takes (include/channel_closure.h)
 CHAN_MLP_NOALLOC_MAX = 65536
 
 _lib = None

@@ -53,7 +53,8 @@ int chan_mlp_forward(chan_mlp *m, const float *X, int64_t n, float *Y);
  * dY[n][6] (FP32), both device pointers of the model's GPU, which must be
  * current.  Same kernel and results as chan_mlp_forward; the BF16 inputs are
  * formed in registers.  n > CHAN_MLP_NOALLOC_MAX is rejected with CHAN_E_ARG:
- * split the call.  Runs on the model's stream and returns when it is done.
+ * split the call.  dX and dY may overlap in any way.  Runs on the model's stream
+ * and returns when it is done.
  * No counterpart in the reference: it is for callers that cannot allocate
  * device memory (code under HIP graph capture, serving loops, harnesses that
  * forbid hipMalloc). */
