@@ -287,11 +287,11 @@ struct GradLds {
   __bf16 dz[3][64 * SP];   // dz of the hidden layers
   __bf16 dy[OP * SP];
   float bias[BSIZE];
-  float red[4];
+  double red[4];
 };
 __global__ __launch_bounds__(256) void k_mlp_grad(Weights w, const __bf16 *__restrict__ X, const float *__restrict__ Tg,
                                                   int n, float inv_count, int chunk, int per,
-                                                  float *__restrict__ part, float *__restrict__ loss_part) {
+                                                  float *__restrict__ part, double *__restrict__ loss_part) {
   extern __shared__ __align__(16) char smem[];
   GradLds &S = *reinterpret_cast<GradLds *>(smem);
   for (int i = threadIdx.x; i < BSIZE; i += 256) S.bias[i] = w.bias[i];
@@ -307,7 +307,8 @@ __global__ __launch_bounds__(256) void k_mlp_grad(Weights w, const __bf16 *__res
   for (int mt = 0; mt < 4; mt++)
 #pragma unroll
     for (int nt = 0; nt < 4; nt++) acc[mt][nt] = g[mt][nt] = f32x4{0, 0, 0, 0};
-  float bacc = 0.0f, bsum = 0.0f, lsum = 0.0f;
+  float bacc = 0.0f, bsum = 0.0f;
+  double lsum = 0.0;
   auto store = [&](const f32x4(&v)[4][4], float bias, int at) {
     float *dst = part + (size_t)at * GSIZE + GOFF[wv];
 #pragma unroll
@@ -365,7 +366,7 @@ __global__ __launch_bounds__(256) void k_mlp_grad(Weights w, const __bf16 *__res
       for (int i = 0; i < 4; i++) {
         float d = o[i] + bb[i] - tg[i];
         if (!valid || 4 * q + i >= OUT) d = 0.0f;
-        lsum += d * d;
+        lsum += (double)d * d;
         dv[i] = (__bf16)(2.0f * d * inv_count);
         S.dy[(4 * q + i) * SP + sc] = dv[i];
       }
@@ -458,21 +459,22 @@ __global__ __launch_bounds__(256) void k_mlp_grad(Weights w, const __bf16 *__res
 // four slots in order), 64 loads in flight; ADAM then updates master/m/v
 // (padded kernel layout) and refreshes the BF16 weight copies in both orientations
 // and the FP32 biases.  Padding entries have zero gradient and stay zero.  The
-// last block sums the loss partials.
+// last block sums the loss partials, in FP64 as they are formed.
 struct AdamArgs {
   float *master, *m1, *m2;
   float lr, b1, b2, eps, c1, c2;
 };
 template <bool ADAM, bool SLOTS>
-__global__ __launch_bounds__(64) void k_mlp_update(const float *__restrict__ part, const float *__restrict__ loss_part,
-                                                   int nchunk, int nloss, float *__restrict__ g, float *__restrict__ loss,
+__global__ __launch_bounds__(64) void k_mlp_update(const float *__restrict__ part, const double *__restrict__ loss_part,
+                                                   int nchunk, int nloss, float *__restrict__ g,
+                                                   std::conditional_t<ADAM, float, double> *__restrict__ loss,
                                                    AdamArgs a, Weights w) {
   if (blockIdx.x == gridDim.x - 1) {
-    float s = 0.0f;
+    double s = 0.0;
     for (int b = threadIdx.x; b < nloss; b += 64) s += loss_part[b];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if (threadIdx.x == 0) *loss = s;
+    if (threadIdx.x == 0) *loss = (std::conditional_t<ADAM, float, double>)s;
     return;
   }
   const int i = blockIdx.x * 64 + threadIdx.x;
@@ -520,9 +522,8 @@ __global__ __launch_bounds__(256) void k_mlp_refresh(const float *__restrict__ m
 }  // namespace chan
 
 // ================================================================ C-ABI ==
-#include <chrono>
-#include <cstring>
 #include <algorithm>
+#include <cstring>
 #include <vector>
 
 #include "../../include/channel_closure.h"
@@ -545,7 +546,7 @@ struct chan_mlp {
   float *Y = nullptr;         // [cap][6], at least [CHAN_MLP_NOALLOC_MAX][6]
   float *master = nullptr, *m1 = nullptr, *m2 = nullptr, *g = nullptr;  // [GSIZE]
   float *part = nullptr;      // gradient partials [gvec][GSIZE]
-  float *lpart = nullptr;     // loss partials [GBLK], then the loss of chan_mlp_grad
+  double *lpart = nullptr;    // loss partials [GBLK], then the loss of chan_mlp_grad
   float *losses = nullptr;    // per training step
   __bf16 *woi = nullptr, *wio = nullptr;
   float *bias = nullptr;
@@ -600,7 +601,8 @@ hipError_t launch_fwd(chan_mlp *m, const Src &src, int64_t n, float *Y, hipStrea
 }
 
 // Gradient of the minibatch [first, first+count): partials, then their sum into
-// m->g or, with `adam`, straight into the weights; the loss sum goes to *loss.
+// m->g and the loss sum to lpart[GBLK] or, with `adam`, straight into the weights
+// and *loss.
 // Chunks are whole multiples of 128 samples, at most GBLK of them; up to GBLK / 4
 // chunks are worked on slot by slot, by two blocks each.
 int grad_pass(chan_mlp *m, int64_t first, int count, const AdamArgs *adam, float *loss) {
@@ -612,15 +614,15 @@ int grad_pass(chan_mlp *m, int64_t first, int count, const AdamArgs *adam, float
   hipLaunchKernelGGL(k_mlp_grad, dim3(nb), dim3(256), sizeof(GradLds), m->st, weights(m), m->X + first * KP,
                      m->T + first * OUT, count, 1.0f / (6.0f * count), chunk, slots ? 2 : 4, m->part, m->lpart);
   MCHK(hipGetLastError());
-  auto update = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3((GSIZE + 63) / 64 + 1), dim3(64), 0, m->st, m->part, m->lpart, nchunk, nb, m->g, loss,
+  auto update = [&](auto kernel, auto *sum) {
+    hipLaunchKernelGGL(kernel, dim3((GSIZE + 63) / 64 + 1), dim3(64), 0, m->st, m->part, m->lpart, nchunk, nb, m->g, sum,
                        adam ? *adam : AdamArgs{}, weights(m));
     return hipGetLastError();
   };
   if (adam)
-    MCHK(slots ? update(k_mlp_update<true, true>) : update(k_mlp_update<true, false>));
+    MCHK(slots ? update(k_mlp_update<true, true>, loss) : update(k_mlp_update<true, false>, loss));
   else
-    MCHK(slots ? update(k_mlp_update<false, true>) : update(k_mlp_update<false, false>));
+    MCHK(slots ? update(k_mlp_update<false, true>, m->lpart + GBLK) : update(k_mlp_update<false, false>, m->lpart + GBLK));
   return 0;
 }
 
@@ -765,14 +767,14 @@ int chan_mlp_forward_noalloc(chan_mlp *m, const float *dX, int64_t n, float *dY)
 int chan_mlp_grad(chan_mlp *m, int64_t first, int64_t count, float *grad, double *loss) {
   if (!m || !grad || !loss || first < 0 || count < 1 || first + count > m->n) return set_error(CHAN_E_ARG, "bad argument");
   int rc;
-  if ((rc = grad_pass(m, first, (int)count, nullptr, m->lpart + GBLK))) return rc;
+  if ((rc = grad_pass(m, first, (int)count, nullptr, nullptr))) return rc;
   std::vector<float> pad(GSIZE);
-  float lsum = 0.0f;
+  double lsum = 0.0;
   MCHK(hipMemcpyAsync(pad.data(), m->g, sizeof(float) * GSIZE, hipMemcpyDeviceToHost, m->st));
   MCHK(hipMemcpyAsync(&lsum, m->lpart + GBLK, sizeof lsum, hipMemcpyDeviceToHost, m->st));
   MCHK(hipStreamSynchronize(m->st));
   for (int c = 0; c < NPARAM; c++) grad[c] = pad[canon_to_padded(c)];
-  *loss = (double)lsum / (6.0 * (double)count);
+  *loss = lsum / (6.0 * (double)count);
   return 0;
 }
 
