@@ -513,13 +513,20 @@ int chan_setup_host(const chan_params *p, int32_t sizes[5], double *y, double *d
   return 0;
 }
 
-int chan_set_field(chan_ctx *c, const double *V) {
-  if (!c || !V) return fail(CHAN_E_ARG, "null argument");
+// A host field to its device layout in V, by way of B.  Waits whatever fails: until
+// then the transfer may still read the caller's buffer.
+static hipError_t field_to_device(chan_ctx *c, const double *host, cx<double> *V) {
   const size_t n = (size_t)3 * c->g.npair * c->g.Ny;
   cx<double> *stage = static_cast<cx<double> *>(c->B);
-  HIPCHK(copy_to_device(c->stage, stage, V, n * sizeof(cx<double>), c->st));
-  HIPCHK(launch_to_device_layout(c->st, stage, c->V, c->g));
-  HIPCHK(hipStreamSynchronize(c->st));
+  hipError_t e = copy_to_device(c->stage, stage, host, n * sizeof(cx<double>), c->st);
+  if (e == hipSuccess) e = launch_to_device_layout(c->st, stage, V, c->g);
+  const hipError_t end = hipStreamSynchronize(c->st);
+  return e != hipSuccess ? e : end;
+}
+
+int chan_set_field(chan_ctx *c, const double *V) {
+  if (!c || !V) return fail(CHAN_E_ARG, "null argument");
+  HIPCHK(field_to_device(c, V, c->V));
   c->field_set = true;
   return 0;
 }
@@ -543,11 +550,7 @@ int chan_set_body_force(chan_ctx *c, const double *F) {
   }
   int rc;
   if (!c->F0 && (rc = dalloc(&c->F0, 3 * (size_t)c->g.Ny * c->g.ps))) return rc;
-  const size_t n = (size_t)3 * c->g.npair * c->g.Ny;
-  cx<double> *stage = static_cast<cx<double> *>(c->B);
-  HIPCHK(copy_to_device(c->stage, stage, F, n * sizeof(cx<double>), c->st));
-  HIPCHK(launch_to_device_layout(c->st, stage, c->F0, c->g));
-  HIPCHK(hipStreamSynchronize(c->st));
+  HIPCHK(field_to_device(c, F, c->F0));
   return 0;
 }
 

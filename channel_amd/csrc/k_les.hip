@@ -449,6 +449,25 @@ int les_gradients(chan_ctx *c, LesState *s) {
   return 0;
 }
 
+// the closure's force on the resident field into F0, enqueued on the context's stream
+int les_force(chan_ctx *c, LesState *s, chan_mlp *m, const float *norm, size_t norm_bytes, bool quick) {
+  int rc;
+  LCHK(hipMemcpyAsync(s->norm, norm, norm_bytes, hipMemcpyHostToDevice, c->st));
+  if ((rc = les_gradients(c, s))) return rc;
+  const LesGeom q = les_geom(c);
+  LCHK(mlp::forward_gradients(m, mlp::LesSource{s->Gp, s->norm, s->yplus, s->n, q.Mx * q.Mz, q.ny, quick}, s->Y, c->st));
+  if ((rc = les_fits(q, true))) return rc;
+  hipLaunchKernelGGL(k_les_tau, dim3(q.ny + 1, 6), dim3(GT), tau_lds(q), c->st, s->Y, q, s->norm, s->twz, s->phxT, s->T);
+  LCHK(hipGetLastError());
+  if (!c->F0) {
+    if ((rc = lmal(&c->F0, 3 * (size_t)q.Ny * q.ps))) return rc;
+    LCHK(hipMemsetAsync(c->F0, 0, sizeof(cx<double>) * 3 * (size_t)q.Ny * q.ps, c->st));
+  }
+  hipLaunchKernelGGL(k_les_div, dim3((q.npair + 255) / 256, q.Ny), dim3(256), 0, c->st, s->T, q, s->ydc, s->ydr, c->F0);
+  LCHK(hipGetLastError());
+  return 0;
+}
+
 }  // namespace
 }  // namespace chan
 
@@ -491,20 +510,10 @@ int chan_les_closure_force(chan_ctx *c, chan_mlp *m, const float *norm) {
     nv[mlp::NORM_RECIP + j] = 1.0f / norm[46 + j];
     quick = quick && norm[46 + j] >= 1.0f / mlp::SPAN_D && norm[46 + j] <= mlp::SPAN_D;
   }
-  LCHK(hipMemcpyAsync(s->norm, nv, sizeof nv, hipMemcpyHostToDevice, c->st));
-  if ((rc = les_gradients(c, s))) return rc;
-  const LesGeom q = les_geom(c);
-  LCHK(mlp::forward_gradients(m, mlp::LesSource{s->Gp, s->norm, s->yplus, s->n, q.Mx * q.Mz, q.ny, quick}, s->Y, c->st));
-  if ((rc = les_fits(q, true))) return rc;
-  hipLaunchKernelGGL(k_les_tau, dim3(q.ny + 1, 6), dim3(GT), tau_lds(q), c->st, s->Y, q, s->norm, s->twz, s->phxT, s->T);
-  LCHK(hipGetLastError());
-  if (!c->F0) {
-    if ((rc = lmal(&c->F0, 3 * (size_t)q.Ny * q.ps))) return rc;
-    LCHK(hipMemsetAsync(c->F0, 0, sizeof(cx<double>) * 3 * (size_t)q.Ny * q.ps, c->st));
-  }
-  hipLaunchKernelGGL(k_les_div, dim3((q.npair + 255) / 256, q.Ny), dim3(256), 0, c->st, s->T, q, s->ydc, s->ydr, c->F0);
-  LCHK(hipGetLastError());
-  LCHK(hipStreamSynchronize(c->st));
+  rc = les_force(c, s, m, nv, sizeof nv, quick);
+  const hipError_t end = hipStreamSynchronize(c->st);  // until then nv may still be read
+  if (rc) return rc;
+  LCHK(end);
   return 0;
 }
 

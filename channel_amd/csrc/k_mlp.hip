@@ -626,6 +626,13 @@ int grad_pass(chan_mlp *m, int64_t first, int count, const AdamArgs *adam, float
   return 0;
 }
 
+// The stream's end, whatever failed before: until then a transfer may still read the
+// caller's rows.
+hipError_t settle(chan_mlp *m, hipError_t e) {
+  const hipError_t end = hipStreamSynchronize(m->st);
+  return e != hipSuccess ? e : end;
+}
+
 int row_workspace(chan_mlp *m) {
   int rc;
   if (!m->Xf && (rc = mal(&m->Xf, (size_t)m->cap * IN))) return rc;
@@ -695,10 +702,12 @@ int chan_mlp_set_params(chan_mlp *m, const float *params) {
   if (!m || !params) return set_error(CHAN_E_ARG, "null argument");
   std::vector<float> pad(GSIZE, 0.0f);
   for (int c = 0; c < NPARAM; c++) pad[canon_to_padded(c)] = params[c];
-  MCHK(hipMemcpyAsync(m->master, pad.data(), sizeof(float) * GSIZE, hipMemcpyHostToDevice, m->st));
-  hipLaunchKernelGGL(k_mlp_refresh, dim3((GSIZE + 255) / 256), dim3(256), 0, m->st, m->master, weights(m));
-  MCHK(hipGetLastError());
-  MCHK(hipStreamSynchronize(m->st));
+  hipError_t e = hipMemcpyAsync(m->master, pad.data(), sizeof(float) * GSIZE, hipMemcpyHostToDevice, m->st);
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL(k_mlp_refresh, dim3((GSIZE + 255) / 256), dim3(256), 0, m->st, m->master, weights(m));
+    e = hipGetLastError();
+  }
+  MCHK(settle(m, e));
   return 0;
 }
 
@@ -723,7 +732,7 @@ int chan_mlp_set_data(chan_mlp *m, const float *X, const float *T, int64_t n) {
   if (e == hipSuccess) e = copy_to_device(m->stage, m->T, T, sizeof(float) * n * OUT, m->st);
   if (e == hipSuccess) e = hipMemsetAsync(m->m1, 0, sizeof(float) * GSIZE, m->st);
   if (e == hipSuccess) e = hipMemsetAsync(m->m2, 0, sizeof(float) * GSIZE, m->st);
-  if (e == hipSuccess) e = hipStreamSynchronize(m->st);
+  e = settle(m, e);
   if (e != hipSuccess) return set_error((int)e, "set_data: %s", hipGetErrorString(e));
   m->n = n;
   m->adam_t = 0;
@@ -737,7 +746,7 @@ int chan_mlp_forward(chan_mlp *m, const float *X, int64_t n, float *Y) {
   hipError_t e = copy_to_device(m->stage, m->Xf, X, sizeof(float) * n * IN, m->st);
   if (e == hipSuccess) e = launch_fwd(m, FromFloat{m->Xf}, n, m->Y, m->st);
   if (e == hipSuccess) e = copy_to_host(m->stage, Y, m->Y, sizeof(float) * n * OUT, m->st);
-  if (e != hipSuccess) return set_error((int)e, "forward: %s", hipGetErrorString(e));
+  if (e != hipSuccess) return set_error((int)settle(m, e), "forward: %s", hipGetErrorString(e));
   return 0;
 }
 
