@@ -145,10 +145,14 @@ hipError_t staged(HostStage &s, char *host, char *device, size_t bytes, hipStrea
 
 template <bool TO_HOST>
 hipError_t copy(HostStage &s, void *host, void *device, size_t bytes, hipStream_t st) {
-  if (bytes >= (TO_HOST ? TO_HOST_MIN : TO_DEVICE_MIN) && pageable(host) && (!TO_HOST || to_host_staged(s, bytes))) {
+  if (!s.off && bytes >= (TO_HOST ? TO_HOST_MIN : TO_DEVICE_MIN) && pageable(host) && (!TO_HOST || to_host_staged(s, bytes))) {
     if (staged<TO_HOST>(s, static_cast<char *>(host), static_cast<char *>(device), bytes, st) == hipSuccess)
       return hipSuccess;
-    (void)hipGetLastError();  // no pinned memory left, or a fault that the plain copy meets again
+    // no pinned memory left, or a fault that the plain copy meets again: this owner
+    // gives back what it has and does not try once more
+    (void)hipGetLastError();
+    s.free();
+    s.off = true;
   }
   // to the device the caller's next wait serves as well: a wait of its own here took 7
   // of 42 us from a small closure forward

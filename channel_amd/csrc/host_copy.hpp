@@ -16,6 +16,7 @@ struct HostStage {
   char *buf[STAGE_SLOTS] = {};
   hipEvent_t ev[STAGE_SLOTS] = {};
   size_t direct = 0;  // bytes that went to the host without it
+  bool off = false;   // making or using the slots has failed
   void free();
 };
 
