@@ -14,13 +14,19 @@
 // stencil of v and one of eta = i kz u - i kx w.
 //
 // One thread per (pair, chunk of rows) walks y and adds each row, as it is
-// read, to the sums of the five output rows whose stencils reach it: four
-// complex sums per pending row (explicit and implicit part of each equation),
-// 80 FP64 registers' worth, where a five-row window of the eight fields that
+// read, to the sums of the five output rows whose stencils reach it: five
+// complex sums per pending row (explicit and implicit part of each equation, and
+// D2 v), 100 FP64 registers' worth, where a five-row window of the eight fields that
 // are read would be 40 complex values.  It then finishes the oldest row with
 // the CN-RK3 time scheme (:486), writes the new rhs and replaces the stored
 // explicit term.  The stencil coefficients come transposed (row r's weights
 // in the five rows r-2..r+2), wave-uniform through the scalar cache.
+//
+// D2 v has a sum of its own because its terms nearly cancel: with its weights merged
+// into those of the implicit part, which are rounded one by one, the right-hand side
+// was up to twice and v after the solve up to three times as far from a 64-bit
+// one (384 rows: 1.0e-15 for 3.3e-16).  The sum costs no time (191x384x189 1.10 ms,
+// 1.14 without it).
 //
 // A body force enters the same sums as it is formed from F = F0 + gain * V_src
 // (:643-659): D1(-i kx F_u - i kz F_w) and -k2 D0(F_v) in the D2v equation,
@@ -34,7 +40,7 @@
 // 63x96x47, 1.19 for 2.23 ms at 191x384x189.
 //
 // Bound by HBM and the memory-side cache on large grids: at 191x384x189 (FP64)
-// 1.13 ms with five product fields, 7.0 GB of counted traffic at 6.2 TB/s (1.21
+// 1.10 ms with five product fields, 7.0 GB of counted traffic at 6.3 TB/s (1.21
 // with six, where a five-row window of the nine fields in two waves per SIMD and
 // 48-row chunks took 1.39); by the length of the walk on small ones (31x64x31:
 // 11.3 us, 61 before).
@@ -102,9 +108,10 @@ __global__ __launch_bounds__(RHS_BLOCK) void k_rhs(RhsArgs<R> a, ForceArgs fa, c
   const size_t ps = g.ps, pstride = (size_t)g.Ny * ps;
   const bool mean = (ix == 0 && iz == 0);
   const int col = mean ? g.Nz : iz + g.nz;
-  // weights of the implicit v stencil: cA D2 + cB D0 + ni D4, and of eta: cC D0 + ni D2
+  // weights of the implicit v stencil: rdt D2, a sum of its own with the table's
+  // weights, and cA D2 + cB D0 + ni D4; of eta: cC D0 + ni D2
   const double rdt = a.ode0 / a.dt;
-  const double cA = rdt - 2.0 * a.ni * k2, cB = k2 * (a.ni * k2 - rdt), cC = rdt - a.ni * k2;
+  const double cA = -2.0 * a.ni * k2, cB = k2 * (a.ni * k2 - rdt), cC = rdt - a.ni * k2;
   const size_t rs = (size_t)(g.ny - 1) * ps;  // component stride of old/rhs
 
   // the row being read; all loads are unconditional, with the row clamped
@@ -134,9 +141,9 @@ __global__ __launch_bounds__(RHS_BLOCK) void k_rhs(RhsArgs<R> a, ForceArgs fa, c
   };
   // sums of the pending rows r-2..r+2 (slot m = row r-2+m): explicit and
   // implicit parts of the D2v (v) and eta (e) equations
-  cx<double> sev[5], siv[5], see[5], sie[5];
+  cx<double> sev[5], siv[5], sdv[5], see[5], sie[5];
 #pragma unroll
-  for (int m = 0; m < 5; m++) sev[m] = siv[m] = see[m] = sie[m] = cx<double>{0.0, 0.0};
+  for (int m = 0; m < 5; m++) sev[m] = siv[m] = sdv[m] = see[m] = sie[m] = cx<double>{0.0, 0.0};
   load(y0 - 2);
   for (int r = y0 - 2; r <= y1 + 2; r++) {
     const auto D = [](cx<R> v) { return cx<double>{(double)v.x, (double)v.y}; };
@@ -192,6 +199,8 @@ __global__ __launch_bounds__(RHS_BLOCK) void k_rhs(RhsArgs<R> a, ForceArgs fa, c
       }
       siv[m].x += wi * v.x;
       siv[m].y += wi * v.y;
+      sdv[m].x += d2 * v.x;
+      sdv[m].y += d2 * v.y;
       see[m].x += d0 * G3.x + d1 * G4.x;
       see[m].y += d0 * G3.y + d1 * G4.y;
       sie[m].x += wj * eta.x;
@@ -205,7 +214,7 @@ __global__ __launch_bounds__(RHS_BLOCK) void k_rhs(RhsArgs<R> a, ForceArgs fa, c
         ee.x += sc->meanpx;
         ee.y += sc->meanpz;
       }
-      cx<double> rv = {siv[0].x + a.ode1 * sev[0].x, siv[0].y + a.ode1 * sev[0].y};
+      cx<double> rv = {rdt * sdv[0].x + siv[0].x + a.ode1 * sev[0].x, rdt * sdv[0].y + siv[0].y + a.ode1 * sev[0].y};
       cx<double> re = {sie[0].x + a.ode1 * ee.x, sie[0].y + a.ode1 * ee.y};
       if constexpr (RD) {
         rv = sub(rv, scl(a.ode2, old_v));
@@ -222,10 +231,11 @@ __global__ __launch_bounds__(RHS_BLOCK) void k_rhs(RhsArgs<R> a, ForceArgs fa, c
     for (int m = 0; m < 4; m++) {
       sev[m] = sev[m + 1];
       siv[m] = siv[m + 1];
+      sdv[m] = sdv[m + 1];
       see[m] = see[m + 1];
       sie[m] = sie[m + 1];
     }
-    sev[4] = siv[4] = see[4] = sie[4] = cx<double>{0.0, 0.0};
+    sev[4] = siv[4] = sdv[4] = see[4] = sie[4] = cx<double>{0.0, 0.0};
   }
 }
 
