@@ -510,9 +510,9 @@ __global__ __launch_bounds__((xteams<M, R>() * fft::Plan<M>::T), 2) void k_xpass
 // mode split read their partners from LDS.
 //
 // Bound by the latency of its exchanges and barriers: three waves per SIMD in FP64
-// (33 spilled registers) take 2.04 ms at 191x384x189 (576 x 576 points, 5.5 GB),
-// two without spills 2.38; k_xpass on the 768 x 768 grid 2.49.  FP32 1.10 ms.  At
-// 95x128x95 (288 x 288 for 384 x 384) FP64 175 for 256 us, FP32 87 for 145.
+// (25 spilled registers) take 1.95 ms at 191x384x189 (576 x 576 points, 5.5 GB),
+// two without spills 2.38; k_xpass on the 768 x 768 grid 2.49.  FP32 0.99 ms.  At
+// 95x128x95 (288 x 288 for 384 x 384) FP64 166 for 256 us, FP32 87 for 145.
 template <int M>
 constexpr int xrows() {
   return 192 / fft::Plan<M>::T < ZB ? ZB : 192 / fft::Plan<M>::T;
