@@ -2,7 +2,7 @@
 // (linsolve, linsolve_blocking.inc:3-107).  Grids whose columns fit in LDS
 // (ny <= 130) take k_solve_lds and k_mean; the others three kernels:
 //
-//   k_solve_ve : one lane per (pair, system, real/imaginary part); system 0 =
+//   k_solve_ve (k_solve_ve_wide on wide grids) : one lane per (pair, system, real/imaginary part); system 0 =
 //                eta, 1 = v.  The pairs (kx, kz) and (kx, -kz) have the same
 //                k^2, hence the same matrix: their four lanes (sign x part)
 //                sit side by side and share one row of stored lower factors.
@@ -61,9 +61,10 @@ static unsigned xcd_grid(size_t lanes) {
 
 // One band: the pentadiagonal rows of etamat (SYS 0) or D2vmat (SYS 1) of a
 // wavenumber pair, with the wall conditions folded in: lambda D0 - SQ for eta,
-// lambda (D2 - k2 D0) - OS for v, each entry rounded as the reference forms it
-// (the v band's condition number reaches 1e6, so other groupings of the same
-// sums move the solution by 1e-12 of it).
+// lambda (D2 - k2 D0) - OS for v, each inner row's entry rounded as the reference forms
+// it (the v band's condition number reaches 1e6, so other groupings of the same
+// sums move the solution by 1e-12 of it); the wall columns are folded in by ratios
+// formed beforehand.
 struct Band {
   const double *bc0, *bc0m1, *bcn, *bcnp1;  // wall rows
   const WallRatios *q;                      // their ratios
@@ -76,9 +77,10 @@ struct Band {
         etan(etan), ny(a.g.ny) {}
 };
 
-// 1/a from the hardware's approximation and two Newton steps (relative error
-// below 2^-52): half the dependent operations of the division, which is the
-// longest link of the bottom-up sweep's chain.
+// 1/a from the hardware's approximation and two Newton steps: the correctly rounded
+// quotient but where the mantissa of a is one of the six largest (then one unit off in the
+// last place; compared with the division for 5e10 arguments), in half the dependent
+// operations of the division, which is the longest link of the bottom-up sweep's chain.
 __device__ __forceinline__ double recip(double a) {
   double r = __builtin_amdgcn_rcp(a);
   r = fma(fma(-a, r, 1.0), r, r);
@@ -312,6 +314,177 @@ __global__ __launch_bounds__(256, 5) void k_solve_ve(SolveArgs a, const double *
     solve_column<1>(a, der);
   else
     solve_column<0>(a, der);
+}
+
+// One body for both systems, each pivot a division: slower by itself, but on grids that
+// fill the memory system its waves stay closer together.  us per launch, this against
+// k_solve_ve: 191x384x189 1004 and 1052 (4.5 waves per SIMD), 255x192x255 835 and 876 (8),
+// 175x256x175 482 and 523 (3.8), 159x256x159 447 and 456 (3.1), but 143x256x143
+// 389 and 350 (2.5), 127x384x127 539 and 486 (2): it is taken from three waves per
+// SIMD on.  Its loops are its own: built from k_solve_ve's it took 1044.
+__global__ __launch_bounds__(256) void k_solve_ve_wide(SolveArgs a, const double *__restrict__ der) {
+  const Geom g = a.g;
+  const int gid = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
+  const int grp = gid >> 2, sgn = (gid >> 1) & 1, part = gid & 1;
+  const int ngrp = g.Nx * (g.nz + 1);
+  if (grp > ngrp) return;
+  const bool spare = grp == ngrp;
+  const int ix = spare ? 0 : grp / (g.nz + 1), iza = spare ? 0 : grp % (g.nz + 1);
+  if (sgn && (spare || iza == 0)) return;  // kz = 0 has no mirror
+  const int iz = sgn ? -iza : iza;
+  const int p = spare ? g.npair : ix * g.Nz + g.nz + iz;
+  const int sys = blockIdx.y;  // 0: eta (component 1), 1: v (component 2)
+  const int ny = g.ny;
+  const size_t gs = ((size_t)ngrp + 1 + 63) / 64 * 64;  // group stride of L
+  const double k2 = (g.alfa0 * ix) * (g.alfa0 * ix) + (g.beta0 * iz) * (g.beta0 * iz);
+  const bool mean = !spare && ix == 0 && iz == 0;
+  const size_t ps = g.ps, rs = 2 * ps;  // row stride in doubles
+  double *col = reinterpret_cast<double *>(a.V + (size_t)sys * g.Ny * ps + p) + part;  // row iy at col[(iy+1)*rs]
+  const double *rc = reinterpret_cast<const double *>(a.rhs + (size_t)sys * (ny - 1) * ps + p) + part;
+  double2 *Lc = a.L + (size_t)sys * (ny - 1) * gs + grp;  // row iy at Lc[(iy-1)*gs]
+  const double *bc0 = a.bc[sys ? BC_V0 : BC_ETA0], *bc0m1 = a.bc[sys ? BC_V0M1 : BC_ETA0M1];
+  const double *bcn = a.bc[sys ? BC_VN : BC_ETAN], *bcnp1 = a.bc[sys ? BC_VNP1 : BC_ETANP1];
+  const double eta0 = (mean && sys == 0 && part == 0) ? a.u0 : 0.0;
+  const double etan = (mean && sys == 0 && part == 0) ? a.uN : 0.0;
+  const double bspare = (sys == 0 && part == 0) ? 1.0 : 0.0;  // ucor right-hand side
+
+  // ---- bottom-up: rows, wall folding, factorisation, backward sweep
+  double l1m2 = 0.0, l1m1 = 0.0, l2m2 = 0.0, l2m1 = 0.0;  // lower factors of rows iy+1, iy+2
+  double x1 = 0.0, x2 = 0.0;
+  auto up_row = [&](const int iy, double b) {
+    if (spare) b = bspare;
+    const double *d = der + (size_t)(iy - 1) * 20;
+    double A[5];
+#pragma unroll
+    for (int j = 0; j < 5; j++) {
+      const double d0 = d[j], d2 = d[10 + j], d4 = d[15 + j];
+      if (sys) {
+        const double os = a.ni * (d4 - 2.0 * k2 * d2 + k2 * k2 * d0);
+        A[j] = a.lambda * (d2 - k2 * d0) - os;
+      } else {
+        const double sq = a.ni * (d2 - k2 * d0);
+        A[j] = a.lambda * d0 - sq;
+      }
+    }
+    if (iy == 1) {  // applybc_0 row 1: ghost then wall column
+      const double e = A[0];
+      for (int j = 1; j <= 4; j++) A[j] = A[j] - e * bc0m1[j] / bc0m1[0];
+      const double f = A[1];
+      for (int j = 2; j <= 4; j++) A[j] = A[j] - f * bc0[j] / bc0[1];
+      if (sys == 0) b = b - A[1] * eta0 / bc0[1];
+    } else if (iy == 2) {
+      if (sys == 0) b = b - A[0] * eta0 / bc0[1];
+      const double e = A[0];
+      for (int j = 1; j <= 3; j++) A[j] = A[j] - e * bc0[j + 1] / bc0[1];
+    }
+    if (iy == ny - 1) {  // applybc_n row ny-1
+      const double e = A[4];
+      for (int j = 0; j <= 3; j++) A[j] = A[j] - e * bcnp1[j] / bcnp1[4];
+      const double f = A[3];
+      for (int j = 0; j <= 2; j++) A[j] = A[j] - f * bcn[j] / bcn[3];
+      if (sys == 0) b = b - A[3] * etan / bcn[3];
+      A[3] = 0.0;
+      A[4] = 0.0;
+    } else if (iy == ny - 2) {
+      if (sys == 0) b = b - A[4] * etan / bcn[3];
+      const double e = A[4];
+      for (int j = 1; j <= 3; j++) A[j] = A[j] - e * bcn[j - 1] / bcn[3];
+      A[4] = 0.0;
+    }
+    // factorise row iy against the already factorised rows iy+1, iy+2
+    const double p2 = A[4];
+    A[3] = A[3] - p2 * l2m1;
+    A[2] = A[2] - p2 * l2m2;
+    const double p1 = A[3];
+    A[2] = A[2] - p1 * l1m1;
+    A[1] = A[1] - p1 * l1m2;
+    const double r = 1.0 / A[2];
+    A[0] = A[0] * r;
+    A[1] = A[1] * r;
+    // backward sweep
+    const double xi = (b - (p1 * x1 + p2 * x2)) * r;
+    col[(size_t)(iy + 1) * rs] = xi;
+    Lc[(size_t)(iy - 1) * gs] = make_double2(iy <= 2 ? 0.0 : A[0], iy == 1 ? 0.0 : A[1]);
+    l2m2 = l1m2;
+    l2m1 = l1m1;
+    l1m2 = A[0];
+    l1m1 = A[1];
+    x2 = x1;
+    x1 = xi;
+  };
+  {
+    double ring[PF];  // ring[u] holds the right-hand side of row iy-u
+#pragma unroll
+    for (int u = 0; u < PF; u++) ring[u] = rc[(size_t)max(ny - 2 - u, 0) * rs];
+    int iy = ny - 1;
+    for (; iy - (PF - 1) >= 1; iy -= PF) {
+#pragma unroll
+      for (int u = 0; u < PF; u++) {
+        const int r = iy - u;
+        const double b = ring[u];
+        ring[u] = rc[(size_t)max(r - PF - 1, 0) * rs];
+        up_row(r, b);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < PF; u++)
+      if (iy - u >= 1) up_row(iy - u, ring[u]);
+  }
+
+  // ---- top-down: forward sweep, keep rows 1..3 and ny-3..ny-1
+  double b1 = 0.0, b2 = 0.0, b3 = 0.0;
+  double bot[3] = {0.0, 0.0, 0.0};
+  auto down_row = [&](const int iy, const double x, const double2 L) {
+    const double bi = x - (L.x * b2 + L.y * b1);
+    col[(size_t)(iy + 1) * rs] = bi;
+    if (iy <= 3) bot[iy - 1] = bi;
+    b3 = b2;
+    b2 = b1;
+    b1 = bi;
+  };
+  {
+    double xr[PF];
+    double2 lr[PF];
+#pragma unroll
+    for (int u = 0; u < PF; u++) {
+      const int r = min(1 + u, ny - 1);
+      xr[u] = col[(size_t)(r + 1) * rs];
+      lr[u] = Lc[(size_t)(r - 1) * gs];
+    }
+    int iy = 1;
+    for (; iy + (PF - 1) <= ny - 1; iy += PF) {
+#pragma unroll
+      for (int u = 0; u < PF; u++) {
+        const int r = iy + u;
+        const double x = xr[u];
+        const double2 L = lr[u];
+        const int nr = min(r + PF, ny - 1);
+        xr[u] = col[(size_t)(nr + 1) * rs];
+        lr[u] = Lc[(size_t)(nr - 1) * gs];
+        down_row(r, x, L);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < PF; u++)
+      if (iy + u <= ny - 1) down_row(iy + u, xr[u], lr[u]);
+  }
+  // wall and ghost rows
+  {
+    const double s0 = bc0[2] * bot[0] + bc0[3] * bot[1] + bc0[4] * bot[2];
+    const double w0 = (eta0 - s0) / bc0[1];
+    const double s1 = bc0m1[1] * w0 + bc0m1[2] * bot[0] + bc0m1[3] * bot[1] + bc0m1[4] * bot[2];
+    const double wm1 = sys ? (0.0 - s1) / bc0m1[0] : -(s1 / bc0m1[0]);
+    col[rs] = w0;
+    col[0] = wm1;
+  }
+  {
+    const double s0 = bcn[0] * b3 + bcn[1] * b2 + bcn[2] * b1;  // rows ny-3, ny-2, ny-1
+    const double wn = (etan - s0) / bcn[3];
+    const double s1 = bcnp1[0] * b3 + bcnp1[1] * b2 + bcnp1[2] * b1 + bcnp1[3] * wn;
+    const double wp1 = sys ? (0.0 - s1) / bcnp1[4] : -(s1 / bcnp1[4]);
+    col[(size_t)(ny + 1) * rs] = wn;
+    col[(size_t)(ny + 2) * rs] = wp1;
+  }
 }
 
 // ---------------------------------------------------------------- k_mean --
@@ -971,7 +1144,10 @@ hipError_t launch_solve_lds(hipStream_t st, const SolveArgs &a, const UwArgs &u)
 hipError_t launch_solve(hipStream_t st, const SolveArgs &a) {
   const size_t lanes = (size_t)4 * (a.g.Nx * (a.g.nz + 1) + 1);
   dim3 grid(xcd_grid(lanes), 2);
-  hipLaunchKernelGGL(k_solve_ve, grid, dim3(256), 0, st, a, a.der);
+  if (2 * lanes >= (size_t)12 * 64 * a.g.ncu)  // k_solve_ve_wide
+    hipLaunchKernelGGL(k_solve_ve_wide, grid, dim3(256), 0, st, a, a.der);
+  else
+    hipLaunchKernelGGL(k_solve_ve, grid, dim3(256), 0, st, a, a.der);
   return hipGetLastError();
 }
 hipError_t launch_mean(hipStream_t st, const MeanArgs &a) {
