@@ -274,6 +274,31 @@ int dalloc(T **p, size_t n) {
   return 0;
 }
 
+// A context's small device arrays in one allocation, brought there by one copy: with
+// one of each per array, chan_create took 95 us longer at 15x32x15 and 310 at 95x128x95.
+struct Tables {
+  std::vector<char> image;
+  std::vector<std::pair<void **, size_t>> wanted;  // whom to tell where an array came to lie
+  template <class T>
+  size_t add(const T *src, size_t n) {
+    const size_t at = image.size();
+    image.resize((at + n * sizeof(T) + 255) / 256 * 256);
+    std::memcpy(image.data() + at, src, n * sizeof(T));
+    return at;
+  }
+  template <class T>
+  size_t add(const std::vector<T> &v) {
+    return add(v.data(), v.size());
+  }
+  template <class T>
+  void want(T **p, size_t at) {
+    wanted.push_back({(void **)p, at});
+  }
+  void place(char *base) {
+    for (auto &w : wanted) *w.first = base + w.second;
+  }
+};
+
 ForceArgs force_args(const chan_ctx *c) {
   ForceArgs a;
   a.V = c->V;
@@ -363,7 +388,8 @@ int chan_create(const chan_params *p, chan_ctx **out) {
   const size_t slab = (size_t)g.nzd * g.Nx;  // one component of one plane in physical z
   if ((rc = dalloc(&c->V, 3 * NyP))) return bail(rc);
   if ((rc = dalloc(&c->rhs, 2 * (size_t)(g.ny - 1) * plane))) return bail(rc);
-  if ((rc = dalloc(&c->L, 2 * (size_t)(g.ny - 1) * plane))) return bail(rc);
+  const size_t factors = solve_factors(g);
+  if (factors && (rc = dalloc(&c->L, factors))) return bail(rc);
   if (hipHostMalloc(&c->step_row, sizeof(StepRow), hipHostMallocDefault) != hipSuccess)
     return bail(fail(CHAN_E_STATE, "hipHostMalloc failed"));
   const size_t esz = c->split ? sizeof(cx<float>) : sizeof(cx<double>);
@@ -374,42 +400,38 @@ int chan_create(const chan_params *p, chan_ctx **out) {
   if ((rc = dalloc_bytes(&c->A, 3 * (size_t)g.Ny * slab * esz))) return bail(rc);
   if ((rc = dalloc_bytes(&c->B, NPROD * (size_t)g.Ny * slab * esz))) return bail(rc);
   if ((rc = dalloc_bytes(&c->P, NyP * (NPROD * esz > 48 ? NPROD * esz : 48)))) return bail(rc);
-  if ((rc = dalloc_bytes(&c->twz, (size_t)fft::tw_table_size(g.nzd) * esz))) return bail(rc);
-  if ((rc = dalloc_bytes(&c->twx, (size_t)fft::tw_table_size(2 * g.nxd) * esz))) return bail(rc);
   // no mode that is kept may alias: more than 3 nz points in z; 3 (nx + 1) in x,
   // which the x pass's slots need
   c->nzs = alias_free_size(3 * g.nz + 1, g.nzd);
   c->mxs = alias_free_size(3 * g.Nx, 2 * g.nxd);
-  if ((rc = dalloc_bytes(&c->twzs, (size_t)fft::tw_table_size(c->nzs) * esz)) ||
-      (rc = dalloc_bytes(&c->twxs, (size_t)fft::tw_table_size(c->mxs) * esz)))
-    return bail(rc);
-  if ((rc = dalloc(&c->der, (size_t)(g.ny - 1) * 20))) return bail(rc);
-  if ((rc = dalloc(&c->derT, (size_t)g.Ny * 20)) || (rc = dalloc(&c->derF, (size_t)g.Ny * 10)) ||
-      (rc = dalloc(&c->tab, (size_t)(g.ny - 1) * SROW))) return bail(rc);
-  if ((rc = dalloc(&c->d0fac, (size_t)(g.ny + 1) * 5))) return bail(rc);
-  if ((rc = dalloc(&c->y, (size_t)g.Ny))) return bail(rc);
-  if ((rc = dalloc(&c->dy, (size_t)g.ny + 1))) return bail(rc);
-  if ((rc = dalloc(&c->sc, 1)) || (rc = dalloc(&c->cfl_max, CFL_SLOTS * CFL_STRIDE))) return bail(rc);
-  if ((rc = dalloc(&c->stat, (size_t)10 * (g.ny + 1)))) return bail(rc);
-
-  auto upload_tw = [&](auto proto) {
-    std::vector<decltype(proto)> tw;
-    twiddles(tw, g.nzd);
-    if (hipMemcpy(c->twz, tw.data(), tw.size() * sizeof(tw[0]), hipMemcpyHostToDevice) != hipSuccess) return 1;
-    twiddles_x(tw, 2 * g.nxd);
-    if (hipMemcpy(c->twx, tw.data(), tw.size() * sizeof(tw[0]), hipMemcpyHostToDevice) != hipSuccess) return 1;
-    twiddles(tw, c->nzs);
-    if (hipMemcpy(c->twzs, tw.data(), tw.size() * sizeof(tw[0]), hipMemcpyHostToDevice) != hipSuccess) return 1;
-    twiddles_x(tw, c->mxs);
-    if (hipMemcpy(c->twxs, tw.data(), tw.size() * sizeof(tw[0]), hipMemcpyHostToDevice) != hipSuccess) return 1;
-    return 0;
+  Tables tb;
+  auto twiddle_tables = [&](auto proto) {
+    typedef decltype(proto) W;
+    std::vector<W> tw;
+    auto z = [&](int n) {
+      twiddles(tw, n);
+      return tb.add(tw);
+    };
+    auto x = [&](int n) {
+      twiddles_x(tw, n);
+      return tb.add(tw);
+    };
+    const size_t tz = z(g.nzd), tx = x(2 * g.nxd);
+    const size_t tzs = c->nzs == g.nzd ? tz : z(c->nzs);
+    const size_t txs = c->mxs == 2 * g.nxd ? tx : (c->mxs == c->nzs ? tzs : x(c->mxs));  // 9*2^k: one table
+    tb.want(&c->twz, tz);
+    tb.want(&c->twx, tx);
+    tb.want(&c->twzs, tzs);
+    tb.want(&c->twxs, txs);
   };
-  if (c->split ? upload_tw(cx<float>{}) : upload_tw(cx<double>{})) return bail(fail(CHAN_E_STATE, "upload failed"));
-  if (hipMemcpy(c->der, h.der, sizeof(double) * 20 * (g.ny - 1), hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(c->d0fac, h.d0fac, sizeof(double) * 5 * (g.ny + 1), hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(c->y, h.y, sizeof(double) * g.Ny, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(c->dy, h.dy, sizeof(double) * (g.ny + 1), hipMemcpyHostToDevice) != hipSuccess)
-    return bail(fail(CHAN_E_STATE, "upload of the set-up failed"));
+  if (c->split)
+    twiddle_tables(cx<float>{});
+  else
+    twiddle_tables(cx<double>{});
+  tb.want(&c->der, tb.add(h.der, (size_t)20 * (g.ny - 1)));
+  tb.want(&c->d0fac, tb.add(h.d0fac, (size_t)5 * (g.ny + 1)));
+  tb.want(&c->y, tb.add(h.y, (size_t)g.Ny));
+  tb.want(&c->dy, tb.add(h.dy, (size_t)g.ny + 1));
   {
     // row r's weights in the stencils of the interior rows r-2..r+2; those of
     // a body force have its wall rows folded in: F(0) = F(ny) = 0, and the
@@ -430,20 +452,24 @@ int chan_create(const chan_params *p, chan_ctx **out) {
           tf[(size_t)(r + 1) * 10 + 2 * m + f] = w;
         }
       }
-    std::vector<double> tb;
-    solve_table(h, g.ny, tb);
-    if (hipMemcpy(c->tab, tb.data(), tb.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(c->derT, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(c->derF, tf.data(), tf.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
-      return bail(fail(CHAN_E_STATE, "upload of the set-up failed"));
+    tb.want(&c->derT, tb.add(t));
+    tb.want(&c->derF, tb.add(tf));
+    if (solve_in_lds(g)) {
+      solve_table(h, g.ny, t);
+      tb.want(&c->tab, tb.add(t));
+    }
   }
   DevScalars s0;
   std::memset(&s0, 0, sizeof s0);
   s0.meanpx = p->meanpx;
   s0.meanpz = p->meanpz;
-  if (hipMemcpy(c->sc, &s0, sizeof s0, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemset(c->cfl_max, 0, sizeof(unsigned long long) * CFL_SLOTS * CFL_STRIDE) != hipSuccess)
-    return bail(fail(CHAN_E_STATE, "upload failed"));
+  tb.want(&c->sc, tb.add(&s0, 1));
+  tb.want(&c->cfl_max, tb.add(std::vector<unsigned long long>(CFL_SLOTS * CFL_STRIDE)));
+  tb.want(&c->stat, tb.add(std::vector<double>((size_t)10 * (g.ny + 1))));
+  if ((rc = dalloc_bytes((void **)&c->tables, tb.image.size()))) return bail(rc);
+  if (hipMemcpy(c->tables, tb.image.data(), tb.image.size(), hipMemcpyHostToDevice) != hipSuccess)
+    return bail(fail(CHAN_E_STATE, "upload of the set-up failed"));
+  tb.place(c->tables);
   // stored explicit terms start at zero (ODE3 = 0 in the first substep)
   if (hipMemset(c->old, 0, esz * 2 * (g.ny - 1) * plane) != hipSuccess ||
       hipMemset(c->V, 0, sizeof(cx<double>) * 3 * NyP) != hipSuccess)
@@ -463,8 +489,7 @@ int chan_destroy(chan_ctx *c) {
     hipEventDestroy(r.b);
   }
   for (auto e : c->pool) hipEventDestroy(e);
-  void *bufs[] = {c->V, c->old, c->rhs, c->L, c->A, c->B, c->P, c->twz, c->twx, c->twzs, c->twxs,
-                  c->der, c->derT, c->derF, c->tab, c->d0fac, c->y, c->dy, c->sc, c->cfl_max, c->stat, c->F0, c->gain, c->Fkeep};
+  void *bufs[] = {c->V, c->old, c->rhs, c->L, c->A, c->B, c->P, c->tables, c->F0, c->gain, c->Fkeep};
   for (void *b : bufs)
     if (b) hipFree(b);
   if (c->st) hipStreamDestroy(c->st);

@@ -91,7 +91,7 @@ struct SolveArgs {
                            // slot npair of component 1 the ucor response
   const cx<double> *rhs;   // [2][ny-1][ps]
   double2 *L;              // [2][ny-1][gs] lower factors of the UL decomposition, one
-                           // row per (kx, |kz|) group, gs <= ps
+                           // column per (kx, |kz|) group, gs <= ps; null where solve_factors is 0
   const double *der;
   double bc[8][5];
   WallRatios wall[2];  // of eta, v
@@ -116,7 +116,7 @@ constexpr int SROW = 26;
 
 struct UwArgs {
   cx<double> *V;
-  const double *tab;  // [ny-1][SROW]
+  const double *tab;  // [ny-1][SROW]; only where solve_in_lds
   const double *der;
   const double *d0fac;
   double bnd[10][5];
@@ -149,6 +149,7 @@ hipError_t launch_force(hipStream_t st, const ForceArgs &a);
 hipError_t launch_stats(hipStream_t st, const cx<double> *V, const double *avg, double *out, const Geom &g);
 hipError_t launch_solve(hipStream_t st, const SolveArgs &a);
 bool solve_in_lds(const Geom &g);  // whether launch_solve_lds serves the grid, in place of launch_solve and launch_uw
+size_t solve_factors(const Geom &g);  // elements of SolveArgs::L that the solve needs
 hipError_t launch_solve_lds(hipStream_t st, const SolveArgs &a, const UwArgs &u);
 hipError_t launch_mean(hipStream_t st, const MeanArgs &a);
 hipError_t launch_uw(hipStream_t st, const UwArgs &a);

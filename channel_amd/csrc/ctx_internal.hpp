@@ -20,6 +20,7 @@ struct chan_ctx {
   chan::Geom g;
   hipStream_t st = nullptr;
   // device state
+  char *tables = nullptr;  // holds the small arrays: twiddles, stencils, scalars
   chan::cx<double> *V = nullptr, *rhs = nullptr;
   void *step_row = nullptr;  // pinned: what a step's end reads on the host
   void *old = nullptr;  // explicit terms: complex FP64, or FP32 in the split mode

@@ -55,6 +55,8 @@ constexpr int PF = 4;  // rows of software prefetch in the sequential sweeps
 __device__ __forceinline__ int xcd_block(int b, int nb) {
   return (b & 7) * (nb >> 3) + (b >> 3);
 }
+// elements per row of the lower factors: a group each, and ucor's
+__host__ __device__ __forceinline__ size_t group_stride(int ngrp) { return ((size_t)ngrp + 1 + 63) / 64 * 64; }
 static unsigned xcd_grid(size_t lanes) {
   return (unsigned)(((lanes + 255) / 256 + 7) / 8 * 8);
 }
@@ -235,7 +237,7 @@ __device__ __forceinline__ void solve_column(const SolveArgs &a, const double *_
   const int p = spare ? g.npair : ix * g.Nz + g.nz + iz;
   constexpr int sys = SYS;  // 0: eta (component 1), 1: v (component 2)
   const int ny = g.ny;
-  const size_t gs = ((size_t)ngrp + 1 + 63) / 64 * 64;  // group stride of L
+  const size_t gs = group_stride(ngrp);
   const double k2 = (g.alfa0 * ix) * (g.alfa0 * ix) + (g.beta0 * iz) * (g.beta0 * iz);
   const bool mean = !spare && ix == 0 && iz == 0;
   const size_t ps = g.ps, rs = 2 * ps;  // row stride in doubles
@@ -335,7 +337,7 @@ __global__ __launch_bounds__(256) void k_solve_ve_wide(SolveArgs a, const double
   const int p = spare ? g.npair : ix * g.Nz + g.nz + iz;
   const int sys = blockIdx.y;  // 0: eta (component 1), 1: v (component 2)
   const int ny = g.ny;
-  const size_t gs = ((size_t)ngrp + 1 + 63) / 64 * 64;  // group stride of L
+  const size_t gs = group_stride(ngrp);
   const double k2 = (g.alfa0 * ix) * (g.alfa0 * ix) + (g.beta0 * iz) * (g.beta0 * iz);
   const bool mean = !spare && ix == 0 && iz == 0;
   const size_t ps = g.ps, rs = 2 * ps;  // row stride in doubles
@@ -1036,7 +1038,7 @@ __global__ __launch_bounds__(256) void k_solve_lds(SolveArgs a, UwArgs uw, const
   const int ix = spare ? 0 : grp / (g.nz + 1), iza = spare ? 0 : grp % (g.nz + 1);
   const int iz = sgn ? -iza : iza;
   const int p = spare ? g.npair : ix * g.Nz + g.nz + iz;
-  const size_t gs = ((size_t)ngrp + 1 + 63) / 64 * 64;
+  const size_t gs = group_stride(ngrp);
   const double k2 = (g.alfa0 * ix) * (g.alfa0 * ix) + (g.beta0 * iz) * (g.beta0 * iz);
   const bool mean = !spare && ix == 0 && iz == 0;
   const size_t ps = g.ps, rs = 2 * ps;
@@ -1127,6 +1129,11 @@ constexpr size_t LDS_MAX = 160 * 1024;
 // (3.7x at 31x64x31, 1.3x at 191x128x189, nine rounds of blocks) but stays.
 bool solve_in_lds(const Geom &g) {
   return solve_lds_columns(g) <= LDS_MAX;
+}
+
+size_t solve_factors(const Geom &g) {
+  if (solve_lds_columns(g) + solve_lds_factors(g) <= LDS_MAX) return 0;
+  return (size_t)2 * (g.ny - 1) * group_stride(g.Nx * (g.nz + 1));
 }
 
 hipError_t launch_solve_lds(hipStream_t st, const SolveArgs &a, const UwArgs &u) {
