@@ -39,7 +39,7 @@ struct DevScalars {
   double pad[8];
 };
 // The x pass's blocks take their CFL maxima to CFL_SLOTS places on cache lines of
-// their own, which k_step_row and k_fold_cfl then take to cfl_bits: atomics on one
+// their own, which k_step_row then takes to cfl_bits: atomics on one
 // place run one after another, 5 ns each (31x64x31, 1608 blocks: 20.4 for 28.2 us).
 constexpr int CFL_SLOTS = 64, CFL_STRIDE = 16;
 
