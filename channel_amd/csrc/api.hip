@@ -406,8 +406,8 @@ int chan_create(const chan_params *p, chan_ctx **out) {
   if ((rc = dalloc_bytes(&c->P, NyP * (NPROD * esz > 48 ? NPROD * esz : 48)))) return bail(rc);
   // no mode that is kept may alias: more than 3 nz points in z; 3 (nx + 1) in x,
   // which the x pass's slots need
-  c->nzs = alias_free_size(3 * g.nz + 1, g.nzd);
-  c->mxs = alias_free_size(3 * g.Nx, 2 * g.nxd);
+  c->nzs = alias_free_z(3 * g.nz + 1, g.nzd);
+  c->mxs = alias_free_x(3 * g.Nx, 2 * g.nxd, (unsigned)(c->nzs / ZB * g.Ny), g.ncu, c->split);
   Tables tb;
   auto twiddle_tables = [&](auto proto) {
     typedef decltype(proto) W;

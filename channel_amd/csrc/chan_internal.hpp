@@ -128,7 +128,8 @@ int set_error(int code, const char *fmt, ...);
 
 // ----------------------------------------------------------- launchers --
 int fft_size_supported(int N);
-int alias_free_size(int need, int below);
+int alias_free_z(int need, int below);
+int alias_free_x(int need, int below, unsigned tiles, int ncu, bool fp32);
 template <typename R>
 hipError_t launch_zinv(int NZ, hipStream_t st, const cx<double> *V, cx<R> *A, const cx<R> *tw, const Geom &g, int plane0,
                        int nplanes);

@@ -315,7 +315,7 @@ __device__ __forceinline__ void run_pass(cx<R> (&v)[Plan<N>::E], R *lds, const c
         // Three entries for eleven powers, each of the others (but the tenth) one
         // product away, in the order that keeps fewest of them alive.  From one entry,
         // in up to four products, the FP32 modes of 144- to 576-point grids were 2.3 to
-        // 2.7 times as far from FP64's, and rows of 576 took 2.03 ms instead of 1.95.
+        // 2.7 times as far from FP64's, and rows of 288 took 176 us instead of 166.
         cx<R> *x = &v[m * RAD], w3 = tw[PL::tw_base(P) + NS + k], w8 = tw[PL::tw_base(P) + 2 * NS + k];
         if constexpr (S > 0) {
           w3.y = -w3.y;

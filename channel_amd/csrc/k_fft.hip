@@ -18,8 +18,9 @@
 // Grids.  The physical grid is the reference's (fftFIT, sizes 2^k and 3*2^k) where
 // the CFL maximum is taken over its points.  The kept modes of the products are
 // the same sums on every grid of more than 3 nz points in z and 3 nx in x, so
-// where no CFL is asked for, the smallest supported size that large is used:
-// 9*2^k where it is smaller than fftFIT's (576 for 768, 288 for 384, 144 for 192).
+// where no CFL is asked for, the smallest supported size that large is used in z:
+// 9*2^k where it is smaller than fftFIT's (576 for 768, 288 for 384, 144 for 192).  In x
+// only where rows of that length are the faster ones (alias_free_x).
 //
 // The reference's pencil transposes (zTOx / xTOz, mpi_transpose.f90:50-117)
 // are the layout changes between K1/K2 and K2/K3: both sides move ZB*16
@@ -502,17 +503,17 @@ __global__ __launch_bounds__((xteams<M, R>() * fft::Plan<M>::T), 2) void k_xpass
 }
 
 // ------------------------------------------------------------ K2, 9*2^k --
-// The x pass of the 9*2^k grids (no CFL): a block of 192 threads holds RW rows in
-// teams of T = M/12 lanes, which straddle the wavefronts, so that the block
+// The x pass of rows of 72, 144 and 288 points (no CFL): a block of 192 threads holds RW
+// rows in teams of T = M/12 lanes, which straddle the wavefronts, so that the block
 // synchronises as a whole; four rows are a z block.  As it does so anyway, it
 // moves its global data through the teams' exchange areas: thread (mode, row) of
 // a whole run reads and writes contiguous memory, the Hermitian extension and the
 // mode split read their partners from LDS.
 //
-// Bound by the latency of its exchanges and barriers: three waves per SIMD in FP64
-// (25 spilled registers) take 1.95 ms at 191x384x189 (576 x 576 points, 5.5 GB),
-// two without spills 2.38; k_xpass on the 768 x 768 grid 2.49.  FP32 0.99 ms.  At
-// 95x128x95 (288 x 288 for 384 x 384) FP64 166 for 256 us, FP32 87 for 145.
+// Bound by the latency of its exchanges and barriers, at three waves per SIMD in FP64 (14
+// spilled registers at 288 points).  us, against k_xpass on rows of 384 and 192 points
+// of the same z grid: 95x128x95 166 for 188, 47x128x95 66 for 80; FP32 88 for 100,
+// 40 for 42.
 template <int M>
 constexpr int xrows() {
   return 192 / fft::Plan<M>::T < ZB ? ZB : 192 / fft::Plan<M>::T;
@@ -894,7 +895,8 @@ hipError_t launch_fft_bench(int N, int sign, int variant, const cx<double> *in, 
 }
 
 // ------------------------------------------------------------ launchers --
-#define CHAN_FOR_NINES(X) X(36) X(72) X(144) X(288) X(576) X(1152)
+#define CHAN_FOR_NINES_X(X) X(36) X(72) X(144) X(288)
+#define CHAN_FOR_NINES(X) CHAN_FOR_NINES_X(X) X(576) X(1152)
 #define CHAN_FOR_SIZES(X) X(12) X(24) X(48) X(96) X(192) X(384) X(768) X(1536) X(16) X(32) X(64) X(128) X(256) X(512) X(1024)
 
 #define CHAN_FOR_FEW(X) X(12) X(24) X(48) X(96) X(16) X(32) X(64) X(128) X(36) X(72)
@@ -980,7 +982,7 @@ hipError_t launch_xpass(int M, hipStream_t st, const cx<R> *A, cx<R> *B, const c
                          st, A, B, tw, g, factor, nplanes);                                                           \
     return hipGetLastError();                                                                                         \
   }
-    CHAN_FOR_NINES(X)
+    CHAN_FOR_NINES_X(X)
 #undef X
   }
   return hipErrorInvalidValue;
@@ -1023,10 +1025,27 @@ hipError_t launch_fft_test(int N, int sign, hipStream_t st, cx<double> *data, co
 }
 
 // the smallest size of the form 9*2^k in [need, below), or `below` when none is
-int alias_free_size(int need, int below) {
+int alias_free_z(int need, int below) {
 #define X(N) \
   if (N >= need && N < below) return N;
   CHAN_FOR_NINES(X)
+#undef X
+  return below;
+}
+// The same for the rows of the x pass, of which there are `tiles` groups of ZB.  Rows of
+// 576 and 1152 points lose to k_xpass's four-step rows of 768 and 1536 (us, same z
+// grid: 191x384x189 1972 and 1687, FP32 994 and 822, 191x48x47 72 and 66, 383x48x95 438 and
+// 328).  Rows of 144 and 288 need tiles enough for their larger blocks: four per CU
+// (95x16x11, 171 tiles, 20.6 and 16.0; 95x24x23, 486, 21.8 and 21.6; 95x24x47, 972, 27.2
+// and 28.8; 47x40x23, 774, 17.4 and 17.0; 47x40x47, 1548, 20.8 and 23.4), rows of 144 in FP32
+// eight (1548 tiles 16.1 and 15.6, 2412 19.2 and 19.4).  Shorter rows have k_xpass_few.
+int alias_free_x(int need, int below, unsigned tiles, int ncu, bool fp32) {
+#define X(N)                                                                              \
+  if (N >= need && N < below) {                                                           \
+    const unsigned per_cu = N < 144 ? 0 : (N == 144 && fp32 ? 8 : 4);                     \
+    return tiles >= per_cu * (unsigned)ncu ? N : below;                                   \
+  }
+  CHAN_FOR_NINES_X(X)
 #undef X
   return below;
 }
