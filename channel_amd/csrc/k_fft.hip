@@ -39,21 +39,12 @@ constexpr int ZXCH = fft::XCH_PAD;
 // transactions: the z kernels stage through LDS, where the G x modes of a
 // block form one contiguous run of G*ZB values per z block, and lanes move
 // whole runs (a wave touches 4 runs of 128 or 256 bytes).
-template <int NZ, typename R>
-constexpr bool z_staged() {
-  return true;
-}
 // team stride of the staging area (a 32-byte shift per team keeps the
 // staged writes and reads free of LDS bank conflicts)
 template <int NZ>
 constexpr int stage_stride() {
   return NZ + 4;
 }
-// The blocks stage the real and the imaginary parts in two rounds through
-// one real-valued area: half the LDS of whole complex values, which would
-// hold an FP64 block to three waves per SIMD and an FP32 block to six (four
-// and eight with the two rounds: the FP64 step 1.5% and the FP32 z kernels
-// 4-9% faster)
 // x modes per block of the z kernels, and its threads: 256, or 192 where the team
 // size is 3*2^k (N = 9*2^k)
 template <int NZ>
@@ -64,11 +55,16 @@ template <int NZ>
 constexpr int zthreads() {
   return zteams<NZ>() * fft::Plan<NZ>::T;
 }
-template <int NZ, typename R>
+// The blocks stage the real and the imaginary parts in two rounds through
+// one real-valued area: half the LDS of whole complex values, which would
+// hold an FP64 block to three waves per SIMD and an FP32 block to six (four
+// and eight with the two rounds: the FP64 step 1.5% and the FP32 z kernels
+// 4-9% faster)
+template <int NZ>
 constexpr int zbuf_reals() {
   constexpr int G = zteams<NZ>();
   constexpr int fftr = G * fft::lds_reals<NZ, ZXCH>();
-  constexpr int stg = z_staged<NZ, R>() ? G * stage_stride<NZ>() : 0;
+  constexpr int stg = G * stage_stride<NZ>();
   return fftr > stg ? fftr : stg;
 }
 
@@ -77,7 +73,7 @@ __global__ __launch_bounds__(zthreads<NZ>()) void k_zinv(const cx<double> *__res
                                               const cx<R> *__restrict__ tw, Geom g, int plane0) {
   using PL = fft::Plan<NZ>;
   constexpr int T = PL::T, E = PL::E, G = zteams<NZ>(), NT = zthreads<NZ>(), SP = stage_stride<NZ>();
-  __shared__ __align__(16) R lds[zbuf_reals<NZ, R>()];
+  __shared__ __align__(16) R lds[zbuf_reals<NZ>()];
   const int team = threadIdx.x / T, t = threadIdx.x % T;
   const int nxg = (g.Nx + G - 1) / G;
   int b = blockIdx.x;
@@ -98,34 +94,26 @@ __global__ __launch_bounds__(zthreads<NZ>()) void k_zinv(const cx<double> *__res
   }
   fft::fft_slots<NZ, +1, true, ZXCH>(e, lds + team * fft::lds_reals<NZ, ZXCH>(), tw, t);
   cx<R> *dst = A + (size_t)(pl * 3 + c) * NZ * g.Nx;
-  if constexpr (z_staged<NZ, R>()) {
-    const int ix0 = xg * G, nact = min(G, g.Nx - ix0);
-    R out[2][E];
+  const int ix0 = xg * G, nact = min(G, g.Nx - ix0);
+  R out[2][E];
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-      __syncthreads();  // the transforms' exchanges, or the previous round's reads, are done
+  for (int h = 0; h < 2; h++) {
+    __syncthreads();  // the transforms' exchanges, or the previous round's reads, are done
 #pragma unroll
-      for (int s = 0; s < E; s++) lds[team * SP + t + T * s] = h ? e[s].y : e[s].x;
-      __syncthreads();
-#pragma unroll
-      for (int i = 0; i < E; i++) {
-        const int el = (int)threadIdx.x + NT * i;  // G*NZ = NT*E elements per block
-        const int zb = el / (G * ZB), w = el % (G * ZB), tm = w / ZB, r = w % ZB;
-        out[h][i] = lds[min(tm, nact - 1) * SP + zb * ZB + r];
-      }
-    }
+    for (int s = 0; s < E; s++) lds[team * SP + t + T * s] = h ? e[s].y : e[s].x;
+    __syncthreads();
 #pragma unroll
     for (int i = 0; i < E; i++) {
-      const int el = (int)threadIdx.x + NT * i;
-      const int zb = el / (G * ZB), w = el % (G * ZB), tm = w / ZB;
-      if (tm < nact) dst[((size_t)zb * g.Nx + ix0) * ZB + w] = cx<R>{out[0][i], out[1][i]};
+      const int el = (int)threadIdx.x + NT * i;  // G*NZ = NT*E elements per block
+      const int zb = el / (G * ZB), w = el % (G * ZB), tm = w / ZB, r = w % ZB;
+      out[h][i] = lds[min(tm, nact - 1) * SP + zb * ZB + r];
     }
-  } else if (act) {
+  }
 #pragma unroll
-    for (int s = 0; s < E; s++) {
-      const int z = t + T * s;
-      dst[((size_t)(z / ZB) * g.Nx + ix) * ZB + (z % ZB)] = e[s];
-    }
+  for (int i = 0; i < E; i++) {
+    const int el = (int)threadIdx.x + NT * i;
+    const int zb = el / (G * ZB), w = el % (G * ZB), tm = w / ZB;
+    if (tm < nact) dst[((size_t)zb * g.Nx + ix0) * ZB + w] = cx<R>{out[0][i], out[1][i]};
   }
 }
 
@@ -713,7 +701,7 @@ __global__ __launch_bounds__(zthreads<NZ>()) void k_zfwd(const cx<R> *__restrict
                                               const cx<R> *__restrict__ tw, Geom g, int plane0) {
   using PL = fft::Plan<NZ>;
   constexpr int T = PL::T, E = PL::E, G = zteams<NZ>(), NT = zthreads<NZ>(), SP = stage_stride<NZ>();
-  __shared__ __align__(16) R lds[zbuf_reals<NZ, R>()];
+  __shared__ __align__(16) R lds[zbuf_reals<NZ>()];
   const int team = threadIdx.x / T, t = threadIdx.x % T;
   const int nxg = (g.Nx + G - 1) / G;
   int b = blockIdx.x;
@@ -724,34 +712,26 @@ __global__ __launch_bounds__(zthreads<NZ>()) void k_zfwd(const cx<R> *__restrict
   const bool act = ix < g.Nx;
   const cx<R> *src = B + (size_t)(pl * NPROD + q) * NZ * g.Nx;
   cx<R> e[E];
-  if constexpr (z_staged<NZ, R>()) {
-    const int ix0 = xg * G, nact = min(G, g.Nx - ix0);
-    cx<R> v[E];
+  const int ix0 = xg * G, nact = min(G, g.Nx - ix0);
+  cx<R> v[E];
 #pragma unroll
-    for (int i = 0; i < E; i++) {  // all loads in flight together, clamped into the block's runs
+  for (int i = 0; i < E; i++) {  // all loads in flight together, clamped into the block's runs
+    const int el = (int)threadIdx.x + NT * i;
+    const int zb = el / (G * ZB), w = el % (G * ZB);
+    v[i] = src[((size_t)zb * g.Nx + ix0) * ZB + min(w, nact * ZB - 1)];
+  }
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+#pragma unroll
+    for (int i = 0; i < E; i++) {
       const int el = (int)threadIdx.x + NT * i;
-      const int zb = el / (G * ZB), w = el % (G * ZB);
-      v[i] = src[((size_t)zb * g.Nx + ix0) * ZB + min(w, nact * ZB - 1)];
+      const int zb = el / (G * ZB), w = el % (G * ZB), tm = w / ZB, r = w % ZB;
+      lds[tm * SP + zb * ZB + r] = tm < nact ? (h ? v[i].y : v[i].x) : R(0);
     }
+    __syncthreads();
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-#pragma unroll
-      for (int i = 0; i < E; i++) {
-        const int el = (int)threadIdx.x + NT * i;
-        const int zb = el / (G * ZB), w = el % (G * ZB), tm = w / ZB, r = w % ZB;
-        lds[tm * SP + zb * ZB + r] = tm < nact ? (h ? v[i].y : v[i].x) : R(0);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int s = 0; s < E; s++) (h ? e[s].y : e[s].x) = lds[team * SP + t + T * s];
-      __syncthreads();  // the next round and the transforms reuse the staging area
-    }
-  } else {
-#pragma unroll
-    for (int s = 0; s < E; s++) {
-      const int z = t + T * s;
-      e[s] = act ? src[((size_t)(z / ZB) * g.Nx + ix) * ZB + (z % ZB)] : cx<R>{0, 0};
-    }
+    for (int s = 0; s < E; s++) (h ? e[s].y : e[s].x) = lds[team * SP + t + T * s];
+    __syncthreads();  // the next round and the transforms reuse the staging area
   }
   fft::fft_slots<NZ, -1, true, ZXCH>(e, lds + team * fft::lds_reals<NZ, ZXCH>(), tw, t);
   if (act) {

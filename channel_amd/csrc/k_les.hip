@@ -90,7 +90,9 @@ __device__ __forceinline__ float2 cmulf(float2 a, float2 b) {
 // row (65 and 66 us; the LDS reads of the shared operands bound them now).
 constexpr int ZT = 8;     // x modes per thread in the z sums
 constexpr int XT = 8;     // x points (or modes) per thread in the x sums
-constexpr int GT = 384;   // threads: 8 x 96 points of the 96 x 96 grid in whole rounds
+// threads: 8 x 96 points of the 96 x 96 grid in whole rounds (a force at 31x64x31 187 us,
+// 219 with 256), and no slower on the others (48 x 48: 69 and 71, 24 x 24: 49.5 and 49.9)
+constexpr int GT = 384;
 
 __host__ __device__ __forceinline__ int round_up(int n, int k) { return (n + k - 1) / k * k; }
 // The phases of the x sums, e^{+2 pi i ix xj / Mx}, come as [Nx][Mx up to XT] and
