@@ -31,18 +31,18 @@ namespace {
 constexpr int MOVE_BLOCKS = 64;
 // Where staging begins.  To the host it wins from the first size that is worth its
 // threads (0.1 ms): 9 MB take 0.5 ms, 0.7 directly.  To the device the runtime
-// pins the caller's pages and moves 29 GB/s, so the line lies where a first
-// transfer, which also pins the slots, is no slower: 115 MB first 3.7 ms, then 2.6,
-// directly 3.9; 75 MB first 4.0, then 1.8, directly 2.9 and 2.6; 12 MB the same 0.5.
+// pins the caller's pages and moves 29 GB/s, so there is less to win: 115 MB 2.6 ms,
+// directly 3.9; 12 MB the same 0.5.
 constexpr size_t TO_HOST_MIN = 8u << 20, TO_DEVICE_MIN = 96u << 20;
 
-// To the host an owner's first transfers go directly until they have moved what the
-// slots hold: what they lose by it (0.07 ms/MB) is then what pinning the slots costs
-// (2 to 3 ms), so that a short-lived owner does not pay for slots it will not use
-// (a first 15 MB took 2.0 ms with the pinning, 1.4 without).
-bool to_host_staged(HostStage &s, size_t bytes) {
+// An owner's first transfers go directly until what they lose by it (0.07 ms/MB to the
+// host, 0.012 to the device, a sixth) is what pinning the slots costs (2 to 3 ms), so that
+// a short-lived owner does not pay for slots it will not use: a first 15 MB to the host took
+// 2.0 ms with the pinning, 1.4 without, a first 110 MB to the device (a closure forward
+// of 599040 rows in all) 4.1 to 8.4 ms, 5.4 without.
+bool staging_pays(HostStage &s, size_t bytes, bool to_host) {
   if (s.ev[0]) return true;
-  s.direct += bytes;
+  s.direct += to_host ? bytes : bytes / 6;
   return s.direct > STAGE_SLOTS * STAGE_CHUNK;
 }
 
@@ -145,7 +145,7 @@ hipError_t staged(HostStage &s, char *host, char *device, size_t bytes, hipStrea
 
 template <bool TO_HOST>
 hipError_t copy(HostStage &s, void *host, void *device, size_t bytes, hipStream_t st) {
-  if (!s.off && bytes >= (TO_HOST ? TO_HOST_MIN : TO_DEVICE_MIN) && pageable(host) && (!TO_HOST || to_host_staged(s, bytes))) {
+  if (!s.off && bytes >= (TO_HOST ? TO_HOST_MIN : TO_DEVICE_MIN) && pageable(host) && staging_pays(s, bytes, TO_HOST)) {
     if (staged<TO_HOST>(s, static_cast<char *>(host), static_cast<char *>(device), bytes, st) == hipSuccess)
       return hipSuccess;
     // no pinned memory left, or a fault that the plain copy meets again: this owner

@@ -15,7 +15,7 @@ constexpr int STAGE_THREADS = 8, STAGE_SLOTS = 2 * STAGE_THREADS;
 struct HostStage {
   char *buf[STAGE_SLOTS] = {};
   hipEvent_t ev[STAGE_SLOTS] = {};
-  size_t direct = 0;  // bytes that went to the host without it
+  size_t direct = 0;  // bytes that went without it, those to the device at a sixth
   bool off = false;   // making or using the slots has failed
   void free();
 };

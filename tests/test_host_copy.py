@@ -61,17 +61,22 @@ def test_to_host_is_staged_once_it_has_moved_the_slots_size(driver, n):
         held = want
 
 
-def test_to_device(driver):
-    n = 97 * MB + 12
+def test_to_device_is_staged_once_the_slots_pay(driver):
+    n = 97 * MB + 12  # a sixth of what goes to the device counts
     rows = driver("d%d" % n, "d%d" % n, "g")
-    assert rows[0] == ["1", str(chunks(n)), "0", str(SLOTS), str(SLOTS)]
-    assert rows[1] == ["1", str(chunks(n)), "0", str(SLOTS), "0"]
+    assert rows[0] == ["1", "0", "1", "0", "0"]
+    assert rows[1] == ["1", str(chunks(n)), "0", str(SLOTS), str(SLOTS)]
     assert rows[2] == ["held", "0", "0"]
+    n = 193 * MB  # a first one as large as that
+    rows = driver("d%d" % n, "d%d" % (97 * MB), "d%d" % (96 * MB - 4))
+    assert rows[0] == ["1", str(chunks(n)), "0", str(SLOTS), str(SLOTS)]
+    assert rows[1] == ["1", str(chunks(97 * MB)), "0", str(SLOTS), "0"]
+    assert rows[2] == ["1", "0", "1", str(SLOTS), "0"]
 
 
 @pytest.mark.parametrize("slots", [0, 1, 9])
 def test_an_owner_without_slots_goes_on(driver, slots):
-    n, m = 97 * MB, 40 * MB
+    n, m = 193 * MB, 40 * MB
     first, second, third = driver("f%d" % slots, "d%d" % n, "d%d" % n, "h%d" % m)
     assert first[0] == "1" and first[2] == "1"  # the plain copy brought it all
     assert first[3] == "0"  # the slots it had are given back
