@@ -71,6 +71,7 @@ __device__ __forceinline__ unsigned pack2(__bf16 x, __bf16 y) {
 
 // The weights of the forward pass as A fragments, 104 registers, and the biases
 // in LDS.
+constexpr int WROW = 72;  // BF16 values per unit's row of weights in LDS, padded
 struct Layers {
   bf16x8 h[3][4][2], o[2];
   __device__ __forceinline__ void load(const Weights &w, int c16, int q) {
@@ -82,6 +83,17 @@ struct Layers {
         for (int ks = 0; ks < 2; ks++) h[L][mt][ks] = load8(w.woi + WOFF[L] + (mt * 16 + c16) * KP + ks * 32 + 8 * q);
 #pragma unroll
     for (int ks = 0; ks < 2; ks++) o[ks] = load8(w.woi + WOFF[3] + c16 * KP + ks * 32 + 8 * q);
+  }
+  // the same from rows of WROW values
+  __device__ __forceinline__ void load_rows(const __bf16 *r, int c16, int q) {
+#pragma unroll
+    for (int L = 0; L < 3; L++)
+#pragma unroll
+      for (int mt = 0; mt < 4; mt++)
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) h[L][mt][ks] = load8(r + (L * H + mt * 16 + c16) * WROW + ks * 32 + 8 * q);
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) o[ks] = load8(r + (3 * H + c16) * WROW + ks * 32 + 8 * q);
   }
 };
 
@@ -162,22 +174,30 @@ struct FromFloat {  // FP32 rows [n][46], any alignment of a float
   }
 };
 
-// y [N][6] of 16-sample tiles, one wave each, the weights in registers.  With
-// the weights read from LDS per tile and the activations turned through LDS
-// between layers, 599040 BF16 rows took 58 us, now 41; 65536 FP32 rows 8.9 us
-// with a conversion pass before it.
+// y [N][6] of 16-sample tiles, one wave each, the weights in registers.  A block's
+// waves fetch them together, by way of LDS, while the first rows are on their way: each for
+// itself, the waves spend most of a short call on that (us for 1024, 32768, 65536 and 599040
+// BF16 rows: 5.3, 8.7, 10.3 and 34.5; together 3.6, 4.8, 6.3 and 31.4).  With the
+// weights read from LDS per tile and the activations turned through LDS
+// between layers it was 4.6, 6.0, 8.8 and 54.7.
 template <class Src>
 __global__ __launch_bounds__(256, 2) void k_mlp_fwd(Weights w, Src src, int n, float *__restrict__ Y) {
   __shared__ __align__(16) float bias[BSIZE];
-  for (int i = threadIdx.x; i < BSIZE; i += 256) bias[i] = w.bias[i];
+  __shared__ __align__(16) __bf16 wl[WSIZE / KP * WROW];
   const int wv = threadIdx.x / 64, l = threadIdx.x % 64, c16 = l % 16, q = l / 16;
   const int ntile = (n + 15) / 16, stride = gridDim.x * 4;
-  Layers W;
-  W.load(w, c16, q);
-  __syncthreads();
   int tt = blockIdx.x * 4 + wv;
-  if (tt >= ntile) return;
   auto next = src.raw(min(tt * 16 + c16, n - 1), q);
+#pragma unroll
+  for (int k = 0; k < (WSIZE / 8 + 255) / 256; k++) {
+    const int i = threadIdx.x + 256 * k;
+    if (i < WSIZE / 8) *reinterpret_cast<bf16x8 *>(wl + i / (KP / 8) * WROW + i % (KP / 8) * 8) = load8(w.woi + 8 * i);
+  }
+  for (int i = threadIdx.x; i < BSIZE; i += 256) bias[i] = w.bias[i];
+  __syncthreads();
+  Layers W;
+  W.load_rows(wl, c16, q);
+  if (tt >= ntile) return;
   for (; tt < ntile; tt += stride) {
     const auto cur = next;
     next = src.raw(min((tt + stride) * 16 + c16, n - 1), q);  // rows past n read row n-1
