@@ -616,8 +616,8 @@ int chan_get_body_force(chan_ctx *c, double *F) {
     std::memset(F, 0, n * sizeof(cx<double>));
     return 0;
   }
-  // the products buffer (dead between calls; 6*Ny*ps elements of at least
-  // 8 bytes) holds the force in the device layout, 3*Ny*ps complex FP64
+  // the products buffer (dead between calls; chan_create gives it at least 48
+  // bytes per point) holds the force in the device layout, 3*Ny*ps complex FP64
   cx<double> *dev = static_cast<cx<double> *>(c->P);
   ForceArgs a = force_args(c);
   a.out = dev;

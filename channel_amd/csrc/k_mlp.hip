@@ -299,8 +299,8 @@ __global__ __launch_bounds__(256, 2) void k_mlp_fwd_les(Weights w, LesSource s, 
 // registers, leaving inputs, activations and dz of every layer in LDS as
 // [unit][sample]; then wave L adds the sets' weight gradient of layer L.  With per
 // = 4 the block writes its chunk's sum, with per = 2 (few chunks: twice the blocks
-// at work) each slot's.  8192 samples take 14 us in this one launch, where separate
-// forward, three backward and four weight-gradient kernels through memory took 97.
+// at work) each slot's.  8192 samples take 19 us in this one launch (16384: 25), where
+// separate forward, three backward and four weight-gradient kernels through memory took 97.
 constexpr int SP = 72;  // samples per LDS row, padded: 16-byte rows, spread over the banks
 struct GradLds {
   __bf16 in[4][64 * SP];   // inputs of the layers: X, act 1..3
