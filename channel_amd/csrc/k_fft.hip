@@ -1005,6 +1005,12 @@ hipError_t launch_fft_test(int N, int sign, hipStream_t st, cx<double> *data, co
 }
 
 // the smallest size of the form 9*2^k in [need, below), or `below` when none is
+// (z).  Faster wherever the grid fills the chip, and the x pass has fewer rows; us, this and
+// the physical size, z inverse and z forward: 191x384x189 (576 and 768 points) 646 and 758,
+// 1090 and 1291; 383x48x383 (1152 and 1536) 329 and 400, 642 and 779, FP32 293 and 304, 403
+// and 493; 15x24x383 15.5 and 18.3, 20.7 and 24.9.  Grids of one round of blocks lose up to a
+// us on the inverse in FP32 (7x12x95, 288 and 384, 10.0 and 9.1) and gain it on the x pass (8.2
+// and 9.1 with the CFL maximum).
 int alias_free_z(int need, int below) {
 #define X(N) \
   if (N >= need && N < below) return N;
